@@ -181,6 +181,20 @@ template <class R> struct StepArgs {
   int pswap;
 };
 
+// The launch boxes of one phase that share a kernel variant, taken by one launch: box k covers
+// loop-axis indices alo .. alo + an - 1 (with its row groups for the vectorised kernels) and
+// the blocks from first on (before the slot split); count is its threads.
+constexpr int MAXBOX = 8;
+struct LaunchBox {
+  int alo[3], an[3];
+  int g0, ngroups;
+  uint32_t first, count;
+};
+struct BoxSet {
+  int n;
+  LaunchBox b[MAXBOX];
+};
+
 // Halo connection (connect_the_chunks / process_incoming_chunk_data,
 // src/boundaries.cpp:368-600, src/step.cpp:172-223): non-owned point dst of array slot
 // `slot` takes the owned point src, copied (cls 2), negated (cls 1) or multiplied by the
@@ -262,15 +276,16 @@ void launch_step_batch(const BatchItem<R> *items, const uint32_t *blk_item, cons
 template <class R>
 void launch_dft_batch(const BatchDft<R> *items, const uint32_t *blk_item, const uint32_t *blk_first, unsigned nblk, long step,
                       hipStream_t s);
-// deferred accumulation of a batch whose chunks all accumulate every step: step `step`'s point
-// values into slot `slot` (block tables over points), and the steps first .. first + nsteps - 1
-// into the accumulators (block tables over points x frequency quads)
+// deferred accumulation over a window of steps first + 1, first + 2, ... after each item's
+// t_start (at most DFT_DEFER of which count for an item): the point values of the window's n-th step into the rings (block
+// tables over points), and the window's n steps into the accumulators (block tables over points
+// x frequency quads).  A step counts for an item when it is a multiple of its decimation.
 template <class R>
-void launch_dft_snap_batch(const BatchDft<R> *items, const uint32_t *blk_item, const uint32_t *blk_first, unsigned nblk, int slot,
-                           hipStream_t s);
+void launch_dft_snap_batch(const BatchDft<R> *items, const uint32_t *blk_item, const uint32_t *blk_first, unsigned nblk, long first,
+                           long n, hipStream_t s);
 template <class R>
 void launch_dft_flush_batch(const BatchDft<R> *items, const uint32_t *blk_item, const uint32_t *blk_first, unsigned nblk, long first,
-                            int nsteps, hipStream_t s);
+                            long n, hipStream_t s);
 // halo lists of many chunks: item k is (conns, phases, n, slots, ncmp)
 struct BatchConn {
   const Conn *conns;
@@ -334,11 +349,11 @@ template <class R> void launch_adj_dft_scatter(R *bar, const int64_t *idx, const
 template <class R> void launch_record(R *hist, const R *D, const Grid &g, const int *lo, const int *hi, hipStream_t s);
 
 // launchers (kernels.hip)
-// generic scalar kernel over the box a.g.blo..bhi (any cells, uPML included)
-template <class R> void launch_step(const StepArgs<R> &a, bool curl, bool upd, hipStream_t s);
-// vectorised kernel (16-byte accesses); pml: the uPML branches per point (else the box must
-// have no active uPML profile)
-template <class R> void launch_fast(const StepArgs<R> &a, bool curl, bool upd, bool pml, hipStream_t s);
+// generic scalar kernel over the boxes of bs (any cells, uPML included), alo and an filled
+template <class R> void launch_step(const StepArgs<R> &a, const BoxSet &bs, bool curl, bool upd, hipStream_t s);
+// vectorised kernel (16-byte accesses) over the boxes of bs; pml: the uPML branches per point
+// (else the boxes must have no active uPML profile)
+template <class R> void launch_fast(const StepArgs<R> &a, const BoxSet &bs, bool curl, bool upd, bool pml, hipStream_t s);
 // the 3D row kernel for a box with no active x or y uPML profile and no folded images; false
 // when the box or its slots do not qualify (the caller then uses launch_fast).
 // MEEP_AMD_NO_ROW3 (read once) turns it off.

@@ -313,6 +313,25 @@ struct DevBuf {
   }
 };
 
+template <class T> static void upload_vec(DevBuf &b, const std::vector<T> &v) {
+  b.alloc(sizeof(T) * std::max<size_t>(v.size(), 1));
+  if (!v.empty()) HIPCHECK(hipMemcpy(b.p, v.data(), sizeof(T) * v.size(), hipMemcpyHostToDevice));
+}
+// block tables of a list of item thread counts for block size bs, padded to 8 blocks
+static void block_tables(const std::vector<uint32_t> &counts, unsigned bs, std::vector<uint32_t> &item, std::vector<uint32_t> &first) {
+  item.clear();
+  first.clear();
+  for (size_t k = 0; k < counts.size(); ++k)
+    for (uint32_t f = 0; f < counts[k]; f += bs) {
+      item.push_back(uint32_t(k));
+      first.push_back(f);
+    }
+  while (item.size() % 8) {
+    item.push_back(0);
+    first.push_back(0x7fffffffu); // beyond every item's count: the block exits at once
+  }
+}
+
 static void ensure_gpu() {
   int n = 0;
   hipError_t e = hipGetDeviceCount(&n);
@@ -1178,13 +1197,12 @@ template <class R> struct Fields : FieldsBase {
       u.kapw = u.dsigw >= 0 ? a.pml.kap[u.dsigw] : nullptr;
     }
   }
+  // a launch box: index ranges per direction, inclusive
+  struct Box {
+    int lo[3], hi[3];
+  };
   void launch_box(StepArgs<R> &b, const int *lo, const int *hi, bool curl, bool upd, bool fast, bool pml) {
-    for (int d = 0; d < 3; ++d) {
-      b.g.blo[d] = lo[d];
-      b.g.bhi[d] = hi[d];
-    }
-    finalize_args(b);
-    check_args(b, curl, upd, fast);
+    set_box(b, lo, hi, curl, upd, fast);
     if (collector) {
       BatchItem<R> it;
       it.a = b;
@@ -1203,11 +1221,41 @@ template <class R> struct Fields : FieldsBase {
       collector->items[cur_phase][kind * 4 + (curl ? 2 : 0) + (upd ? 1 : 0)].push_back(it);
       return;
     }
-    if (fast) {
-      if (!launch_row3<R>(b, curl, upd, stream)) launch_fast<R>(b, curl, upd, pml, stream);
-    }
+    BoxSet bs;
+    bs.n = 0;
+    add_box(bs, b.g);
+    launch_boxes(b, bs, curl, upd, fast, pml);
+  }
+  static void add_box(BoxSet &bs, const Grid &g) {
+    if (bs.n >= MAXBOX) fail("internal: too many launch boxes");
+    LaunchBox &x = bs.b[bs.n++];
+    memset(&x, 0, sizeof x);
+    for (int k = 0; k < 3; ++k) x.alo[k] = g.alo[k], x.an[k] = g.an[k];
+  }
+  void launch_boxes(const StepArgs<R> &b, const BoxSet &bs, bool curl, bool upd, bool fast, bool pml) {
+    if (fast)
+      launch_fast<R>(b, bs, curl, upd, pml, stream);
     else
-      launch_step<R>(b, curl, upd, stream);
+      launch_step<R>(b, bs, curl, upd, stream);
+  }
+  // the boxes of `list` (validated one by one) in one launch of a chunk stepped alone
+  void launch_box_list(StepArgs<R> &b, const std::vector<Box> &list, bool curl, bool upd, bool fast, bool pml) {
+    BoxSet bs;
+    bs.n = 0;
+    for (const Box &bx : list) {
+      set_box(b, bx.lo, bx.hi, curl, upd, fast);
+      add_box(bs, b.g);
+    }
+    if (bs.n) launch_boxes(b, bs, curl, upd, fast, pml);
+  }
+  // b's launch box, with the loop-axis view derived and everything validated
+  void set_box(StepArgs<R> &b, const int *lo, const int *hi, bool curl, bool upd, bool fast) const {
+    for (int d = 0; d < 3; ++d) {
+      b.g.blo[d] = lo[d];
+      b.g.bhi[d] = hi[d];
+    }
+    finalize_args(b);
+    check_args(b, curl, upd, fast);
   }
   // ---- batched stepping: one step's launches recorded as items ---------------------------
   struct Collect {
@@ -1273,31 +1321,9 @@ template <class R> struct Fields : FieldsBase {
       DftChunk<R> &ch = *cp;
       if (!f[ch.c][0]) continue;
       if (ch.nfreq > 512) return false; // beyond the batched kernel's phase table
-      BatchDft<R> bd;
-      memset(&bd, 0, sizeof bd);
-      bd.a.f0 = f[ch.c][0];
-      bd.a.f1 = f[ch.c][1];
-      bd.a.idx = static_cast<const int64_t *>(ch.idx.p);
-      bd.a.w = static_cast<const double *>(ch.w.p);
-      bd.a.omega = static_cast<const double *>(ch.omega.p);
-      bd.a.scale_re = ch.scale.real();
-      bd.a.scale_im = ch.scale.imag();
-      bd.a.avg1 = ch.avg1;
-      bd.a.avg2 = ch.avg2;
-      bd.a.npts = ch.npts;
-      bd.a.nfreq = ch.nfreq;
-      bd.a.acc = ch.acc.p;
-      bd.a.comp = ch.comp.p;
-      bd.a.acc_kind = ch.acc_kind;
-      bd.dt = dt;
-      bd.half = (is_magnetic(ch.c) || is_B(ch.c)) ? 1 : 0;
-      bd.decimation = ch.decimation;
+      if (ch.nsnap || window_open) fail("internal: deferred DFT steps pending at batch planning");
+      BatchDft<R> bd = batch_dft(ch);
       bd.t_start = t;
-      if (ch.nsnap) fail("internal: deferred DFT steps pending at batch planning");
-      const size_t need = sizeof(R) * size_t(ch.npts) * DFT_DEFER * (f[ch.c][1] ? 2 : 1);
-      if (ch.snap.bytes < need) ch.snap.alloc(need);
-      bd.snap0 = static_cast<R *>(ch.snap.p);
-      bd.snap1 = f[ch.c][1] ? bd.snap0 + size_t(DFT_DEFER) * size_t(ch.npts) : nullptr;
       C.dft.push_back(bd);
     }
     return plan_valid;
@@ -1323,26 +1349,42 @@ template <class R> struct Fields : FieldsBase {
     if (curl)
       for (int d = 0; d < 3; ++d) cond_curl = cond_curl || (b.cc[d].f && b.cc[d].cnd);
     const bool fast = use_fast && !cond_curl && (!curl || fast_partners(kind == MP_K_STEP_BH ? B_ft : D_ft, cur_cmp, b));
+    if (collector) {
+      if (!interior_empty) launch_box(b, interior.lo, interior.hi, curl, upd, fast, rows_pml);
+      for (const Box &bx : slabs) launch_box(b, bx.lo, bx.hi, curl, upd, fast, true);
+      kend();
+      return;
+    }
+    // The interior goes to the row kernel where that takes it, else it joins the slabs'
+    // launch when it runs the same variant; the slabs of a phase are always one launch.
+    std::vector<Box> rest = slabs;
     if (!interior_empty) {
       // backward differences read the previous plane: walk the planes downwards so it was
       // fetched just before (forward differences prefetch their neighbour naturally)
       b.rev = fast && kind == MP_K_STEP_DE ? 1 : 0;
+      set_box(b, interior.lo, interior.hi, curl, upd, fast);
       // the interior launch alone is timed too (the class of the phase's largest kernel)
-      const bool mark = ktiming && !collector;
       hipEvent_t e0 = nullptr;
-      if (mark) {
+      if (ktiming) {
         e0 = get_event();
         HIPCHECK(hipEventRecord(e0, stream));
       }
-      launch_box(b, interior.lo, interior.hi, curl, upd, fast, rows_pml);
-      if (mark) {
+      bool done = fast && launch_row3<R>(b, curl, upd, stream);
+      if (!done && !slabs.empty() && (!fast || rows_pml))
+        rest.insert(rest.begin(), interior);
+      else if (!done) {
+        launch_box(b, interior.lo, interior.hi, curl, upd, fast, rows_pml);
+        done = true;
+      }
+      if (ktiming) {
+        if (!done) launch_box_list(b, rest, curl, upd, fast, true), rest.clear();
         hipEvent_t e1 = get_event();
         HIPCHECK(hipEventRecord(e1, stream));
         pending.push_back({kind == MP_K_STEP_BH ? MP_K_BH_INTERIOR : MP_K_DE_INTERIOR, e0, e1});
       }
     }
     b.rev = 0;
-    for (const Box &bx : slabs) launch_box(b, bx.lo, bx.hi, curl, upd, fast, true);
+    launch_box_list(b, rest, curl, upd, fast, true);
     kend();
   }
   // ---- per-step argument blocks ----
@@ -1370,9 +1412,6 @@ template <class R> struct Fields : FieldsBase {
   // The interior box: array indices j along each direction where no uPML profile is active
   // for either Yee shift (so every component there updates with the plain formulas), and
   // the slabs that cover the rest of the grid without overlap.
-  struct Box {
-    int lo[3], hi[3];
-  };
   bool boxes_valid = false;
   int quiet_lo[3] = {1, 1, 1}, quiet_hi[3] = {0, 0, 0}; // per direction: no uPML profile active
   Box interior;
@@ -3003,10 +3042,98 @@ template <class R> struct Fields : FieldsBase {
     return da;
   }
   bool dft_defer_steps = false; // set by step_n for calls of several steps
+  // Every chunk's accumulation arguments and block tables in device memory, so that one launch
+  // takes a step's point values of all chunks and one launch applies the deferred steps of
+  // all: a six-face flux box has 24 chunks, whose 24 launches of 2.9 us a step (and 24 of
+  // 10.2 us every DFT_DEFER steps) were half the step of a 131 x 118 x 125 cell.  Used where
+  // every chunk's phases fit the flush kernel's table.
+  struct DftGroup {
+    long dft_v = -1, plan_v = -1;
+    bool ok = false;
+    DevBuf items, snap_item, snap_first, flush_item, flush_first;
+    unsigned snap_nblk = 0, flush_nblk = 0;
+    std::vector<int> decs; // the chunks' distinct decimations
+    // whether a chunk accumulates, and the most times one does, in the steps t0 + 1 .. t1
+    long most_hits(long t0, long t1) const {
+      long m = 0;
+      for (int d : decs) m = std::max(m, t1 / d - t0 / d);
+      return m;
+    }
+    bool hits(long t0, long t1) const { return most_hits(t0, t1) > 0; }
+  } dgroup;
+  bool dft_group() {
+    if (dgroup.dft_v == dft_version && dgroup.plan_v == plan_version) return dgroup.ok;
+    flush_dft_group(); // steps deferred under the old tables
+    dgroup.dft_v = dft_version;
+    dgroup.plan_v = plan_version;
+    dgroup.ok = false;
+    dgroup.decs.clear();
+    std::vector<BatchDft<R>> items;
+    std::vector<uint32_t> pts, quads, item, first;
+    for (auto &cp : dft_chunks) {
+      DftChunk<R> &ch = *cp;
+      if (!f[ch.c][0]) continue;
+      if (std::find(dgroup.decs.begin(), dgroup.decs.end(), ch.decimation) == dgroup.decs.end()) dgroup.decs.push_back(ch.decimation);
+      if (ch.defer < DFT_DEFER || ch.npts < 1) return false;
+      if (ch.nsnap) fail("internal: deferred DFT steps pending");
+      items.push_back(batch_dft(ch));
+      pts.push_back(uint32_t(ch.npts));
+      const size_t q = size_t(ch.npts) * size_t((ch.nfreq + 3) / 4);
+      if (q >= (size_t(1) << 31)) return false;
+      quads.push_back(uint32_t(q));
+    }
+    if (items.empty()) return false;
+    upload_vec(dgroup.items, items);
+    block_tables(pts, 256, item, first);
+    upload_vec(dgroup.snap_item, item);
+    upload_vec(dgroup.snap_first, first);
+    dgroup.snap_nblk = unsigned(item.size());
+    block_tables(quads, 256, item, first);
+    upload_vec(dgroup.flush_item, item);
+    upload_vec(dgroup.flush_first, first);
+    dgroup.flush_nblk = unsigned(item.size());
+    return dgroup.ok = true;
+  }
+  // the open window of deferred steps: window_t + 1 .. window_end
+  bool window_open = false;
+  long window_t = 0, window_end = 0;
+  void flush_dft_group() {
+    if (!window_open) return;
+    launch_dft_flush_batch<R>(static_cast<const BatchDft<R> *>(dgroup.items.p), static_cast<const uint32_t *>(dgroup.flush_item.p),
+                              static_cast<const uint32_t *>(dgroup.flush_first.p), dgroup.flush_nblk, window_t,
+                              window_end - window_t, stream);
+    window_open = false;
+  }
+  // chunk ch as a batch item, its ring of deferred values allocated
+  BatchDft<R> batch_dft(DftChunk<R> &ch) {
+    BatchDft<R> bd;
+    memset(&bd, 0, sizeof bd);
+    bd.a = dft_args(ch);
+    bd.dt = dt;
+    bd.half = (is_magnetic(ch.c) || is_B(ch.c)) ? 1 : 0;
+    bd.decimation = ch.decimation;
+    bd.t_start = 0;
+    const size_t need = sizeof(R) * size_t(ch.npts) * DFT_DEFER * (bd.a.f1 ? 2 : 1);
+    if (ch.snap.bytes < need) ch.snap.alloc(need);
+    bd.snap0 = static_cast<R *>(ch.snap.p);
+    bd.snap1 = bd.a.f1 ? bd.snap0 + size_t(DFT_DEFER) * size_t(ch.npts) : nullptr;
+    return bd;
+  }
   // DFT accumulation of this step (dft_chunk::update_dft for every chunk, src/dft.cpp:250-308):
   // chunks whose phases for DFT_DEFER steps fit the flush kernel's table keep this step's
   // point values and accumulate every DFT_DEFER steps (and at the end of every step_n call)
   void update_dfts() {
+    if (dft_defer_steps && !dft_chunks.empty() && dft_group()) {
+      if (!dgroup.hits(t - 1, t)) return;
+      kbegin(MP_K_DFT);
+      if (!window_open) window_open = true, window_t = t - 1;
+      window_end = t;
+      launch_dft_snap_batch<R>(static_cast<const BatchDft<R> *>(dgroup.items.p), static_cast<const uint32_t *>(dgroup.snap_item.p),
+                               static_cast<const uint32_t *>(dgroup.snap_first.p), dgroup.snap_nblk, window_t, t - window_t, stream);
+      if (dgroup.most_hits(window_t, t) == DFT_DEFER) flush_dft_group();
+      kend();
+      return;
+    }
     for (auto &cp : dft_chunks) {
       DftChunk<R> &ch = *cp;
       if (t % ch.decimation) continue;
@@ -3046,6 +3173,7 @@ template <class R> struct Fields : FieldsBase {
     ch.nsnap = 0;
   }
   void flush_dfts() {
+    flush_dft_group();
     for (auto &cp : dft_chunks) flush_dft(*cp);
   }
 
@@ -4229,24 +4357,6 @@ template <class R> struct Batch : BatchBase {
     *ms = last_ms;
   }
   static int bs_index(int b) { return b == 64 ? 0 : b == 128 ? 1 : b == 256 ? 2 : 3; }
-  // block tables of a list of item thread counts for block size bs, padded to 8 blocks
-  static void tables(const std::vector<uint32_t> &counts, unsigned bs, std::vector<uint32_t> &item, std::vector<uint32_t> &first) {
-    item.clear();
-    first.clear();
-    for (size_t k = 0; k < counts.size(); ++k)
-      for (uint32_t f = 0; f < counts[k]; f += bs) {
-        item.push_back(uint32_t(k));
-        first.push_back(f);
-      }
-    while (item.size() % 8) {
-      item.push_back(0);
-      first.push_back(0x7fffffffu); // beyond every item's count: the block exits at once
-    }
-  }
-  template <class T> static void upload(DevBuf &b, const std::vector<T> &v) {
-    b.alloc(sizeof(T) * std::max<size_t>(v.size(), 1));
-    if (!v.empty()) HIPCHECK(hipMemcpy(b.p, v.data(), sizeof(T) * v.size(), hipMemcpyHostToDevice));
-  }
   bool stale() const {
     if (!planned) return true;
     for (size_t q = 0; q < sims.size(); ++q)
@@ -4305,14 +4415,14 @@ template <class R> struct Batch : BatchBase {
           if (it != c.items[phase].end()) g.host.insert(g.host.end(), it->second.begin(), it->second.end());
         }
         if (g.host.empty()) continue;
-        upload(g.items, g.host);
+        upload_vec(g.items, g.host);
         std::vector<uint32_t> counts;
         for (auto &it : g.host) counts.push_back(it.count);
         for (int b = 0; b < 4; ++b) {
           std::vector<uint32_t> item, first;
-          tables(counts, unsigned(BATCH_BLOCKS[b]), item, first);
-          upload(g.blk_item[b], item);
-          upload(g.blk_first[b], first);
+          block_tables(counts, unsigned(BATCH_BLOCKS[b]), item, first);
+          upload_vec(g.blk_item[b], item);
+          upload_vec(g.blk_first[b], first);
           g.nblk[b] = unsigned(item.size());
         }
         groups.push_back(std::move(gp));
@@ -4323,10 +4433,10 @@ template <class R> struct Batch : BatchBase {
       std::vector<uint32_t> counts;
       for (auto &c : ci) counts.push_back(uint32_t(c.n));
       std::vector<uint32_t> item, first;
-      tables(counts, 256, item, first);
-      upload(conn_items[grp], ci);
-      upload(conn_item_tab[grp], item);
-      upload(conn_first_tab[grp], first);
+      block_tables(counts, 256, item, first);
+      upload_vec(conn_items[grp], ci);
+      upload_vec(conn_item_tab[grp], item);
+      upload_vec(conn_first_tab[grp], first);
       conn_nblk[grp] = ci.empty() ? 0 : unsigned(item.size());
     }
     dft_host.clear();
@@ -4335,9 +4445,9 @@ template <class R> struct Batch : BatchBase {
       std::vector<uint32_t> counts;
       for (auto &d : dft_host) counts.push_back(uint32_t(size_t(d.a.npts) * d.a.nfreq));
       std::vector<uint32_t> item, first;
-      tables(counts, 256, item, first);
-      upload(dft_item_tab, item);
-      upload(dft_first_tab, first);
+      block_tables(counts, 256, item, first);
+      upload_vec(dft_item_tab, item);
+      upload_vec(dft_first_tab, first);
       dft_nblk = dft_host.empty() ? 0 : unsigned(item.size());
     }
     // deferred accumulation when every chunk accumulates every step and its phases for
@@ -4348,15 +4458,15 @@ template <class R> struct Batch : BatchBase {
     if (dft_defer) {
       std::vector<uint32_t> counts, item, first;
       for (auto &d : dft_host) counts.push_back(uint32_t(d.a.npts));
-      tables(counts, 256, item, first);
-      upload(dft_snap_item, item);
-      upload(dft_snap_first, first);
+      block_tables(counts, 256, item, first);
+      upload_vec(dft_snap_item, item);
+      upload_vec(dft_snap_first, first);
       dft_snap_nblk = unsigned(item.size());
       counts.clear();
       for (auto &d : dft_host) counts.push_back(uint32_t(size_t(d.a.npts) * size_t((d.a.nfreq + 3) / 4)));
-      tables(counts, 256, item, first);
-      upload(dft_flush_item, item);
-      upload(dft_flush_first, first);
+      block_tables(counts, 256, item, first);
+      upload_vec(dft_flush_item, item);
+      upload_vec(dft_flush_first, first);
       dft_flush_nblk = unsigned(item.size());
     }
     plan_versions.clear();
@@ -4389,7 +4499,7 @@ template <class R> struct Batch : BatchBase {
     }
     const int slot = int(s % DFT_DEFER);
     launch_dft_snap_batch<R>(di, static_cast<const uint32_t *>(dft_snap_item.p), static_cast<const uint32_t *>(dft_snap_first.p),
-                             dft_snap_nblk, slot, stream);
+                             dft_snap_nblk, s - slot, slot + 1, stream);
     if (slot == DFT_DEFER - 1 || s == call_steps - 1)
       launch_dft_flush_batch<R>(di, static_cast<const uint32_t *>(dft_flush_item.p), static_cast<const uint32_t *>(dft_flush_first.p),
                                 dft_flush_nblk, s - slot, slot + 1, stream);
@@ -4413,14 +4523,14 @@ template <class R> struct Batch : BatchBase {
       for (long st = 0; st < m; ++st)
         for (size_t e = 0; e < rec.size(); ++e) hrows[size_t(st) * rl + row_off[q] + e] = F->recipe_value(rec[e], F->t + st);
     }
-    upload(rows, hrows);
+    upload_vec(rows, hrows);
     {
       size_t k = 0;
       for (size_t q = 0; q < sims.size(); ++q)
         for (auto &cp : sims[q]->dft_chunks)
           if (sims[q]->f[cp->c][0]) dft_host[k++].t_start = sims[q]->t;
       if (k != dft_host.size()) fail("internal: batch DFT chunks changed");
-      upload(dft_items, dft_host);
+      upload_vec(dft_items, dft_host);
     }
     const double *drows = static_cast<const double *>(rows.p);
     call_steps = m;

@@ -73,36 +73,6 @@ template <class R> __device__ __forceinline__ void put(R *f, uint32_t i, R v, co
   }
 }
 
-// vrow: the step's row of source values
-template <class R> __device__ __forceinline__ R apply_tab(const SrcTab &t, int c, uint32_t i, R v, const double *vrow) {
-#pragma unroll
-  for (int s = 0; s < SRC_TAB; ++s)
-    if (s < t.n && t.comp[s] == c && t.idx[s] == int64_t(i)) v = R(double(v) - vrow[t.vbase + s]);
-  return v;
-}
-
-// value of box source S at loop-axis indices (j0, j1, j2); contraction is off so the complex
-// product rounds as the host's does
-template <int S> __device__ __forceinline__ double box_value(const SrcBoxes &b, int cmp, int j0, int j1, int j2, const double *vrow) {
-#pragma clang fp contract(off)
-  const int64_t k = int64_t(j0 - b.lo[S][0]) * b.bst[S][0] + int64_t(j1 - b.lo[S][1]) * b.bst[S][1] +
-                    int64_t(j2 - b.lo[S][2]) * b.bst[S][2];
-  const double2 am = b.amp[S][k];
-  const double sx = vrow[b.vbase + 2 * S], sy = vrow[b.vbase + 2 * S + 1];
-  const double re = am.x * sx - am.y * sy, im = am.x * sy + am.y * sx;
-  return cmp ? im * b.mult[S] : re * b.mult[S];
-}
-template <int S> __device__ __forceinline__ bool in_box(const SrcBoxes &b, int c, int j0, int j1, int j2) {
-  return S < b.n && b.comp[S] == c && j0 >= b.lo[S][0] && j0 <= b.hi[S][0] && j1 >= b.lo[S][1] && j1 <= b.hi[S][1] &&
-         j2 >= b.lo[S][2] && j2 <= b.hi[S][2];
-}
-template <class R>
-__device__ __forceinline__ R apply_boxes(const SrcBoxes &b, int cmp, int c, int j0, int j1, int j2, R v, const double *vrow) {
-  static_assert(SRC_BOX == 2, "one term per box");
-  if (in_box<0>(b, c, j0, j1, j2)) v = R(double(v) - box_value<0>(b, cmp, j0, j1, j2, vrow));
-  if (in_box<1>(b, c, j0, j1, j2)) v = R(double(v) - box_value<1>(b, cmp, j0, j1, j2, vrow));
-  return v;
-}
 // whether the V points from (j0, j1, z0) along the row meet the launch's source box
 template <int V, class R> __device__ __forceinline__ bool in_src_box(const StepArgs<R> &a, int j0, int j1, int z0) {
   return j0 >= a.sbox_lo[0] && j0 <= a.sbox_hi[0] && j1 >= a.sbox_lo[1] && j1 <= a.sbox_hi[1] && z0 + V - 1 >= a.sbox_lo[2] &&
@@ -241,15 +211,36 @@ __device__ __forceinline__ void step_slot(const StepArgs<R> &a, uint32_t i, int 
   cell_update<R, CURL, UPD, C>(a, i, j0, j1, j2, cu, vrow);
 }
 
-// point t of the launch box of a
+// A launch's boxes are one launch because each is small beside the chip: the four x and y uPML
+// slabs of a 131 x 118 x 125 cell took 4 x 10.2 us as launches of their own and fill a
+// fraction of the 256 CUs each.  The block finds its box by its index (uniform selects over
+// constant offsets); a box's geometry travels in scalar registers.
+__device__ __forceinline__ LaunchBox pick_box(const BoxSet &bs, uint32_t lb) {
+  LaunchBox x = bs.b[0];
+#pragma unroll
+  for (int k = 1; k < MAXBOX; ++k)
+    if (k < bs.n && lb >= bs.b[k].first) x = bs.b[k];
+  return x;
+}
+// the launch box in a batch item's own grid
+__device__ __forceinline__ LaunchBox item_box(const Grid &g, int g0, int ngroups) {
+  LaunchBox x;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) x.alo[k] = g.alo[k], x.an[k] = g.an[k];
+  x.g0 = g0;
+  x.ngroups = ngroups;
+  return x;
+}
+
+// point t of launch box x
 template <class R, bool CURL, bool UPD>
-__device__ __forceinline__ void step_body(const StepArgs<R> &a, uint32_t t, const double *vrow) {
+__device__ __forceinline__ void step_body(const StepArgs<R> &a, const LaunchBox &x, uint32_t t, const double *vrow) {
   const Grid &g = a.g;
-  const uint32_t r = t / uint32_t(g.an[2]);
-  const int q2 = int(t - r * uint32_t(g.an[2]));
-  const int q0 = int(r / uint32_t(g.an[1]));
-  const int q1 = int(r - uint32_t(q0) * uint32_t(g.an[1]));
-  const int j0 = g.alo[0] + q0, j1 = g.alo[1] + q1, j2 = g.alo[2] + q2;
+  const uint32_t r = t / uint32_t(x.an[2]);
+  const int q2 = int(t - r * uint32_t(x.an[2]));
+  const int q0 = int(r / uint32_t(x.an[1]));
+  const int q1 = int(r - uint32_t(q0) * uint32_t(x.an[1]));
+  const int j0 = x.alo[0] + q0, j1 = x.alo[1] + q1, j2 = x.alo[2] + q2;
   const uint32_t i = uint32_t(j0 * g.ast[0] + j1 * g.ast[1] + j2 * g.ast[2]);
   step_slot<R, CURL, UPD, 0>(a, i, j0, j1, j2, vrow);
   step_slot<R, CURL, UPD, 1>(a, i, j0, j1, j2, vrow);
@@ -257,10 +248,12 @@ __device__ __forceinline__ void step_body(const StepArgs<R> &a, uint32_t t, cons
 }
 
 template <class R, bool CURL, bool UPD>
-__global__ __launch_bounds__(BLOCK) void k_step(const StepArgs<R> a, uint32_t count) {
-  const uint32_t t = xcd_block() * uint32_t(BLOCK) + threadIdx.x;
-  if (t >= count) return;
-  step_body<R, CURL, UPD>(a, t, a.vrow);
+__global__ __launch_bounds__(BLOCK) void k_step(const StepArgs<R> a, const BoxSet bs) {
+  const uint32_t lb = xcd_block();
+  const LaunchBox x = pick_box(bs, lb);
+  const uint32_t t = (lb - x.first) * uint32_t(BLOCK) + threadIdx.x;
+  if (t >= x.count) return;
+  step_body<R, CURL, UPD>(a, x, t, a.vrow);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -672,22 +665,22 @@ __device__ __forceinline__ void fast_slot(const StepArgs<R> &a, uint32_t i, int 
   }
 }
 
-// group t of the launch box of a (groups of V points along the rows, from group g0)
+// group t of launch box x (groups of V points along the rows, from group x.g0)
 template <class R, int V, bool CURL, bool UPD, bool PML, int NP>
-__device__ __forceinline__ void fast_body(const StepArgs<R> &a, uint32_t t, int g0, int ngroups, const double *vrow) {
+__device__ __forceinline__ void fast_body(const StepArgs<R> &a, const LaunchBox &x, uint32_t t, const double *vrow) {
   const Grid &g = a.g;
-  const uint32_t r = t / uint32_t(ngroups);
-  const int grp = int(t - r * uint32_t(ngroups));
-  const int q0 = int(r / uint32_t(g.an[1]));
-  const int q1 = int(r - uint32_t(q0) * uint32_t(g.an[1]));
-  const int j0 = g.alo[0] + q0, j1 = g.alo[1] + q1;
-  const int z0 = (g0 + grp) * V;
+  const uint32_t r = t / uint32_t(x.ngroups);
+  const int grp = int(t - r * uint32_t(x.ngroups));
+  const int q0 = int(r / uint32_t(x.an[1]));
+  const int q1 = int(r - uint32_t(q0) * uint32_t(x.an[1]));
+  const int j0 = x.alo[0] + q0, j1 = x.alo[1] + q1;
+  const int z0 = (x.g0 + grp) * V;
   const uint32_t i = uint32_t(j0 * g.ast[0] + j1 * g.ast[1] + z0);
   // points of the group inside the launch box along the row
   unsigned boxmask = 0;
 #pragma unroll
   for (int k = 0; k < V; ++k)
-    if (z0 + k >= g.alo[2] && z0 + k < g.alo[2] + g.an[2]) boxmask |= 1u << k;
+    if (z0 + k >= x.alo[2] && z0 + k < x.alo[2] + x.an[2]) boxmask |= 1u << k;
   // ownership of each component slot in this group
   unsigned m0 = 0, m1 = 0, m2 = 0;
   if (CURL ? a.cc[0].f : a.uc[0].f) m0 = group_owned<V>(g, CURL ? a.cc[0].ax.ybits : a.uc[0].ax.ybits, j0, j1, z0, boxmask);
@@ -707,21 +700,21 @@ __device__ __forceinline__ void fast_body(const StepArgs<R> &a, uint32_t t, int 
 }
 
 
-// group t of the launch box for slot C alone
+// group t of launch box x for slot C alone
 template <class R, int V, bool CURL, bool UPD, bool PML, int NP, int C>
-__device__ __forceinline__ void fast_body_slot(const StepArgs<R> &a, uint32_t t, int g0, int ngroups) {
+__device__ __forceinline__ void fast_body_slot(const StepArgs<R> &a, const LaunchBox &x, uint32_t t) {
   const Grid &g = a.g;
-  const uint32_t r = t / uint32_t(ngroups);
-  const int grp = int(t - r * uint32_t(ngroups));
-  const int q0 = int(r / uint32_t(g.an[1]));
-  const int q1 = int(r - uint32_t(q0) * uint32_t(g.an[1]));
-  const int j0 = g.alo[0] + q0, j1 = g.alo[1] + q1;
-  const int z0 = (g0 + grp) * V;
+  const uint32_t r = t / uint32_t(x.ngroups);
+  const int grp = int(t - r * uint32_t(x.ngroups));
+  const int q0 = int(r / uint32_t(x.an[1]));
+  const int q1 = int(r - uint32_t(q0) * uint32_t(x.an[1]));
+  const int j0 = x.alo[0] + q0, j1 = x.alo[1] + q1;
+  const int z0 = (x.g0 + grp) * V;
   const uint32_t i = uint32_t(j0 * g.ast[0] + j1 * g.ast[1] + z0);
   unsigned boxmask = 0;
 #pragma unroll
   for (int k = 0; k < V; ++k)
-    if (z0 + k >= g.alo[2] && z0 + k < g.alo[2] + g.an[2]) boxmask |= 1u << k;
+    if (z0 + k >= x.alo[2] && z0 + k < x.alo[2] + x.an[2]) boxmask |= 1u << k;
   if (!(CURL ? a.cc[C].f : a.uc[C].f)) return;
   const unsigned m = group_owned<V>(g, CURL ? a.cc[C].ax.ybits : a.uc[C].ax.ybits, j0, j1, z0, boxmask);
   if (!m) return;
@@ -739,20 +732,20 @@ __device__ __forceinline__ void fast_body_slot(const StepArgs<R> &a, uint32_t t,
 // rows in its L2.  A curl alone keeps the three slots in one thread (measured faster there:
 // its threads are light, and the shared centre rows are loaded once).
 template <class R, int V, bool CURL, bool UPD, bool PML, int NP>
-__global__ __launch_bounds__(BLOCK) void k_fast(const StepArgs<R> a, uint32_t count, int g0, int ngroups) {
+__global__ __launch_bounds__(BLOCK) void k_fast(const StepArgs<R> a, const BoxSet bs) {
+  const uint32_t lb = xcd_block(a.rev);
+  const uint32_t q = UPD ? lb / 3u : lb;
+  const LaunchBox x = pick_box(bs, q);
+  const uint32_t t = (q - x.first) * uint32_t(BLOCK) + threadIdx.x;
+  if (t >= x.count) return;
   if (!UPD) {
-    const uint32_t t = xcd_block(a.rev) * uint32_t(BLOCK) + threadIdx.x;
-    if (t >= count) return;
-    fast_body<R, V, CURL, UPD, PML, NP>(a, t, g0, ngroups, a.vrow);
+    fast_body<R, V, CURL, UPD, PML, NP>(a, x, t, a.vrow);
     return;
   }
-  const uint32_t lb = xcd_block(a.rev);
-  const int C = int(lb % 3u);
-  const uint32_t t = (lb / 3u) * uint32_t(BLOCK) + threadIdx.x;
-  if (t >= count) return;
-  if (C == 0) fast_body_slot<R, V, CURL, UPD, PML, NP, 0>(a, t, g0, ngroups);
-  else if (C == 1) fast_body_slot<R, V, CURL, UPD, PML, NP, 1>(a, t, g0, ngroups);
-  else fast_body_slot<R, V, CURL, UPD, PML, NP, 2>(a, t, g0, ngroups);
+  const int C = int(lb - 3u * q);
+  if (C == 0) fast_body_slot<R, V, CURL, UPD, PML, NP, 0>(a, x, t);
+  else if (C == 1) fast_body_slot<R, V, CURL, UPD, PML, NP, 1>(a, x, t);
+  else fast_body_slot<R, V, CURL, UPD, PML, NP, 2>(a, x, t);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -1553,57 +1546,71 @@ __global__ void k_check(const R *const *ptrs, const int64_t *idx, const double *
 }
 
 
-template <class R> void launch_step(const StepArgs<R> &a, bool curl, bool upd, hipStream_t s) {
-  const size_t count = size_t(a.g.an[0]) * size_t(a.g.an[1]) * size_t(a.g.an[2]);
-  const unsigned nb = nblocks8(count);
-  const uint32_t c32 = uint32_t(count);
+// blocks of the boxes of bs (each box from a block of its own), their first blocks filled in
+static unsigned box_blocks(BoxSet &bs) {
+  size_t nb = 0;
+  for (int k = 0; k < bs.n; ++k) {
+    bs.b[k].first = uint32_t(nb);
+    nb += nblocks(bs.b[k].count);
+  }
+  if (3 * nb + 8 >= (size_t(1) << 31)) throw std::runtime_error("meep: launch boxes too large for one launch");
+  return unsigned(nb);
+}
+static uint32_t box_count(const char *what, size_t n) {
+  if (n >= (size_t(1) << 32)) throw std::runtime_error(what);
+  return uint32_t(n);
+}
+template <class R> void launch_step(const StepArgs<R> &a, const BoxSet &boxes, bool curl, bool upd, hipStream_t s) {
+  BoxSet bs = boxes;
+  for (int k = 0; k < bs.n; ++k)
+    bs.b[k].count = box_count("meep: launch box too large for one launch",
+                              size_t(bs.b[k].an[0]) * size_t(bs.b[k].an[1]) * size_t(bs.b[k].an[2]));
+  const unsigned nb = (box_blocks(bs) + 7u) / 8u * 8u;
   if (curl && upd)
-    hipLaunchKernelGGL((k_step<R, true, true>), dim3(nb), dim3(BLOCK), 0, s, a, c32);
+    hipLaunchKernelGGL((k_step<R, true, true>), dim3(nb), dim3(BLOCK), 0, s, a, bs);
   else if (curl)
-    hipLaunchKernelGGL((k_step<R, true, false>), dim3(nb), dim3(BLOCK), 0, s, a, c32);
+    hipLaunchKernelGGL((k_step<R, true, false>), dim3(nb), dim3(BLOCK), 0, s, a, bs);
   else if (upd)
-    hipLaunchKernelGGL((k_step<R, false, true>), dim3(nb), dim3(BLOCK), 0, s, a, c32);
+    hipLaunchKernelGGL((k_step<R, false, true>), dim3(nb), dim3(BLOCK), 0, s, a, bs);
 }
 
-// groups of V points along the rows of a's launch box: first group, groups per row, threads
-template <int V> static inline void fast_groups(const Grid &g, int &g0, int &ngroups, uint32_t &count) {
-  g0 = g.alo[2] / V;
-  ngroups = (g.alo[2] + g.an[2] - 1) / V - g0 + 1;
-  const size_t n = size_t(ngroups) * size_t(g.an[0]) * size_t(g.an[1]);
-  if (n >= (size_t(1) << 32)) throw std::runtime_error("meep: launch box too large for one launch");
-  count = uint32_t(n);
-}
-template <class R, int V, bool PML, int NP> void launch_fast_np(const StepArgs<R> &a, bool curl, bool upd, hipStream_t s) {
-  int g0, ngroups;
-  uint32_t c32;
-  fast_groups<V>(a.g, g0, ngroups, c32);
-  const unsigned nb = upd ? (3u * nblocks(c32) + 7u) / 8u * 8u : nblocks8(c32); // with an update, one slot per block
+template <class R, int V, bool PML, int NP>
+void launch_fast_np(const StepArgs<R> &a, const BoxSet &boxes, bool curl, bool upd, hipStream_t s) {
+  BoxSet bs = boxes;
+  for (int k = 0; k < bs.n; ++k) { // groups of V points along the rows of each box
+    LaunchBox &x = bs.b[k];
+    x.g0 = x.alo[2] / V;
+    x.ngroups = (x.alo[2] + x.an[2] - 1) / V - x.g0 + 1;
+    x.count = box_count("meep: launch box too large for one launch", size_t(x.ngroups) * size_t(x.an[0]) * size_t(x.an[1]));
+  }
+  const unsigned n = box_blocks(bs);
+  const unsigned nb = ((upd ? 3u * n : n) + 7u) / 8u * 8u; // with an update, one slot per block
   if (curl && upd)
-    hipLaunchKernelGGL((k_fast<R, V, true, true, PML, NP>), dim3(nb), dim3(BLOCK), 0, s, a, c32, g0, ngroups);
+    hipLaunchKernelGGL((k_fast<R, V, true, true, PML, NP>), dim3(nb), dim3(BLOCK), 0, s, a, bs);
   else if (curl)
-    hipLaunchKernelGGL((k_fast<R, V, true, false, PML, NP>), dim3(nb), dim3(BLOCK), 0, s, a, c32, g0, ngroups);
+    hipLaunchKernelGGL((k_fast<R, V, true, false, PML, NP>), dim3(nb), dim3(BLOCK), 0, s, a, bs);
   else if (upd)
-    hipLaunchKernelGGL((k_fast<R, V, false, true, PML, NP>), dim3(nb), dim3(BLOCK), 0, s, a, c32, g0, ngroups);
+    hipLaunchKernelGGL((k_fast<R, V, false, true, PML, NP>), dim3(nb), dim3(BLOCK), 0, s, a, bs);
 }
 // The pole-carrying updates hold P, P_prev and sigma of every pole in registers: in FP32 they
 // take 8-byte groups (V = 2) to keep the occupancy of the 16-byte form's plain kernels.
-template <class R, bool PML> void launch_fast_t(const StepArgs<R> &a, bool curl, bool upd, hipStream_t s) {
+template <class R, bool PML> void launch_fast_t(const StepArgs<R> &a, const BoxSet &bs, bool curl, bool upd, hipStream_t s) {
   constexpr int V = 16 / sizeof(R), VP = V > 2 ? 2 : V;
   if (!upd || a.npole == 0) {
-    launch_fast_np<R, V, PML, 0>(a, curl, upd, s);
+    launch_fast_np<R, V, PML, 0>(a, bs, curl, upd, s);
     return;
   }
   switch (a.npole) {
-    case 1: launch_fast_np<R, VP, PML, 1>(a, curl, upd, s); break;
-    case 2: launch_fast_np<R, VP, PML, 2>(a, curl, upd, s); break;
-    default: launch_fast_np<R, VP, PML, MAXPOLE>(a, curl, upd, s); break;
+    case 1: launch_fast_np<R, VP, PML, 1>(a, bs, curl, upd, s); break;
+    case 2: launch_fast_np<R, VP, PML, 2>(a, bs, curl, upd, s); break;
+    default: launch_fast_np<R, VP, PML, MAXPOLE>(a, bs, curl, upd, s); break;
   }
 }
-template <class R> void launch_fast(const StepArgs<R> &a, bool curl, bool upd, bool pml, hipStream_t s) {
+template <class R> void launch_fast(const StepArgs<R> &a, const BoxSet &bs, bool curl, bool upd, bool pml, hipStream_t s) {
   if (pml)
-    launch_fast_t<R, true>(a, curl, upd, s);
+    launch_fast_t<R, true>(a, bs, curl, upd, s);
   else
-    launch_fast_t<R, false>(a, curl, upd, s);
+    launch_fast_t<R, false>(a, bs, curl, upd, s);
 }
 
 template <class R>
@@ -1727,16 +1734,17 @@ __global__ __launch_bounds__(BS) void k_step_batch(const BatchItem<R> *items, co
   const uint32_t t = blk_first[lb] + threadIdx.x;
   if (t >= it.count) return;
   const double *row = vrow + it.a.vofs;
+  const LaunchBox x = item_box(it.a.g, it.g0, it.ngroups);
   if (KIND == 1)
-    fast_body<R, 16 / sizeof(R), CURL, UPD, false, 0>(it.a, t, it.g0, it.ngroups, row);
+    fast_body<R, 16 / sizeof(R), CURL, UPD, false, 0>(it.a, x, t, row);
   else if (KIND == 2)
-    fast_body<R, 16 / sizeof(R), CURL, UPD, true, 0>(it.a, t, it.g0, it.ngroups, row);
+    fast_body<R, 16 / sizeof(R), CURL, UPD, true, 0>(it.a, x, t, row);
   else if (KIND == 3)
-    fast_body<R, 16 / sizeof(R), CURL, UPD, false, MAXPOLE>(it.a, t, it.g0, it.ngroups, row);
+    fast_body<R, 16 / sizeof(R), CURL, UPD, false, MAXPOLE>(it.a, x, t, row);
   else if (KIND == 4)
-    fast_body<R, 16 / sizeof(R), CURL, UPD, true, MAXPOLE>(it.a, t, it.g0, it.ngroups, row);
+    fast_body<R, 16 / sizeof(R), CURL, UPD, true, MAXPOLE>(it.a, x, t, row);
   else
-    step_body<R, CURL, UPD>(it.a, t, row);
+    step_body<R, CURL, UPD>(it.a, x, t, row);
 }
 
 template <class R, int BS, int KIND>
@@ -1792,29 +1800,37 @@ __global__ __launch_bounds__(BLOCK) void k_dft_batch(const BatchDft<R> *items, c
   if (o >= size_t(a.npts) * size_t(nf)) return;
   dft_one<R>(a, o, ph[int(o % size_t(nf))]);
 }
+// The deferred steps of a window: the steps first + 1 .. first + n after the item's t_start, of
+// which those an item accumulates (multiples of its decimation) take consecutive slots of its
+// ring.
 template <class R>
 __global__ __launch_bounds__(BLOCK) void k_dft_snap_batch(const BatchDft<R> *items, const uint32_t *blk_item, const uint32_t *blk_first,
-                                                        int slot) {
+                                                        long first, long n) {
   const BatchDft<R> &it = items[blk_item[blockIdx.x]];
+  const int64_t tt = it.t_start + first + n;
+  if (tt % it.decimation) return;
   const uint32_t p = blk_first[blockIdx.x] + threadIdx.x; // padding blocks start past every item
   if (p >= uint32_t(it.a.npts)) return;
   R f0, f1;
   dft_point(it.a, int(p), f0, f1);
+  const int slot = int(tt / it.decimation - (it.t_start + first) / it.decimation) - 1;
   const size_t o = size_t(slot) * size_t(it.a.npts) + p;
   it.snap0[o] = f0;
   if (it.snap1) it.snap1[o] = f1;
 }
 template <class R>
 __global__ __launch_bounds__(BLOCK) void k_dft_flush_batch(const BatchDft<R> *items, const uint32_t *blk_item, const uint32_t *blk_first,
-                                                         long first, int ns) {
+                                                         long first, long n) {
   __shared__ double2 ph[DFT_FLUSH_TAB];
   const BatchDft<R> &it = items[blk_item[blockIdx.x]];
   const DftArgs<R> &a = it.a;
   const int nf = a.nfreq;
-  if (nf * ns > DFT_FLUSH_TAB) return; // the host keeps such chunks out of deferral
+  const int64_t h0 = (it.t_start + first) / it.decimation;
+  const int ns = int((it.t_start + first + n) / it.decimation - h0);
+  if (ns < 1 || nf * ns > DFT_FLUSH_TAB) return; // the host keeps longer lists out of deferral
   for (int q = threadIdx.x; q < ns * nf; q += BLOCK) {
     const int j = q / nf;
-    const int64_t tt = it.t_start + first + j + 1;
+    const int64_t tt = (h0 + 1 + j) * it.decimation;
     const double time = double(tt) * it.dt - (it.half ? 0.5 * it.dt : 0.0);
     ph[q] = dft_phase(a.omega[q - j * nf], time, a.scale_re, a.scale_im);
   }
@@ -1843,16 +1859,16 @@ __global__ __launch_bounds__(BLOCK) void k_dft_flush_batch(const BatchDft<R> *it
   }
 }
 template <class R>
-void launch_dft_snap_batch(const BatchDft<R> *items, const uint32_t *blk_item, const uint32_t *blk_first, unsigned nblk, int slot,
-                           hipStream_t s) {
-  if (slot < 0 || slot >= DFT_DEFER) throw std::runtime_error("meep: internal: bad deferred DFT slot");
-  if (nblk) hipLaunchKernelGGL(k_dft_snap_batch<R>, dim3(nblk), dim3(BLOCK), 0, s, items, blk_item, blk_first, slot);
+void launch_dft_snap_batch(const BatchDft<R> *items, const uint32_t *blk_item, const uint32_t *blk_first, unsigned nblk, long first,
+                           long n, hipStream_t s) {
+  if (n < 1) throw std::runtime_error("meep: internal: bad deferred DFT slot");
+  if (nblk) hipLaunchKernelGGL(k_dft_snap_batch<R>, dim3(nblk), dim3(BLOCK), 0, s, items, blk_item, blk_first, first, n);
 }
 template <class R>
 void launch_dft_flush_batch(const BatchDft<R> *items, const uint32_t *blk_item, const uint32_t *blk_first, unsigned nblk, long first,
-                            int nsteps, hipStream_t s) {
-  if (nsteps < 1 || nsteps > DFT_DEFER) throw std::runtime_error("meep: internal: bad deferred DFT flush");
-  if (nblk) hipLaunchKernelGGL(k_dft_flush_batch<R>, dim3(nblk), dim3(BLOCK), 0, s, items, blk_item, blk_first, first, nsteps);
+                            long n, hipStream_t s) {
+  if (n < 1) throw std::runtime_error("meep: internal: bad deferred DFT flush");
+  if (nblk) hipLaunchKernelGGL(k_dft_flush_batch<R>, dim3(nblk), dim3(BLOCK), 0, s, items, blk_item, blk_first, first, n);
 }
 template <class R>
 void launch_dft_batch(const BatchDft<R> *items, const uint32_t *blk_item, const uint32_t *blk_first, unsigned nblk, long step,
@@ -1876,12 +1892,12 @@ void launch_conn_batch(const BatchConn *items, const uint32_t *blk_item, const u
   template void launch_step_batch<R>(const BatchItem<R> *, const uint32_t *, const uint32_t *, unsigned, int, bool, bool, int, \
                                      const double *, hipStream_t);                                 \
   template void launch_dft_batch<R>(const BatchDft<R> *, const uint32_t *, const uint32_t *, unsigned, long, hipStream_t); \
-  template void launch_dft_snap_batch<R>(const BatchDft<R> *, const uint32_t *, const uint32_t *, unsigned, int, hipStream_t); \
-  template void launch_dft_flush_batch<R>(const BatchDft<R> *, const uint32_t *, const uint32_t *, unsigned, long, int, hipStream_t); \
+  template void launch_dft_snap_batch<R>(const BatchDft<R> *, const uint32_t *, const uint32_t *, unsigned, long, long, hipStream_t); \
+  template void launch_dft_flush_batch<R>(const BatchDft<R> *, const uint32_t *, const uint32_t *, unsigned, long, long, hipStream_t); \
   template void launch_conn_batch<R>(const BatchConn *, const uint32_t *, const uint32_t *, unsigned, hipStream_t);
 #define INSTANTIATE(R)                                                                             \
-  template void launch_step<R>(const StepArgs<R> &, bool, bool, hipStream_t);                      \
-  template void launch_fast<R>(const StepArgs<R> &, bool, bool, bool, hipStream_t);                \
+  template void launch_step<R>(const StepArgs<R> &, const BoxSet &, bool, bool, hipStream_t);                      \
+  template void launch_fast<R>(const StepArgs<R> &, const BoxSet &, bool, bool, bool, hipStream_t);                \
   template bool launch_row3<R>(const StepArgs<R> &, bool, bool, hipStream_t);                      \
   template void launch_conn<R>(const Conn *, const double2 *, int, R *const *, int, hipStream_t);  \
   template void launch_src<R>(R *, const int64_t *, const double2 *, int, double2, double, int,      \
