@@ -12,7 +12,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OUT_DIR = os.path.join(HERE, "_lib")
 LIB = os.path.join(OUT_DIR, "libmeep_amd.so")
-SOURCES = ["kernels.hip", "adjoint.hip", "near2far.hip", "fields.cpp"]
+SOURCES = ["kernels.hip", "step2d.hip", "adjoint.hip", "near2far.hip", "fields.cpp"]
 SINGLE_UNIT = ("near2far.hip",)  # FP64 whatever the field precision: compiled once
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = ["--offload-arch=gfx950", "-O3", "-fPIC", "-std=c++17",

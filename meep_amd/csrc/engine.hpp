@@ -298,6 +298,90 @@ template <class R>
 void launch_conn_batch(const BatchConn *items, const uint32_t *blk_item, const uint32_t *blk_first, unsigned nblk, hipStream_t s);
 constexpr int BATCH_BLOCKS[4] = {64, 128, 256, 512}; // block sizes the batch autotuner tries
 
+// ---- several steps of a 2D chunk in one launch (step2d.hip) --------------------------------
+// Arrays are double-buffered: a launch reads the first pointer of each pair and writes the
+// second over its tiles' cores; the host swaps the pairs after it.
+constexpr int S2_POLES = 2;   // poles the kernel carries
+constexpr int S2_STEPS = 8;   // most steps of a launch
+constexpr int S2_COLS = 64;   // points of a tile along the stride-1 direction, one per lane
+constexpr int S2_ROWS = 32;   // points of a tile along the other direction
+constexpr int S2_VALS = 128;  // source values of a step that a tile keeps at hand
+constexpr int S2_MONS = 64;   // DFT chunks of a launch's item
+constexpr int S2_ENTRIES = 1024; // monitor points of a tile kept in LDS (more are read each step)
+template <class R> struct S2Comp {
+  const R *f;       // D or B; null: the chunk lacks the component
+  R *fo;
+  const R *e;       // E or H; null where it aliases f
+  R *eo;
+  const double *fu; // uPML auxiliaries, null when absent
+  double *fuo;
+  const double *fw;
+  double *fwo;
+  const R *chi;     // diagonal chi1inv (null: 1)
+  const R *P[S2_POLES], *Pp[S2_POLES], *sigma[S2_POLES];
+  R *Po[S2_POLES], *Ppo[S2_POLES];
+  int sigone;
+  R sigval[S2_POLES];
+  // by axis X, Y: owned range, planes zeroed by a High metallic / Low magnetic wall (-1: none)
+  int lo[2], hi[2], mhi[2], mlo[2];
+};
+// a DFT monitor point of a tile: chunk, point and weight, and its place in the tile
+struct S2Entry {
+  double w;
+  uint32_t k;
+  uint16_t pos, chunk;
+};
+template <class R> struct S2Mon {
+  R *snap;      // the chunk's ring of deferred values
+  uint32_t npts;
+  int fld;      // 0..2 E or H along X, Y, Z; 3..5 the D or B
+  int o1, o2;   // centring offsets within a tile (0: none)
+  int dec;
+};
+// A chunk's tiles and arrays, in device memory (one block per parity of the buffers): read there
+// by the few blocks that need the sources, monitors or poles, so the others' scalar registers
+// stay free.
+template <class R> struct Step2dArgs {
+  int nx, ny;         // cells
+  uint32_t sx;        // row stride
+  int cx, cy;         // core points of a tile
+  int ntx, nty;       // tiles
+  int margin;         // points loaded below the core: the launch's most steps
+  R dtdx;
+  const R *sig[2], *kap[2], *siginv[2];
+  int qlo[2], qhi[2]; // quiet ranges along X and Y
+  S2Comp<R> c[3];     // along X, Y, Z
+  int npole;
+  PoleCoef<R> pole[S2_POLES];
+  const SrcSet *src[2]; // B and D phase; null: none
+  int sbox_lo[2][2], sbox_hi[2][2]; // [phase][axis]
+  int64_t vofs;       // batches: this chunk's offset in the step's value row
+  int cmp;
+  const uint32_t *mon_first; // per tile, entries mon_first[q] .. mon_first[q + 1]; null: no monitors
+  const S2Entry *mon;
+  const S2Mon<R> *mons;
+  int monmask;        // fields some monitor reads (bits as S2Mon::fld)
+  int nmon;           // DFT chunks
+  int64_t t0;         // step count that Step2dLaunch::s counts from
+};
+// what changes from launch to launch
+template <class R> struct Step2dLaunch {
+  const Step2dArgs<R> *items;
+  const uint32_t *blk_item, *blk_tile; // the blocks' chunks and tiles; null: the tiles of items[0]
+  uint32_t ntile;     // tiles of the launch
+  int nsteps;
+  const double *vrow; // the first step's source values
+  int64_t rl;         // the values of an item's step
+  int64_t stride;     // and from one step to the next
+  int64_t s, w;       // step counts before the launch, and before the open deferral window
+  int hits;           // some monitor accumulates in these steps
+  R *rec;             // reverse-mode history of one D component on a box: null, or the first step's
+  int rec_c, rec_lo[2], rec_hi[2];
+};
+// tm: Ez, Hx, Hy (else Hz, Ex, Ey); npole: the most poles of an item; monmask: fields that the
+// items' monitors read together
+template <class R> void launch_step2d(const Step2dLaunch<R> &l, bool tm, int npole, int monmask, hipStream_t s);
+
 // ---- reverse-mode step (adjoint.hip) -------------------------------------------------------
 // The adjoint of one step applies the transpose of each forward update, in reverse order, to
 // cotangent arrays ("bar" arrays, one per forward state array, aliased as the forward arrays

@@ -2185,6 +2185,395 @@ template <class R> struct Fields : FieldsBase {
                       static_cast<const double *>(d_chk_w.p), n_chk, static_cast<int *>(d_flag.p), stream);
   }
 
+  // ---- several steps of a 2D chunk per launch (step2d.hip) --------------------------------
+  // n steps: the tile kernel where it takes the chunk, one_step elsewhere (a call's first steps
+  // after a change, which allocate; a step left over; the last step where flux planes read it)
+  void advance(long n, bool probe) {
+    for (long q = 0; q < n;) {
+      const long tail = probe && !flux_vols.empty() ? 1 : 0;
+      if (n - q - tail >= 2 && s2_ready()) {
+        const long did = s2_run(n - q - tail);
+        q += did;
+        if (did) {
+          if (q == n && probe) probe_on(stream);
+          continue;
+        }
+      }
+      rows_hint = n - q;
+      one_step(probe && q == n - 1);
+      ++q;
+    }
+  }
+  struct S2Set { // one polarisation: its launch arguments by part (real, imaginary) and parity
+    bool tm;
+    Step2dArgs<R> a[2][2];
+    DevBuf args, mon_first, mon, mons[2]; // args: a, row by row
+    const Step2dArgs<R> *dev(int cmp, int parity) const { return static_cast<const Step2dArgs<R> *>(args.p) + 2 * cmp + parity; }
+  };
+  struct S2Plan {
+    long plan_v = -1, dft_v = -1, src_v = -1, ptr_v = -1;
+    bool ok = false;
+    std::vector<std::unique_ptr<S2Set>> sets;
+  } s2;
+  std::map<const void *, std::unique_ptr<DevBuf>> s2_alt; // each state array's second buffer
+  bool s2_off = getenv("MEEP_AMD_NO_TILE2D") != nullptr;
+  bool s2_nomem = false;
+  // the second buffer of a state array, made as a copy of it; null when memory is short
+  template <class T> T *s2_second(const T *p) {
+    std::unique_ptr<DevBuf> &b = s2_alt[p];
+    if (!b) {
+      std::unique_ptr<DevBuf> n(new DevBuf);
+      if (hipMalloc(&n->p, sizeof(T) * gv.ntot) != hipSuccess) {
+        (void)hipGetLastError();
+        n->p = nullptr;
+        s2_nomem = true;
+        return nullptr;
+      }
+      n->bytes = sizeof(T) * gv.ntot;
+      HIPCHECK(hipMemcpyAsync(n->p, p, sizeof(T) * gv.ntot, hipMemcpyDeviceToDevice, stream));
+      b = std::move(n);
+    }
+    return static_cast<T *>(b->p);
+  }
+  // Whether the tile kernel takes this chunk's next steps: 2D, no periodic halos, no
+  // conductivity, no magnetic poles and at most S2_POLES electric ones, every source in a table
+  // or box, every DFT chunk in the deferred group, and nothing left to allocate.
+  bool s2_ready() {
+    if (s2_off || gv.dim != 2 || !use_fast || whole_rows_env >= 0 || !(dft_defer_steps || dft_off)) return false;
+    if (!plan_valid || srcplan_stale() || t > INT32_MAX / 2) return false;
+    if (s2.plan_v == plan_version && s2.dft_v == dft_version && s2.src_v == src_version && s2.ptr_v == ptr_version) return s2.ok;
+    s2.plan_v = plan_version;
+    s2.dft_v = dft_version;
+    s2.src_v = src_version;
+    s2.ptr_v = ptr_version;
+    s2.ok = false;
+    s2.sets.clear();
+    if (any_cond || n_conn[0] || n_conn[1] || wrap_dir[0] || wrap_dir[1] || have_fmp_H() || int(pols.size()) > S2_POLES) return false;
+    for (auto &p : pols)
+      if (!p.allocated) return false;
+    bool fmp = false;
+    for (auto &sv : sources[B_ft])
+      if (srcs[sv.src].is_integrated) return false;
+    for (auto &sv : sources[D_ft]) fmp = fmp || srcs[sv.src].is_integrated;
+    for (auto &p : pols)
+      for (int c = 0; c < 5; ++c)
+        for (int cmp = 0; cmp < ncmp(); ++cmp) fmp = fmp || needs_P(p, c, cmp);
+    for (int ph = 0; ph < 2; ++ph)
+      for (int cmp = 0; cmp < ncmp(); ++cmp) {
+        if (!splan.L[ph][cmp].rest_cur.empty() || !splan.L[ph][cmp].rest_dip.empty()) return false;
+        int which[3];
+        slot_comps(ph ? D_ft : B_ft, cmp, which);
+        if (upd_pending(cmp, which, 3, ph && fmp)) return false;
+      }
+    if (splan.rec.size() > S2_VALS || dft_chunks.size() > S2_MONS) return false;
+    if (!dft_chunks.empty() && !dft_group()) return false;
+    for (auto &cp : dft_chunks)
+      if (!f[cp->c][0]) return false;
+    if (!boxes_valid) compute_boxes();
+    for (int pol = 0; pol < 2; ++pol) {
+      const bool tm = pol == 0;
+      int have = 0;
+      for (int d = 0; d < 3; ++d) have += f[dir_comp(tm == (d == 2) ? 10 : 15, d)][0] != nullptr;
+      if (!have) continue;
+      if (have != 3 || !s2_set(tm, fmp)) return false;
+    }
+    if (s2_nomem) { // no room for the second buffers: one step per launch
+      HIPCHECK(hipStreamSynchronize(stream));
+      s2.sets.clear();
+      s2_alt.clear();
+      s2_off = true;
+      return false;
+    }
+    return s2.ok = !s2.sets.empty();
+  }
+  // the launch arguments and monitor tables of one polarisation; false when its plan has
+  // another shape than the kernel's
+  bool s2_set(bool tm, bool fmp) {
+    std::unique_ptr<S2Set> S(new S2Set);
+    S->tm = tm;
+    const int margin = s2_margin();
+    for (int cmp = 0; cmp < ncmp(); ++cmp) {
+      StepArgs<R> AB = base_args(), AD = base_args();
+      int wB[3], wD[3];
+      AB.nc = curl_comps(B_ft, cmp, AB.cc, wB);
+      upd_comps(H_ft, cmp, wB, AB.nc, AB.uc, false);
+      AD.nc = curl_comps(D_ft, cmp, AD.cc, wD);
+      upd_comps(E_ft, cmp, wD, AD.nc, AD.uc, fmp);
+      if (!plan_valid) fail("internal: arrays still to allocate for the tile kernel");
+      AD.npole = int(pols.size());
+      for (int p = 0; p < AD.npole; ++p) AD.pole[p] = pols[p].coef;
+      if (!fast_partners(B_ft, cmp, AB) || !fast_partners(D_ft, cmp, AD)) return false;
+      finalize_args(AB);
+      finalize_args(AD);
+      AB.src = AD.src = nullptr;
+      check_args(AB, true, true, true);
+      check_args(AD, true, true, true);
+      Step2dArgs<R> &a = S->a[cmp][0];
+      memset(&a, 0, sizeof a);
+      const Grid &g = AD.g;
+      a.nx = gv.num[0];
+      a.ny = gv.num[1];
+      if (gv.st[1] != 1 || gv.ntot >= (size_t(1) << 32)) return false;
+      a.sx = uint32_t(gv.st[0]);
+      a.margin = margin;
+      a.ntx = (a.nx + 1 + S2_ROWS - 2 * margin - 2) / (S2_ROWS - 2 * margin - 1);
+      a.nty = (a.ny + 1 + S2_COLS - 2 * margin - 2) / (S2_COLS - 2 * margin - 1);
+      a.cx = (a.nx + a.ntx) / a.ntx;
+      a.cy = (a.ny + a.nty) / a.nty;
+      if (size_t(a.ntx) * size_t(a.nty) >= (size_t(1) << 30)) return false;
+      a.dtdx = AD.dtdx;
+      for (int d = 0; d < 2; ++d) {
+        a.sig[d] = AD.pml.sig[d];
+        a.kap[d] = AD.pml.kap[d];
+        a.siginv[d] = AD.pml.siginv[d];
+        a.qlo[d] = g.qlo[1 + d];
+        a.qhi[d] = g.qhi[1 + d];
+      }
+      a.npole = AD.npole;
+      for (int p = 0; p < a.npole; ++p) a.pole[p] = AD.pole[p];
+      a.cmp = cmp;
+      for (int ph = 0; ph < 2; ++ph) {
+        StepArgs<R> A;
+        set_batch_sources(A, ph, cmp, 0);
+        a.src[ph] = A.src;
+        for (int q = 0; q < 2; ++q) a.sbox_lo[ph][q] = A.sbox_lo[1 + q], a.sbox_hi[ph][q] = A.sbox_hi[1 + q];
+      }
+      for (int d = 0; d < 3; ++d) {
+        const bool mag = tm != (d == 2);
+        const StepArgs<R> &A = mag ? AB : AD;
+        const CurlComp<R> &k = A.cc[d];
+        const UpdComp<R> &u = A.uc[d];
+        S2Comp<R> &c = a.c[d];
+        if (!k.f || k.cnd) return false;
+        // the 2D plan: along X uPML acts through dsig = Y and dsigw = X, along Y through
+        // dsigu = X and dsigw = Y, along Z through dsig = X and dsigu = Y; each curl takes the
+        // partner differences that exist
+        const int px = pml_in(0) ? 0 : -1, py = pml_in(1) ? 1 : -1;
+        if (k.dsig != (d == 0 ? py : d == 2 ? px : -1) || k.dsigu != (d == 1 ? px : d == 2 ? py : -1)) return false;
+        if (A.hasp[d] != (d == 1 ? 0 : 1) || A.hasm[d] != (d == 0 ? 0 : 1)) return false;
+        if (u.f && u.dsigw != (d == 0 ? px : d == 1 ? py : -1)) return false;
+        if (!u.f && d < 2 && pml_in(d)) return false;
+        if ((k.dsigu >= 0 && !k.fu) || (u.f && u.dsigw >= 0 && !u.fw)) return false;
+        c.f = k.f;
+        c.fo = s2_second(k.f);
+        if (u.f) {
+          c.e = u.f;
+          c.eo = s2_second(static_cast<const R *>(u.f));
+          c.chi = u.u;
+        }
+        if (k.dsigu >= 0) c.fu = k.fu, c.fuo = s2_second(static_cast<const double *>(k.fu));
+        if (u.f && u.dsigw >= 0) c.fw = u.fw, c.fwo = s2_second(static_cast<const double *>(u.fw));
+        if (!mag && u.f)
+          for (int p = 0; p < a.npole; ++p) {
+            if (!u.P[p]) continue;
+            c.P[p] = u.P[p];
+            c.Pp[p] = u.Pp[p];
+            c.Po[p] = s2_second(static_cast<const R *>(u.P[p]));
+            c.Ppo[p] = s2_second(static_cast<const R *>(u.Pp[p]));
+            c.sigma[p] = u.sigma[p];
+            c.sigval[p] = u.sigval[p];
+            if ((u.sigone >> p) & 1) c.sigone |= 1 << p;
+          }
+        const AxisSlot &ax = k.ax; // loop axes 1 and 2 are X and Y
+        for (int q = 0; q < 2; ++q) c.lo[q] = ax.lo[1 + q], c.hi[q] = ax.hi[1 + q], c.mhi[q] = ax.mhi[1 + q], c.mlo[q] = ax.mlo[1 + q];
+      }
+    }
+    s2_monitors(*S);
+    for (int cmp = 0; cmp < ncmp(); ++cmp) { // the other parity: every pair exchanged
+      s2_check(S->a[cmp][0]);
+      S->a[cmp][1] = S->a[cmp][0];
+      for (S2Comp<R> &c : S->a[cmp][1].c) {
+        auto swap = [](auto *&in, auto *&out) {
+          auto *o = out;
+          out = const_cast<std::remove_const_t<std::remove_pointer_t<std::remove_reference_t<decltype(in)>>> *>(in);
+          in = o;
+        };
+        swap(c.f, c.fo);
+        swap(c.e, c.eo);
+        swap(c.fu, c.fuo);
+        swap(c.fw, c.fwo);
+        for (int p = 0; p < S2_POLES; ++p) swap(c.P[p], c.Po[p]), swap(c.Pp[p], c.Ppo[p]);
+      }
+    }
+    std::vector<Step2dArgs<R>> all;
+    for (int cmp = 0; cmp < 2; ++cmp)
+      for (int par = 0; par < 2; ++par) all.push_back(S->a[cmp][par]);
+    upload_vec(S->args, all);
+    s2.sets.push_back(std::move(S));
+    return true;
+  }
+  // every pointer the tile kernel can dereference, and the tiles against its registers and lanes
+  static void s2_check(const Step2dArgs<R> &a) {
+    bool ok = a.margin >= 1 && a.cx >= 1 && a.cx + 2 * a.margin + 1 <= S2_ROWS && a.cy >= 1 && a.cy + 2 * a.margin + 1 <= S2_COLS &&
+              a.npole <= S2_POLES && a.ntx * a.cx > a.nx && a.nty * a.cy > a.ny;
+    for (int c = 0; c < 3; ++c) {
+      ok = ok && a.c[c].f && a.c[c].fo && (!a.c[c].e || a.c[c].eo);
+      for (int p = 0; p < a.npole; ++p)
+        if (a.c[c].P[p]) ok = ok && a.c[c].Pp[p] && a.c[c].Po[p] && a.c[c].Ppo[p] && a.c[c].e;
+    }
+    if (a.sig[0]) ok = ok && a.c[1].fu && a.c[1].fuo && a.c[0].fw && a.c[0].fwo && a.c[0].e;
+    if (a.sig[1]) ok = ok && a.c[2].fu && a.c[2].fuo && a.c[1].fw && a.c[1].fwo && a.c[1].e;
+    if (!ok) fail("internal: bad 2D tile plan");
+  }
+  // steps a tile has room for: 8 against 3, 4 and 6 took 1.97 / 3.7, 3.0, 2.9 ms for 400 steps of
+  // a 320 x 160 FP64 cell (the launch and the tile load cost as much as four steps)
+  int s2_margin() const { return S2_STEPS; }
+  // the monitor points of each tile
+  void s2_monitors(S2Set &S) {
+    Step2dArgs<R> &a = S.a[0][0];
+    const size_t nt = size_t(a.ntx) * size_t(a.nty);
+    std::vector<std::vector<S2Entry>> lists(nt);
+    std::vector<S2Mon<R>> mons[2];
+    int mask = 0;
+    for (auto &cp : dft_chunks) {
+      DftChunk<R> &ch = *cp;
+      const int d = comp_dir(ch.c);
+      const bool mag = is_magnetic(ch.c) || is_B(ch.c);
+      if ((S.tm != (d == 2)) != mag) continue; // of the other polarisation
+      S2Mon<R> m;
+      memset(&m, 0, sizeof m);
+      m.npts = uint32_t(ch.npts);
+      m.fld = d + (is_D(ch.c) || is_B(ch.c) ? 3 : 0);
+      m.dec = ch.decimation;
+      auto off = [&](int64_t o) {
+        if (o != 0 && o != 1 && o != gv.st[0]) fail("internal: DFT centring offset");
+        return o == 0 ? 0 : o == 1 ? 1 : S2_COLS;
+      };
+      m.o1 = off(ch.avg1);
+      m.o2 = off(ch.avg2);
+      mask |= 1 << m.fld;
+      const size_t ci = mons[0].size();
+      m.snap = static_cast<R *>(ch.snap.p);
+      mons[0].push_back(m);
+      m.snap += size_t(DFT_DEFER) * size_t(ch.npts);
+      mons[1].push_back(m);
+      std::vector<int64_t> idx(size_t(ch.npts));
+      std::vector<double> w(size_t(ch.npts));
+      HIPCHECK(hipMemcpy(idx.data(), ch.idx.p, sizeof(int64_t) * idx.size(), hipMemcpyDeviceToHost));
+      HIPCHECK(hipMemcpy(w.data(), ch.w.p, sizeof(double) * w.size(), hipMemcpyDeviceToHost));
+      for (size_t k = 0; k < idx.size(); ++k) {
+        const int x = int(idx[k] / gv.st[0]), y = int(idx[k] % gv.st[0]);
+        if (x < 0 || x > a.nx || y < 0 || y > a.ny) fail("internal: DFT point outside the grid");
+        const int tx = x / a.cx, ty = y / a.cy;
+        const int lx = x - tx * a.cx + a.margin, ly = y - ty * a.cy + a.margin;
+        if (tx >= a.ntx || ty >= a.nty || lx + 1 >= S2_ROWS || ly + 1 >= S2_COLS) fail("internal: DFT point outside its tile");
+        S2Entry e;
+        memset(&e, 0, sizeof e);
+        e.w = w[k];
+        e.k = uint32_t(k);
+        e.pos = uint16_t(lx * S2_COLS + ly);
+        e.chunk = uint16_t(ci);
+        lists[size_t(tx) * size_t(a.nty) + size_t(ty)].push_back(e);
+      }
+    }
+    if (mons[0].empty()) return;
+    std::vector<uint32_t> first(1, 0);
+    std::vector<S2Entry> all;
+    for (auto &l : lists) {
+      all.insert(all.end(), l.begin(), l.end());
+      first.push_back(uint32_t(all.size()));
+    }
+    upload_vec(S.mon_first, first);
+    upload_vec(S.mon, all);
+    for (int cmp = 0; cmp < ncmp(); ++cmp) {
+      upload_vec(S.mons[cmp], mons[cmp]);
+      Step2dArgs<R> &b = S.a[cmp][0];
+      b.mon_first = static_cast<const uint32_t *>(S.mon_first.p);
+      b.mon = static_cast<const S2Entry *>(S.mon.p);
+      b.mons = static_cast<const S2Mon<R> *>(S.mons[cmp].p);
+      b.monmask = mask;
+      b.nmon = int(mons[cmp].size());
+    }
+  }
+  // Up to m steps by the tile kernel; returns the steps taken.  The launches of a call come in
+  // an even number, so that the state ends where every other reader has it: a last launch that
+  // would leave it in the second buffers is split in two, and a single step is left to the
+  // caller.  Launches end where the reverse mode keeps a checkpoint or starts a history block,
+  // and where the open window of deferred DFT steps is full.
+  long s2_run(long m) {
+    const long m0 = m;
+    int parity = 0;
+    while (m > 0) {
+      long T = std::min<long>(m, s2_margin());
+      const bool rec = adj && adj->recording;
+      if (rec) {
+        Adj &A = *adj;
+        if (A.interval > 0 && !seg_active)
+          T = std::min(T, A.interval - (t - A.t0) % A.interval);
+        else if (A.interval <= 0)
+          T = std::min(T, HBLK - A.nrec % HBLK);
+      }
+      const bool dft = !dft_chunks.empty() && !dft_off;
+      if (dft) {
+        const long w = window_open ? window_t : t;
+        while (T > 1 && dgroup.most_hits(w, t + T) > DFT_DEFER) --T;
+      }
+      if (T == m && parity == 0) {
+        if (m == 1) break;
+        T = (m + 1) / 2;
+      }
+      rows_hint = m;
+      const double *row = src_row(t);
+      if (row && t + T > rows_t0 + rows_n) fail("internal: source rows shorter than the tile kernel's steps");
+      const bool hits = dft && dgroup.hits(t, t + T);
+      if (hits && !window_open) window_open = true, window_t = t;
+      kbegin(MP_K_STEP_DE);
+      for (auto &S : s2.sets)
+        for (int cmp = 0; cmp < ncmp(); ++cmp) {
+          const Step2dArgs<R> &a = S->a[cmp][parity];
+          Step2dLaunch<R> l;
+          memset(&l, 0, sizeof l);
+          l.items = S->dev(cmp, parity);
+          l.ntile = uint32_t(a.ntx) * uint32_t(a.nty);
+          l.nsteps = int(T);
+          l.vrow = row;
+          l.rl = l.stride = int64_t(splan.rec.size());
+          l.s = t;
+          l.w = window_open ? window_t : t;
+          l.hits = hits && a.mon_first;
+          if (rec && cmp == 0) s2_record(*S, l, T);
+          launch_step2d<R>(l, S->tm, a.npole, a.monmask, stream);
+        }
+      kend();
+      parity ^= 1;
+      t += T;
+      m -= T;
+      if (rec) {
+        adj->nrec += T;
+        if (adj->interval > 0 && !seg_active && (t - adj->t0) % adj->interval == 0) save_checkpoint(parity != 0);
+      }
+      if (hits) {
+        window_end = t;
+        if (dgroup.most_hits(window_t, t) == DFT_DEFER) {
+          kbegin(MP_K_DFT);
+          flush_dft_group();
+          kend();
+        }
+      }
+    }
+    return m0 - m;
+  }
+  // where the T recorded steps from now go, for the set that holds the design's component
+  void s2_record(const S2Set &S, Step2dLaunch<R> &a, long T) {
+    Adj &A = *adj;
+    const int d = comp_dir(A.c);
+    if (S.tm != (d == 2)) return;
+    if (A.interval > 0) {
+      if (!seg_active) return;
+      a.rec = static_cast<R *>(A.seg.p) + size_t(A.nrec - seg_first) * A.npts;
+    }
+    else {
+      if (size_t(A.nrec / HBLK) >= A.hist.size()) {
+        A.hist.emplace_back(new DevBuf);
+        A.hist.back()->alloc(sizeof(R) * A.npts * HBLK);
+      }
+      if (A.nrec % HBLK + T > HBLK) fail("internal: recorded steps cross a history block");
+      a.rec = static_cast<R *>(A.hist[size_t(A.nrec / HBLK)]->p) + size_t(A.nrec % HBLK) * A.npts;
+    }
+    a.rec_c = d;
+    for (int q = 0; q < 2; ++q) a.rec_lo[q] = A.lo[1 + q], a.rec_hi[q] = A.hi[1 + q];
+  }
+
   StepArgs<R> base_args() const {
     StepArgs<R> A;
     memset(&A, 0, sizeof A);
@@ -2547,14 +2936,20 @@ template <class R> struct Fields : FieldsBase {
     }
   }
   void adj_end() override { adj.reset(); }
-  void save_checkpoint() {
+  // second: the state stands in the tile kernel's second buffers
+  void save_checkpoint(bool second = false) {
     HIPCHECK(hipStreamSynchronize(stream));
     typename Adj::Checkpoint cp;
     cp.t = t;
     for (const StateArr &a : state_arrays()) {
       cp.data.emplace_back(new DevBuf);
       cp.data.back()->alloc(a.esz * gv.ntot);
-      HIPCHECK(hipMemcpyAsync(cp.data.back()->p, a.p, a.esz * gv.ntot, hipMemcpyDeviceToDevice, stream));
+      const void *from = a.p;
+      if (second) {
+        auto it = s2_alt.find(a.p);
+        if (it != s2_alt.end()) from = it->second->p;
+      }
+      HIPCHECK(hipMemcpyAsync(cp.data.back()->p, from, a.esz * gv.ntot, hipMemcpyDeviceToDevice, stream));
     }
     adj->cps.push_back(std::move(cp));
   }
@@ -2800,10 +3195,7 @@ template <class R> struct Fields : FieldsBase {
         A.nrec = first;
         dft_off = true;
         A.recording = true;
-        for (long q = first; q < last; ++q) {
-          rows_hint = last - q;
-          one_step(false);
-        }
+        advance(last - first, false);
         dft_off = false;
         seg_active = false;
         for (long n = last - 1; n >= first; --n)
@@ -2932,10 +3324,7 @@ template <class R> struct Fields : FieldsBase {
     rows_free = true;
     // the reference checks after every step (src/step.cpp:137-138); a batch probes its last step
     dft_defer_steps = n > 1;
-    for (long q = 0; q < n; ++q) {
-      rows_hint = n - q;
-      one_step(q == n - 1);
-    }
+    advance(n, true);
     flush_dfts(); // every deferred DFT step reaches the accumulators before the call returns
     dft_defer_steps = false;
     HIPCHECK(hipStreamSynchronize(stream));
