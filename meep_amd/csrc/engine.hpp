@@ -356,6 +356,7 @@ template <class R> struct Step2dArgs {
   const SrcSet *src[2]; // B and D phase; null: none
   int sbox_lo[2][2], sbox_hi[2][2]; // [phase][axis]
   int64_t vofs;       // batches: this chunk's offset in the step's value row
+  int rl;             // and its values there
   int cmp;
   const uint32_t *mon_first; // per tile, entries mon_first[q] .. mon_first[q + 1]; null: no monitors
   const S2Entry *mon;
@@ -371,8 +372,7 @@ template <class R> struct Step2dLaunch {
   uint32_t ntile;     // tiles of the launch
   int nsteps;
   const double *vrow; // the first step's source values
-  int64_t rl;         // the values of an item's step
-  int64_t stride;     // and from one step to the next
+  int64_t stride;     // and the values from one step to the next
   int64_t s, w;       // step counts before the launch, and before the open deferral window
   int hits;           // some monitor accumulates in these steps
   R *rec;             // reverse-mode history of one D component on a box: null, or the first step's

@@ -2191,7 +2191,7 @@ template <class R> struct Fields : FieldsBase {
   void advance(long n, bool probe) {
     for (long q = 0; q < n;) {
       const long tail = probe && !flux_vols.empty() ? 1 : 0;
-      if (n - q - tail >= 2 && s2_ready()) {
+      if (n - q - tail >= 2 && (dft_defer_steps || dft_off) && s2_ready(S2_STEPS)) {
         const long did = s2_run(n - q - tail);
         q += did;
         if (did) {
@@ -2211,7 +2211,8 @@ template <class R> struct Fields : FieldsBase {
     const Step2dArgs<R> *dev(int cmp, int parity) const { return static_cast<const Step2dArgs<R> *>(args.p) + 2 * cmp + parity; }
   };
   struct S2Plan {
-    long plan_v = -1, dft_v = -1, src_v = -1, ptr_v = -1;
+    long plan_v = -1, dft_v = -1, src_v = -1, ptr_v = -1, builds = 0;
+    int margin = 0; // steps a tile has room for
     bool ok = false;
     std::vector<std::unique_ptr<S2Set>> sets;
   } s2;
@@ -2238,10 +2239,13 @@ template <class R> struct Fields : FieldsBase {
   // Whether the tile kernel takes this chunk's next steps: 2D, no periodic halos, no
   // conductivity, no magnetic poles and at most S2_POLES electric ones, every source in a table
   // or box, every DFT chunk in the deferred group, and nothing left to allocate.
-  bool s2_ready() {
-    if (s2_off || gv.dim != 2 || !use_fast || whole_rows_env >= 0 || !(dft_defer_steps || dft_off)) return false;
+  bool s2_ready(int margin) {
+    if (s2_off || gv.dim != 2 || !use_fast || whole_rows_env >= 0) return false;
     if (!plan_valid || srcplan_stale() || t > INT32_MAX / 2) return false;
-    if (s2.plan_v == plan_version && s2.dft_v == dft_version && s2.src_v == src_version && s2.ptr_v == ptr_version) return s2.ok;
+    if (s2.plan_v == plan_version && s2.dft_v == dft_version && s2.src_v == src_version && s2.ptr_v == ptr_version && s2.margin == margin)
+      return s2.ok;
+    s2.margin = margin;
+    ++s2.builds;
     s2.plan_v = plan_version;
     s2.dft_v = dft_version;
     s2.src_v = src_version;
@@ -2291,7 +2295,7 @@ template <class R> struct Fields : FieldsBase {
   bool s2_set(bool tm, bool fmp) {
     std::unique_ptr<S2Set> S(new S2Set);
     S->tm = tm;
-    const int margin = s2_margin();
+    const int margin = s2.margin;
     for (int cmp = 0; cmp < ncmp(); ++cmp) {
       StepArgs<R> AB = base_args(), AD = base_args();
       int wB[3], wD[3];
@@ -2332,6 +2336,7 @@ template <class R> struct Fields : FieldsBase {
       a.npole = AD.npole;
       for (int p = 0; p < a.npole; ++p) a.pole[p] = AD.pole[p];
       a.cmp = cmp;
+      a.rl = int(splan.rec.size());
       for (int ph = 0; ph < 2; ++ph) {
         StepArgs<R> A;
         set_batch_sources(A, ph, cmp, 0);
@@ -2415,9 +2420,6 @@ template <class R> struct Fields : FieldsBase {
     if (a.sig[1]) ok = ok && a.c[2].fu && a.c[2].fuo && a.c[1].fw && a.c[1].fwo && a.c[1].e;
     if (!ok) fail("internal: bad 2D tile plan");
   }
-  // steps a tile has room for: 8 against 3, 4 and 6 took 1.97 / 3.7, 3.0, 2.9 ms for 400 steps of
-  // a 320 x 160 FP64 cell (the launch and the tile load cost as much as four steps)
-  int s2_margin() const { return S2_STEPS; }
   // the monitor points of each tile
   void s2_monitors(S2Set &S) {
     Step2dArgs<R> &a = S.a[0][0];
@@ -2494,7 +2496,9 @@ template <class R> struct Fields : FieldsBase {
     const long m0 = m;
     int parity = 0;
     while (m > 0) {
-      long T = std::min<long>(m, s2_margin());
+      // 8 steps a launch against 3, 4 and 6: 1.97 / 3.7, 3.0, 2.9 ms for 400 steps of a 320 x 160
+      // FP64 cell (the launch and the tile load cost as much as four steps)
+      long T = std::min<long>(m, s2.margin);
       const bool rec = adj && adj->recording;
       if (rec) {
         Adj &A = *adj;
@@ -2527,7 +2531,7 @@ template <class R> struct Fields : FieldsBase {
           l.ntile = uint32_t(a.ntx) * uint32_t(a.nty);
           l.nsteps = int(T);
           l.vrow = row;
-          l.rl = l.stride = int64_t(splan.rec.size());
+          l.stride = int64_t(splan.rec.size());
           l.s = t;
           l.w = window_open ? window_t : t;
           l.hits = hits && a.mon_first;
@@ -4870,6 +4874,118 @@ template <class R> struct Batch : BatchBase {
     }
     planned = true;
   }
+  // ---- the tile kernel (step2d.hip) over all chunks ----
+  // Used when it takes every chunk: one launch steps every tile of every chunk of a polarisation
+  // and pole count several times.  Tiles have room for S2_BATCH steps: a batch fills the chip many
+  // times over, so the share of a tile that is core counts as well as the launch and the load.
+  static constexpr int S2_BATCH = 6;
+  struct TileGroup {
+    bool tm;
+    int npole, monmask = 0;
+    std::vector<Step2dArgs<R>> host[2]; // by parity
+    std::vector<size_t> sim;
+    DevBuf items[2], blk_item, blk_tile;
+    uint32_t ntile = 0;
+  };
+  std::vector<std::unique_ptr<TileGroup>> tgroups;
+  std::vector<long> tile_builds;
+  std::vector<int> tile_decs;
+  bool tiles_ready() {
+    bool fresh = tile_builds.size() == sims.size();
+    for (Fields<R> *F : sims)
+      if (!F->s2_ready(S2_BATCH)) {
+        tile_builds.clear();
+        return false;
+      }
+    for (size_t q = 0; q < sims.size() && fresh; ++q) fresh = tile_builds[q] == sims[q]->s2.builds;
+    if (fresh) return true;
+    tgroups.clear();
+    tile_builds.clear();
+    tile_decs.clear();
+    std::map<int, TileGroup *> by;
+    for (size_t q = 0; q < sims.size(); ++q) {
+      Fields<R> *F = sims[q];
+      tile_builds.push_back(F->s2.builds);
+      for (int d : F->dft_chunks.empty() ? std::vector<int>() : F->dgroup.decs)
+        if (std::find(tile_decs.begin(), tile_decs.end(), d) == tile_decs.end()) tile_decs.push_back(d);
+      for (auto &S : F->s2.sets)
+        for (int cmp = 0; cmp < F->ncmp(); ++cmp) {
+          const int key = 2 * S->a[cmp][0].npole + (S->tm ? 1 : 0);
+          TileGroup *&g = by[key];
+          if (!g) {
+            tgroups.emplace_back(g = new TileGroup);
+            g->tm = S->tm;
+            g->npole = S->a[cmp][0].npole;
+          }
+          for (int par = 0; par < 2; ++par) {
+            g->host[par].push_back(S->a[cmp][par]);
+            g->host[par].back().vofs = int64_t(row_off[q]);
+          }
+          g->sim.push_back(q);
+          g->monmask |= S->a[cmp][0].monmask;
+        }
+      HIPCHECK(hipStreamSynchronize(F->stream)); // the second buffers are copies made there
+    }
+    for (auto &g : tgroups) {
+      std::vector<uint32_t> item, tile;
+      for (size_t k = 0; k < g->host[0].size(); ++k)
+        for (uint32_t b = 0; b < uint32_t(g->host[0][k].ntx) * uint32_t(g->host[0][k].nty); ++b) {
+          item.push_back(uint32_t(k));
+          tile.push_back(b);
+        }
+      g->ntile = uint32_t(item.size());
+      upload_vec(g->blk_item, item);
+      upload_vec(g->blk_tile, tile);
+    }
+    return true;
+  }
+  long tile_hits(long t0, long t1) const { // most accumulations of a chunk in steps t0 + 1 .. t1 of the call
+    long m = 0;
+    for (Fields<R> *F : sims)
+      for (int d : tile_decs) m = std::max(m, (F->t + t1) / d - (F->t + t0) / d);
+    return m;
+  }
+  // the m >= 2 steps of a call, an even number of launches (the state ends in its own buffers)
+  void run_tiles(long m, const double *vrow, int64_t stride) {
+    for (auto &g : tgroups)
+      for (int par = 0; par < 2; ++par) {
+        for (size_t k = 0; k < g->sim.size(); ++k) g->host[par][k].t0 = sims[g->sim[k]]->t;
+        upload_vec(g->items[par], g->host[par]);
+      }
+    long nl = (m + S2_BATCH - 1) / S2_BATCH;
+    nl += nl & 1;
+    long s = 0, w = 0;
+    bool open = false;
+    auto flush = [&] {
+      if (!open) return;
+      launch_dft_flush_batch<R>(static_cast<const BatchDft<R> *>(dft_items.p), static_cast<const uint32_t *>(dft_flush_item.p),
+                                static_cast<const uint32_t *>(dft_flush_first.p), dft_flush_nblk, w, s - w, stream);
+      open = false;
+    };
+    for (long q = 0; q < nl; ++q) {
+      const long T = m / nl + (q < m % nl ? 1 : 0);
+      if (open && tile_hits(w, s + T) > DFT_DEFER) flush();
+      const bool hits = !tile_decs.empty() && tile_hits(s, s + T) > 0;
+      if (hits && !open) open = true, w = s;
+      for (auto &g : tgroups) {
+        Step2dLaunch<R> l;
+        memset(&l, 0, sizeof l);
+        l.items = static_cast<const Step2dArgs<R> *>(g->items[q & 1].p);
+        l.blk_item = static_cast<const uint32_t *>(g->blk_item.p);
+        l.blk_tile = static_cast<const uint32_t *>(g->blk_tile.p);
+        l.ntile = g->ntile;
+        l.nsteps = int(T);
+        l.vrow = vrow + s * stride;
+        l.stride = stride;
+        l.s = s;
+        l.w = open ? w : s;
+        l.hits = hits;
+        launch_step2d<R>(l, g->tm, g->npole, g->monmask, stream);
+      }
+      s += T;
+    }
+    flush();
+  }
   void launch_step(long s, int bidx, const double *vrow) {
     for (int phase = 0; phase < 2; ++phase) {
       for (auto &gp : groups)
@@ -4923,6 +5039,12 @@ template <class R> struct Batch : BatchBase {
     }
     const double *drows = static_cast<const double *>(rows.p);
     call_steps = m;
+    if (m >= 2 && (dft_host.empty() || dft_defer) && tiles_ready()) {
+      auto t0 = std::chrono::steady_clock::now();
+      run_tiles(m, drows, int64_t(rl));
+      finish(m, t0);
+      return;
+    }
     auto t0 = std::chrono::steady_clock::now();
     long st = 0;
     if (tune && !tuned) {
@@ -4961,6 +5083,10 @@ template <class R> struct Batch : BatchBase {
       else
         for (long q = st; q < m; ++q) launch_step(q, bidx, drows + size_t(q) * rl);
     }
+    finish(m, t0);
+  }
+  // the end of a call's m steps: the finiteness probes, the steps' time and the chunks' clocks
+  void finish(long m, std::chrono::steady_clock::time_point t0) {
     for (Fields<R> *f : sims) f->probe_on(stream);
     HIPCHECK(hipStreamSynchronize(stream));
     HIPCHECK(hipGetLastError());

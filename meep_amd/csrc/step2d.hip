@@ -191,7 +191,8 @@ template <class R, bool TM, int NP, int NW, int K> struct Tile2d {
       if (srcs[ph] && threadIdx.x < sizeof(SrcSet) / 8)
         reinterpret_cast<uint64_t *>(set + ph)[threadIdx.x] = ((Glob<const uint64_t>)uni(a.src[ph]))[threadIdx.x];
     }
-    for (int q = int(threadIdx.x); q < l.nsteps * int(l.rl); q += NW * 64) vals[q] = l.vrow[a.vofs + int64_t(q / int(l.rl)) * l.stride + q % int(l.rl)];
+    const int rl = uni(a.rl);
+    for (int q = int(threadIdx.x); q < l.nsteps * rl; q += NW * 64) vals[q] = l.vrow[a.vofs + int64_t(q / rl) * l.stride + q % rl];
     __syncthreads();
 #pragma unroll
     for (int q = 0; q < 3; ++q) {
@@ -221,7 +222,7 @@ template <class R, bool TM, int NP, int NW, int K> struct Tile2d {
     static_assert(SRC_TAB * K <= 64, "a bit per list entry and row");
     const SrcTab &t = L == 2 ? set[1].dip : set[L ? 1 : 0].cur;
     const SrcBoxes &b = L == 2 ? set[1].dipb : set[L ? 1 : 0].curb;
-    const double *val = vals + s * int(l.rl);
+    const double *val = vals + s * a.rl;
     if (tmask[L]) {
       const int vb = t.vbase;
 #pragma unroll
@@ -666,7 +667,10 @@ __global__ __launch_bounds__(NW * 64) void k_step2d(const Step2dLaunch<R> l) {
 }
 
 template <class R, bool TM, int NP> static void launch_s2(const Step2dLaunch<R> &l, int monmask, hipStream_t s) {
-  constexpr int NW = 8, K = S2_ROWS / NW;
+  // two rows a thread: four waves on a SIMD hide each other's waits (against four rows and two
+  // waves: 32 / 19 us for up to 8 steps of a 400 x 300 FP32 cell, and less in FP64, where some
+  // registers then spill)
+  constexpr int NW = 16, K = S2_ROWS / NW;
   const unsigned nb = (l.ntile + 7u) / 8u * 8u;
   const size_t lds = l.hits ? S2_ENTRIES * sizeof(S2Entry) + 4 * S2_MONS * sizeof(int) +
                                   size_t(__builtin_popcount(unsigned(monmask))) * S2_ROWS * S2_COLS * sizeof(R)
