@@ -479,7 +479,8 @@ struct FarArgs {
   int cls_lo[7];
   const double2 *f0;
   int nsrc;
-  const double *px, *py, *pz;
+  const double *px, *py, *pz; // null: the one point `one`
+  double one[3];
   int npts;
   const double *freq;
   int nfreq;
@@ -487,12 +488,17 @@ struct FarArgs {
   int dim, segs;
   int uniform; // freq[i] = freq[0] + i (freq[1] - freq[0]) to rounding
 };
-// frequencies a block of the far-field kernel takes together in 3D: 2 and 3 measured alike
-// (4 runs out of registers and halves the rate); 2 divides the usual even frequency counts
-constexpr int FF_GROUP3 = 2;
-inline int farfield_group(int dim) { return dim == 3 ? FF_GROUP3 : 1; }
-// partial: npts * nfreq * segs * 12 doubles of scratch; out: npts * nfreq * 12 doubles, the
-// (re, im) of Ex Ey Ez Hx Hy Hz per (point, frequency), point-major
-void launch_farfield(const FarArgs &a, double *partial, double *out, hipStream_t s);
+// Frequencies a block takes together in 3D, sharing a current's geometry and its two phase
+// evaluations.  Full groups of 3 and of 5 cost the same per frequency (1218 us for 3, 2033 us for 5
+// on a plane of 1600 points and 41 k currents, against 1080 us for 2 and 866 us for 1; 4 runs out of
+// registers: 1690 us), so it is 3 unless only 5 leaves no remainder.
+inline int farfield_group(int dim, int nfreq) {
+  if (dim != 3 || nfreq < 1) return 1;
+  return nfreq % 5 == 0 && nfreq % 3 ? 5 : nfreq < 3 ? nfreq : 3;
+}
+// partial: npts * nfreq * segs * 12 doubles of scratch; done: a counter per (point, frequency
+// group), zero before and after; out: npts * nfreq * 12 doubles, the (re, im) of Ex Ey Ez Hx Hy Hz
+// per (point, frequency), point-major
+void launch_farfield(const FarArgs &a, double *partial, double *out, unsigned *done, hipStream_t s);
 
 } // namespace mx

@@ -472,6 +472,14 @@ template <class R> struct N2F : Flux<R> {
   unsigned built_version = 0, built_acc = 0;
   int nsrc = 0, cls_lo[7] = {};
   DevBuf sx, sy, sz, f0, d_freq;
+  // scratch of the far-field calls, kept while it is small (three allocations and releases were
+  // half of a call for one point)
+  DevBuf points, partial, out, done;
+  std::mutex in_use; // one call at a time has them
+  void trim() {
+    for (DevBuf *b : {&points, &partial, &out})
+      if (b->bytes > (size_t(16) << 20)) b->alloc(0);
+  }
 };
 
 template <class R> struct Fields : FieldsBase {
@@ -4518,9 +4526,10 @@ template <class R> struct Fields : FieldsBase {
     const long batch = std::max(1L, (1L << 20) / Nf);
     const long nb = std::min(np, batch);
     const long pairs_max = nb * Nf;
-    // blocks per segment: the points times the frequency groups a block takes together
-    const long fb = farfield_group(gv.dim), bps = nb * ((Nf + fb - 1) / fb);
-    const int segs = int(std::max(1L, std::min<long>((n.nsrc + 511) / 512, (4096 + bps - 1) / bps)));
+    // Segments of the current list: enough blocks to fill the chip, down to one current a thread
+    // where a call has few points (a point of 1296 currents: 6 segments)
+    const long fb = farfield_group(gv.dim, Nf), bps = nb * ((Nf + fb - 1) / fb);
+    const int segs = int(std::max(1L, std::min<long>((n.nsrc + 255) / 256, (4096 + bps - 1) / bps)));
     // uniformly spaced frequencies (to a few ulps, as linspace makes them) let the kernel step
     // e^{ikr} from one frequency to the next
     bool uniform = Nf > 1;
@@ -4528,22 +4537,33 @@ template <class R> struct Fields : FieldsBase {
       const double want = n.freq[0] + i * (n.freq[1] - n.freq[0]);
       uniform = std::fabs(n.freq[i] - want) <= 8 * DBL_EPSILON * std::max(std::fabs(n.freq[i]), std::fabs(n.freq[0]));
     }
-    DevBuf dp, partial, dout;
-    dp.alloc(8 * 3 * size_t(nb));
-    partial.alloc(8 * 12 * size_t(pairs_max) * segs);
-    dout.alloc(8 * 12 * size_t(pairs_max));
+    std::lock_guard<std::mutex> hold(n.in_use);
+    auto room = [](DevBuf &b, size_t bytes) {
+      if (b.bytes < bytes) b.alloc(bytes);
+    };
+    if (nb > 1) room(n.points, 8 * 3 * size_t(nb));
+    room(n.partial, 8 * 12 * size_t(pairs_max) * size_t(segs > 1 ? segs : 0));
+    room(n.out, 8 * 12 * size_t(pairs_max));
+    if (n.done.bytes < sizeof(unsigned) * size_t(bps)) {
+      n.done.alloc(sizeof(unsigned) * size_t(bps));
+      HIPCHECK(hipMemsetAsync(n.done.p, 0, n.done.bytes, stream));
+    }
     std::vector<double> soa(3 * size_t(nb));
     for (long b0 = 0; b0 < np; b0 += nb) {
       const long m = std::min(nb, np - b0);
       for (long q = 0; q < m; ++q)
         for (int d = 0; d < 3; ++d) soa[size_t(d) * nb + q] = (gv.dim == 2 && d == 2) ? 0.0 : pts[3 * (b0 + q) + d];
-      HIPCHECK(hipMemcpyAsync(dp.p, soa.data(), 8 * 3 * size_t(nb), hipMemcpyHostToDevice, stream));
       FarArgs a;
+      memset(&a, 0, sizeof a);
+      if (nb > 1)
+        HIPCHECK(hipMemcpyAsync(n.points.p, soa.data(), 8 * 3 * size_t(nb), hipMemcpyHostToDevice, stream));
+      else
+        for (int d = 0; d < 3; ++d) a.one[d] = soa[size_t(d)];
       a.sx = static_cast<const double *>(n.sx.p), a.sy = static_cast<const double *>(n.sy.p), a.sz = static_cast<const double *>(n.sz.p);
       for (int c = 0; c <= 6; ++c) a.cls_lo[c] = n.cls_lo[c];
       a.f0 = static_cast<const double2 *>(n.f0.p);
       a.nsrc = n.nsrc;
-      a.px = static_cast<const double *>(dp.p), a.py = a.px + nb, a.pz = a.px + 2 * nb;
+      if (nb > 1) a.px = static_cast<const double *>(n.points.p), a.py = a.px + nb, a.pz = a.px + 2 * nb;
       a.npts = int(m);
       a.freq = static_cast<const double *>(n.d_freq.p);
       a.nfreq = Nf;
@@ -4552,12 +4572,13 @@ template <class R> struct Fields : FieldsBase {
       a.segs = segs;
       a.uniform = uniform ? 1 : 0;
       kbegin(7);
-      launch_farfield(a, static_cast<double *>(partial.p), static_cast<double *>(dout.p), stream);
+      launch_farfield(a, static_cast<double *>(n.partial.p), static_cast<double *>(n.out.p), static_cast<unsigned *>(n.done.p), stream);
       HIPCHECK(hipGetLastError());
       kend();
-      HIPCHECK(hipMemcpyAsync(out + size_t(b0) * Nf * 12, dout.p, 8 * 12 * size_t(m) * Nf, hipMemcpyDeviceToHost, stream));
+      HIPCHECK(hipMemcpyAsync(out + size_t(b0) * Nf * 12, n.out.p, 8 * 12 * size_t(m) * Nf, hipMemcpyDeviceToHost, stream));
       HIPCHECK(hipStreamSynchronize(stream));
     }
+    n.trim();
   }
   void flux_delete(void *flp) override {
     for (size_t q = 0; q < fluxes.size(); ++q)
@@ -5922,7 +5943,7 @@ int mp_near2far_green(int dim, const double *x, double freq, double eps, double 
     const int cls = c0 < 5 ? (c0 == 4 ? 2 : c0) : (c0 == 9 ? 5 : c0 - 2);
     for (int c = 0; c <= 6; ++c) a.cls_lo[c] = c > cls ? 1 : 0;
     a.nsrc = 1, a.npts = 1, a.nfreq = 1, a.eps = eps, a.mu = mu, a.dim = dim, a.segs = 1, a.uniform = 0;
-    launch_farfield(a, static_cast<double *>(part.p), static_cast<double *>(outb.p), nullptr);
+    launch_farfield(a, static_cast<double *>(part.p), static_cast<double *>(outb.p), nullptr, nullptr); // one segment: no counter
     HIPCHECK(hipGetLastError());
     HIPCHECK(hipMemcpy(EH, outb.p, 12 * 8, hipMemcpyDeviceToHost));
   });

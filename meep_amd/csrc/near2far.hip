@@ -70,12 +70,51 @@ __device__ __forceinline__ void green3d_term(Cx acc[6], const double rh[3], doub
   }
 }
 
+// H0 and H1 of the first kind at x >= HANKEL_X by Hankel's asymptotic expansion (DLMF 10.17.5):
+// H_n(x) = sqrt(2 / (pi x)) e^{i (x - n pi/2 - pi/4)} sum_k i^k a_k(n) / x^k with
+// a_k = a_{k-1} (4 n^2 - (2k - 1)^2) / (8 k).  At x = 30 the terms fall below 1e-17 by k = 14; one
+// sine and cosine serve both orders, where j0, y0, j1 and y1 take one each beside their rational
+// approximations (60 one-point calls at 8 frequencies, most of their time the host's: 2.45 ms, now
+// 2.15 ms).
+constexpr double HANKEL_X = 30.0;
+constexpr int HANKEL_K = 14;
+template <int N> __device__ __forceinline__ Cx hankel_sum(double ix) {
+  // even terms (real part) and odd terms (imaginary part), by Horner's rule in i / x
+  double a[HANKEL_K + 1];
+  a[0] = 1.0;
+#pragma unroll
+  for (int k = 1; k <= HANKEL_K; ++k) a[k] = a[k - 1] * (4.0 * N * N - (2.0 * k - 1.0) * (2.0 * k - 1.0)) / (8.0 * k); // constants
+  const double z = -ix * ix;
+  double re = a[HANKEL_K], im = a[HANKEL_K - 1];
+#pragma unroll
+  for (int k = HANKEL_K - 2; k >= 0; k -= 2) re = re * z + a[k];
+#pragma unroll
+  for (int k = HANKEL_K - 3; k >= 1; k -= 2) im = im * z + a[k];
+  return {re, im * ix};
+}
+__device__ __forceinline__ void hankel01(double x, Cx &h0, Cx &h1) {
+  if (x >= HANKEL_X) {
+    double sn, cs;
+    sincos(x, &sn, &cs);
+    const double ix = 1.0 / x, am = sqrt(ix * (1.0 / FF_PI)); // sqrt(2 / (pi x)) / sqrt 2
+    const Cx e = {(cs + sn) * am, (sn - cs) * am};             // e^{i (x - pi/4)}, the 1 / sqrt 2 above
+    const Cx p0 = hankel_sum<0>(ix), p1 = hankel_sum<1>(ix);
+    h0 = cmul(e, p0);
+    const Cx t = cmul(e, p1);
+    h1 = {t.im, -t.re}; // a quarter turn back
+    return;
+  }
+  h0 = {j0(x), y0(x)};
+  h1 = {j1(x), y1(x)};
+}
+
 // green2d (src/near2far.cpp:207-267) for one current, with H_n = J_n + i Y_n of k r; H2 from
 // the recurrence H2 = (2 / x) H1 - H0 (exact for the Hankel functions)
 __device__ __forceinline__ void green2d_acc(Cx acc[6], double dx, double dy, double k, double omega, double eps, double mu,
                                             double imp, int c0, Cx f0) {
   const double r = sqrt(dx * dx + dy * dy), rx = dx / r, ry = dy / r, kr = k * r;
-  const Cx h0 = {j0(kr), y0(kr)}, h1 = {j1(kr), y1(kr)};
+  Cx h0, h1;
+  hankel01(kr, h0, h1);
   const Cx H0 = cmul(h0, f0), H1 = cmul(h1, f0);
   const Cx ikH1 = {-0.25 * k * H1.im, 0.25 * k * H1.re};
   const bool electric = c0 < 5;
@@ -124,8 +163,9 @@ template <int FB> struct FarGroup {
 __device__ __forceinline__ void phase(double t, double &sn, double &cs) { sincospi(2.0 * (t - rint(t)), &sn, &cs); }
 
 // The currents [jlo, jhi) of one class (direction PD, electric or magnetic): the thread's
-// share, strided over the block, added to acc for each frequency of the group.
-template <int DIM, int FB, int PD, bool ELECTRIC>
+// share, strided over the block, added to acc for each frequency of the group.  FULL: the group
+// has FB frequencies, uniformly spaced (the loop over them has no exits to test).
+template <int DIM, int FB, int PD, bool ELECTRIC, bool FULL>
 __device__ __forceinline__ void far_class(Cx (&acc)[FB][6], const FarArgs &a, const FarGroup<FB> &g, int jlo, int jhi,
                                           int f_first, double X, double Y, double Zc) {
   constexpr int c0 = (ELECTRIC ? 0 : 5) + (PD == 2 ? 4 : PD);
@@ -134,35 +174,51 @@ __device__ __forceinline__ void far_class(Cx (&acc)[FB][6], const FarArgs &a, co
     Cx f0[FB];
 #pragma unroll
     for (int q = 0; q < FB; ++q) {
-      const double2 v = q < g.nq ? a.f0[size_t(f_first + q) * a.nsrc + j] : make_double2(0.0, 0.0);
+      const double2 v = FULL || q < g.nq ? a.f0[size_t(f_first + q) * a.nsrc + j] : make_double2(0.0, 0.0);
       f0[q] = {v.x, v.y};
     }
     if (DIM == 3) {
       const double dx = X - a.sx[j], dy = Y - a.sy[j], dz = Zc - a.sz[j];
       const double r2 = dx * dx + dy * dy + dz * dz, ir = rsqrt(r2), r = r2 * ir;
-      const double rh[3] = {dx * ir, dy * ir, dz * ir};
+      const double rh[3] = {dx * ir, dy * ir, dz * ir}, amp = ir * inv_em;
       double cs = 0, sn = 0, dcs = 1, dsn = 0;
-      if (g.recur) {
+      if (FULL || g.recur) {
         phase(g.cyc[0] * r, sn, cs);
-        phase(g.dcyc * r, dsn, dcs);
+        if (FB > 1) phase(g.dcyc * r, dsn, dcs);
       }
 #pragma unroll
       for (int q = 0; q < FB; ++q) {
-        if (q >= g.nq) break;
-        if (!g.recur)
+        if (!FULL && q >= g.nq) break;
+        if (!FULL && !g.recur)
           phase(g.cyc[q] * r, sn, cs);
         else if (q > 0) {
           const double c2 = cs * dcs - sn * dsn;
           sn = sn * dcs + cs * dsn;
           cs = c2;
         }
-        green3d_term<PD, ELECTRIC>(acc[q], rh, ir * g.inv_k[q], cs, sn, g.kn4[q] * ir * inv_em, zf, f0[q]);
+        green3d_term<PD, ELECTRIC>(acc[q], rh, ir * g.inv_k[q], cs, sn, g.kn4[q] * amp, zf, f0[q]);
       }
     }
     else {
 #pragma unroll
       for (int q = 0; q < FB; ++q)
         if (q < g.nq) green2d_acc(acc[q], X - a.sx[j], Y - a.sy[j], g.k[q], g.omega[q], g.eps, g.mu, g.imp, c0, f0[q]);
+    }
+  }
+}
+template <int DIM, int FB, bool FULL>
+__device__ __forceinline__ void far_classes(Cx (&acc)[FB][6], const FarArgs &a, const FarGroup<FB> &g, int lo, int hi, int f_first,
+                                            double X, double Y, double Zc) {
+  for (int cls = 0; cls < 6; ++cls) {
+    const int jlo = max(lo, a.cls_lo[cls]), jhi = min(hi, a.cls_lo[cls + 1]);
+    if (jlo >= jhi) continue;
+    switch (cls) {
+      case 0: far_class<DIM, FB, 0, true, FULL>(acc, a, g, jlo, jhi, f_first, X, Y, Zc); break;
+      case 1: far_class<DIM, FB, 1, true, FULL>(acc, a, g, jlo, jhi, f_first, X, Y, Zc); break;
+      case 2: far_class<DIM, FB, 2, true, FULL>(acc, a, g, jlo, jhi, f_first, X, Y, Zc); break;
+      case 3: far_class<DIM, FB, 0, false, FULL>(acc, a, g, jlo, jhi, f_first, X, Y, Zc); break;
+      case 4: far_class<DIM, FB, 1, false, FULL>(acc, a, g, jlo, jhi, f_first, X, Y, Zc); break;
+      default: far_class<DIM, FB, 2, false, FULL>(acc, a, g, jlo, jhi, f_first, X, Y, Zc); break;
     }
   }
 }
@@ -175,14 +231,14 @@ __device__ __forceinline__ void far_class(Cx (&acc)[FB][6], const FarArgs &a, co
 // group.  The
 // currents come sorted by class (Ex Ey Ez Hx Hy Hz, a.cls_lo), so each class runs a loop of
 // its own with its direction and kind known at compile time.
-template <int DIM, int FB> __global__ __launch_bounds__(FF_BLOCK) void k_farfield(FarArgs a, double *partial) {
+template <int DIM, int FB> __global__ __launch_bounds__(FF_BLOCK) void k_farfield(FarArgs a, double *partial, double *out, unsigned *done) {
   const int b = blockIdx.x;
   const int ngroup = (a.nfreq + FB - 1) / FB;
   const int pair = b / a.segs, seg = b - pair * a.segs;
   const int p = pair / ngroup, f_first = (pair - p * ngroup) * FB;
   const int per = (a.nsrc + a.segs - 1) / a.segs;
   const int lo = seg * per, hi = min(a.nsrc, lo + per);
-  const double X = a.px[p], Y = a.py[p], Zc = a.pz[p];
+  const double X = a.px ? a.px[p] : a.one[0], Y = a.px ? a.py[p] : a.one[1], Zc = a.px ? a.pz[p] : a.one[2];
   FarGroup<FB> g;
   g.nq = min(FB, a.nfreq - f_first);
   const double n = sqrt(a.eps * a.mu);
@@ -203,21 +259,14 @@ template <int DIM, int FB> __global__ __launch_bounds__(FF_BLOCK) void k_farfiel
   for (int q = 0; q < FB; ++q)
 #pragma unroll
     for (int c = 0; c < 6; ++c) acc[q][c] = {0.0, 0.0};
-  for (int cls = 0; cls < 6; ++cls) {
-    const int jlo = max(lo, a.cls_lo[cls]), jhi = min(hi, a.cls_lo[cls + 1]);
-    if (jlo >= jhi) continue;
-    switch (cls) {
-      case 0: far_class<DIM, FB, 0, true>(acc, a, g, jlo, jhi, f_first, X, Y, Zc); break;
-      case 1: far_class<DIM, FB, 1, true>(acc, a, g, jlo, jhi, f_first, X, Y, Zc); break;
-      case 2: far_class<DIM, FB, 2, true>(acc, a, g, jlo, jhi, f_first, X, Y, Zc); break;
-      case 3: far_class<DIM, FB, 0, false>(acc, a, g, jlo, jhi, f_first, X, Y, Zc); break;
-      case 4: far_class<DIM, FB, 1, false>(acc, a, g, jlo, jhi, f_first, X, Y, Zc); break;
-      default: far_class<DIM, FB, 2, false>(acc, a, g, jlo, jhi, f_first, X, Y, Zc); break;
-    }
-  }
+  if (DIM == 3 && g.nq == FB && (FB == 1 || g.recur))
+    far_classes<DIM, FB, true>(acc, a, g, lo, hi, f_first, X, Y, Zc);
+  else
+    far_classes<DIM, FB, false>(acc, a, g, lo, hi, f_first, X, Y, Zc);
   const int nq = g.nq;
   // wave reduction, then across the block's waves through LDS; one partial per frequency
   __shared__ double red[FF_BLOCK / 64][12];
+  __shared__ bool last;
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
 #pragma unroll
   for (int q = 0; q < FB; ++q) {
@@ -236,32 +285,49 @@ template <int DIM, int FB> __global__ __launch_bounds__(FF_BLOCK) void k_farfiel
       double sum = 0;
 #pragma unroll
       for (int w = 0; w < FF_BLOCK / 64; ++w) sum += red[w][threadIdx.x];
-      // partial layout: [point][frequency][segment][12]
-      partial[((size_t(p) * a.nfreq + f_first + q) * a.segs + seg) * 12 + threadIdx.x] = sum;
+      if (a.segs == 1)
+        out[(size_t(p) * a.nfreq + f_first + q) * 12 + threadIdx.x] = sum;
+      else // partial layout: [point][frequency][segment][12]
+        partial[((size_t(p) * a.nfreq + f_first + q) * a.segs + seg) * 12 + threadIdx.x] = sum;
     }
     __syncthreads();
   }
+  if (a.segs == 1) return;
+  // The pair's last block to finish adds the segments' partials, in segment order whichever block
+  // it is (a second launch took 3.2 us of a 40 us call).  Each block publishes its partials
+  // before it counts itself, and the count is left at zero for the next launch.
+  __threadfence();
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    last = __hip_atomic_fetch_add(done + pair, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == unsigned(a.segs) - 1;
+    if (last) __hip_atomic_store(done + pair, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __syncthreads();
+  if (!last) return;
+  __threadfence();
+  for (int t = int(threadIdx.x); t < nq * 12; t += FF_BLOCK) {
+    const int q = t / 12, c = t - q * 12;
+    double sum = 0;
+    for (int z = 0; z < a.segs; ++z)
+      sum += __hip_atomic_load(partial + ((size_t(p) * a.nfreq + f_first + q) * a.segs + z) * 12 + c, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+    out[(size_t(p) * a.nfreq + f_first + q) * 12 + c] = sum;
+  }
 }
 
-// out[pair * 12 + q] = the sum over the pair's segments, in segment order
-__global__ void k_farfield_sum(const double *partial, int npair, int segs, double *out) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= npair * 12) return;
-  const int pair = t / 12, q = t - pair * 12;
-  double s = 0;
-  for (int g = 0; g < segs; ++g) s += partial[(size_t(pair) * segs + g) * 12 + q];
-  out[t] = s;
-}
-
-void launch_farfield(const FarArgs &a, double *partial, double *out, hipStream_t s) {
-  const int fb = farfield_group(a.dim);
+void launch_farfield(const FarArgs &a, double *partial, double *out, unsigned *done, hipStream_t s) {
+  const int fb = farfield_group(a.dim, a.nfreq);
   const size_t nblk = size_t(a.npts) * ((a.nfreq + fb - 1) / fb) * a.segs;
-  if (a.dim == 3)
-    hipLaunchKernelGGL((k_farfield<3, FF_GROUP3>), dim3(unsigned(nblk)), dim3(FF_BLOCK), 0, s, a, partial);
+  const dim3 grid{unsigned(nblk)}, block(FF_BLOCK);
+  if (a.dim != 3)
+    hipLaunchKernelGGL((k_farfield<2, 1>), grid, block, 0, s, a, partial, out, done);
   else
-    hipLaunchKernelGGL((k_farfield<2, 1>), dim3(unsigned(nblk)), dim3(FF_BLOCK), 0, s, a, partial);
-  const int npair = a.npts * a.nfreq;
-  hipLaunchKernelGGL(k_farfield_sum, dim3((npair * 12 + 255) / 256), dim3(256), 0, s, partial, npair, a.segs, out);
+    switch (fb) {
+      case 1: hipLaunchKernelGGL((k_farfield<3, 1>), grid, block, 0, s, a, partial, out, done); break;
+      case 2: hipLaunchKernelGGL((k_farfield<3, 2>), grid, block, 0, s, a, partial, out, done); break;
+      case 3: hipLaunchKernelGGL((k_farfield<3, 3>), grid, block, 0, s, a, partial, out, done); break;
+      default: hipLaunchKernelGGL((k_farfield<3, 5>), grid, block, 0, s, a, partial, out, done); break;
+    }
 }
 
 } // namespace mx
