@@ -74,17 +74,6 @@ __device__ __forceinline__ void adj_upd_slot(const StepArgs<R> &a, const AdjSlot
   }
 }
 
-template <class R>
-__global__ __launch_bounds__(BLOCK) void k_adj_upd(const StepArgs<R> a, const AdjSlots<R> b, const AdjDesign<R> dz, uint32_t count) {
-  const uint32_t t = blockIdx.x * BLOCK + threadIdx.x;
-  if (t >= count) return;
-  Pt p;
-  grid_point(a.g, t, p);
-  adj_upd_slot<R, 0>(a, b, dz, p);
-  adj_upd_slot<R, 1>(a, b, dz, p);
-  adj_upd_slot<R, 2>(a, b, dz, p);
-}
-
 // ---- curl transpose (local part) ------------------------------------------------------------
 template <class R, int C> __device__ __forceinline__ void adj_curl_slot(const StepArgs<R> &a, const AdjSlots<R> &b, const Pt &p) {
   if (C >= a.nc || !a.cc[C].f) return;
@@ -124,14 +113,24 @@ template <class R, int C> __device__ __forceinline__ void adj_curl_slot(const St
   b.cbar[C][i] = cb;
 }
 
-template <class R> __global__ __launch_bounds__(BLOCK) void k_adj_curl(const StepArgs<R> a, const AdjSlots<R> b, uint32_t count) {
+// Both transposes of a half-step in one launch: each touches a thread's own point only, so the
+// curl follows the update in the same thread.  A reverse step of a 2D cell is bound by the
+// latency of its launches, 12 of them where the objective's monitor averages four points; with
+// the partners' gathers in one launch too, and the monitor's points in one, it takes 5 (a gradient
+// over 1200 steps of a 400 x 300 FP32 cell: 64.6 -> 47.0 ms).
+template <class R>
+__global__ __launch_bounds__(BLOCK) void k_adj_phase(const StepArgs<R> a, const AdjSlots<R> u, const AdjDesign<R> dz, const AdjSlots<R> c,
+                                                    uint32_t count) {
   const uint32_t t = blockIdx.x * BLOCK + threadIdx.x;
   if (t >= count) return;
   Pt p;
   grid_point(a.g, t, p);
-  adj_curl_slot<R, 0>(a, b, p);
-  adj_curl_slot<R, 1>(a, b, p);
-  adj_curl_slot<R, 2>(a, b, p);
+  adj_upd_slot<R, 0>(a, u, dz, p);
+  adj_upd_slot<R, 1>(a, u, dz, p);
+  adj_upd_slot<R, 2>(a, u, dz, p);
+  adj_curl_slot<R, 0>(a, c, p);
+  adj_curl_slot<R, 1>(a, c, p);
+  adj_curl_slot<R, 2>(a, c, p);
 }
 
 // ---- curl transpose (gather into a partner) -------------------------------------------------
@@ -144,17 +143,23 @@ template <class R, int E> __device__ __forceinline__ R gather_entry(const Grid &
   const R here = ga.cbar[E][i];
   return ga.plus[E] ? behind - here : here - behind;
 }
-template <class R> __global__ __launch_bounds__(BLOCK) void k_adj_gather(const Grid g, const AdjGather<R> ga, uint32_t count) {
-  const uint32_t t = blockIdx.x * BLOCK + threadIdx.x;
-  if (t >= count) return;
-  Pt p;
-  grid_point(g, t, p);
+template <class R> __device__ __forceinline__ void gather_partner(const Grid &g, const AdjGather<R> &ga, const Pt &p) {
   const int64_t i = p.i;
   R v = gather_entry<R, 0>(g, ga, p, i);
   v += gather_entry<R, 1>(g, ga, p, i);
   v += gather_entry<R, 2>(g, ga, p, i);
   v += gather_entry<R, 3>(g, ga, p, i);
   ga.gb[i] += v;
+}
+// every partner of a half-step (each an array of its own, none of them a cbar)
+template <class R> __global__ __launch_bounds__(BLOCK) void k_adj_gather(const Grid g, const AdjGathers<R> gs, uint32_t count) {
+  const uint32_t t = blockIdx.x * BLOCK + threadIdx.x;
+  if (t >= count) return;
+  Pt p;
+  grid_point(g, t, p);
+  if (gs.n > 0) gather_partner(g, gs.ga[0], p);
+  if (gs.n > 1) gather_partner(g, gs.ga[1], p);
+  if (gs.n > 2) gather_partner(g, gs.ga[2], p);
 }
 
 // ---- halo transpose ------------------------------------------------------------------------
@@ -172,11 +177,9 @@ __global__ __launch_bounds__(BLOCK) void k_adj_halo(const int *first, const uint
 }
 
 // ---- DFT objective cotangent -----------------------------------------------------------------
-template <class R>
-__global__ __launch_bounds__(BLOCK) void k_adj_dft(const double *w, const double2 *acc, const double *omega, int npts, int nfreq,
-                                                  double time, double scale_re, double scale_im, double *G) {
-  const int k = blockIdx.x * BLOCK + threadIdx.x;
-  if (k >= npts) return;
+// w_k times the sum over frequencies, for point k
+__device__ __forceinline__ double adj_dft_point(const double *w, const double2 *acc, const double *omega, int k, int nfreq, double time,
+                                               double scale_re, double scale_im) {
   double sum = 0;
   for (int f = 0; f < nfreq; ++f) {
     double sn, cs;
@@ -185,7 +188,28 @@ __global__ __launch_bounds__(BLOCK) void k_adj_dft(const double *w, const double
     const double2 a = acc[size_t(k) * nfreq + f];
     sum += 2.0 * (a.x * pr + a.y * pim); // 2 Re(conj(a) ph)
   }
-  G[k] = w[k] * sum;
+  return w[k] * sum;
+}
+static __global__ __launch_bounds__(BLOCK) void k_adj_dft(const double *w, const double2 *acc, const double *omega, int npts, int nfreq,
+                                                  double time, double scale_re, double scale_im, double *G) {
+  const int k = blockIdx.x * BLOCK + threadIdx.x;
+  if (k < npts) G[k] = adj_dft_point(w, acc, omega, k, nfreq, time, scale_re, scale_im);
+}
+// At most ADJ_DFT_ONE points: one block, which adds offset after offset (two offsets of different
+// points may meet in one element; the barrier orders them as the launches of the form above are).
+constexpr int ADJ_DFT_ONE = 1024;
+template <class R>
+__global__ __launch_bounds__(ADJ_DFT_ONE) void k_adj_dft_one(R *bar, const int64_t *idx, const double *w, const double2 *acc,
+                                                            const double *omega, int npts, int nfreq, double time, double scale_re,
+                                                            double scale_im, AdjOffsets o) {
+  const int k = threadIdx.x;
+  const bool live = k < npts;
+  const double G = live ? adj_dft_point(w, acc, omega, k, nfreq, time, scale_re, scale_im) : 0;
+  R *p = bar + (live ? idx[k] : 0);
+  for (int q = 0; q < o.n; ++q) {
+    if (q) __syncthreads();
+    if (live) p[o.off[q]] = R(double(p[o.off[q]]) + o.coef * G);
+  }
 }
 template <class R>
 __global__ __launch_bounds__(BLOCK) void k_adj_dft_scatter(R *bar, const int64_t *idx, const double *G, int npts, int64_t off, double coef) {
@@ -211,17 +235,14 @@ __global__ __launch_bounds__(BLOCK) void k_record(R *hist, const R *D, const Gri
 // ---- launchers ---------------------------------------------------------------------------------
 static inline uint32_t grid_count(const Grid &g) { return uint32_t(g.an[0]) * uint32_t(g.an[1]) * uint32_t(g.an[2]); }
 
-template <class R> void launch_adj_upd(const StepArgs<R> &a, const AdjSlots<R> &b, const AdjDesign<R> &dz, hipStream_t s) {
+template <class R>
+void launch_adj_phase(const StepArgs<R> &a, const AdjSlots<R> &u, const AdjDesign<R> &dz, const AdjSlots<R> &c, hipStream_t s) {
   const uint32_t n = grid_count(a.g);
-  hipLaunchKernelGGL(k_adj_upd<R>, dim3(nblocks(n)), dim3(BLOCK), 0, s, a, b, dz, n);
+  hipLaunchKernelGGL(k_adj_phase<R>, dim3(nblocks(n)), dim3(BLOCK), 0, s, a, u, dz, c, n);
 }
-template <class R> void launch_adj_curl(const StepArgs<R> &a, const AdjSlots<R> &b, hipStream_t s) {
-  const uint32_t n = grid_count(a.g);
-  hipLaunchKernelGGL(k_adj_curl<R>, dim3(nblocks(n)), dim3(BLOCK), 0, s, a, b, n);
-}
-template <class R> void launch_adj_gather(const Grid &g, const AdjGather<R> &ga, hipStream_t s) {
+template <class R> void launch_adj_gather(const Grid &g, const AdjGathers<R> &gs, hipStream_t s) {
   const uint32_t n = grid_count(g);
-  if (ga.n > 0) hipLaunchKernelGGL(k_adj_gather<R>, dim3(nblocks(n)), dim3(BLOCK), 0, s, g, ga, n);
+  if (gs.n > 0) hipLaunchKernelGGL(k_adj_gather<R>, dim3(nblocks(n)), dim3(BLOCK), 0, s, g, gs, n);
 }
 template <class R>
 void launch_adj_halo(const int *first, const uint32_t *src, const uint32_t *dst, const int8_t *sgn, const uint16_t *slot, int nsrc,
@@ -229,13 +250,17 @@ void launch_adj_halo(const int *first, const uint32_t *src, const uint32_t *dst,
   if (nsrc > 0) hipLaunchKernelGGL(k_adj_halo<R>, dim3(nblocks(nsrc)), dim3(BLOCK), 0, s, first, src, dst, sgn, slot, nsrc, bars);
 }
 template <class R>
-void launch_adj_dft(const int64_t *, const double *w, const double2 *acc, const double *omega, int npts, int nfreq, double time,
-                    double scale_re, double scale_im, double *G, hipStream_t s) {
-  if (npts > 0)
-    hipLaunchKernelGGL(k_adj_dft<R>, dim3(nblocks(npts)), dim3(BLOCK), 0, s, w, acc, omega, npts, nfreq, time, scale_re, scale_im, G);
-}
-template <class R> void launch_adj_dft_scatter(R *bar, const int64_t *idx, const double *G, int npts, int64_t off, double coef, hipStream_t s) {
-  if (npts > 0) hipLaunchKernelGGL(k_adj_dft_scatter<R>, dim3(nblocks(npts)), dim3(BLOCK), 0, s, bar, idx, G, npts, off, coef);
+void launch_adj_dft(R *bar, const int64_t *idx, const double *w, const double2 *acc, const double *omega, int npts, int nfreq, double time,
+                    double scale_re, double scale_im, const AdjOffsets &o, double *G, hipStream_t s) {
+  if (npts <= 0) return;
+  if (npts <= ADJ_DFT_ONE) {
+    hipLaunchKernelGGL(k_adj_dft_one<R>, dim3(1), dim3((npts + 63) / 64 * 64), 0, s, bar, idx, w, acc, omega, npts, nfreq, time, scale_re,
+                       scale_im, o);
+    return;
+  }
+  hipLaunchKernelGGL(k_adj_dft, dim3(nblocks(npts)), dim3(BLOCK), 0, s, w, acc, omega, npts, nfreq, time, scale_re, scale_im, G);
+  for (int q = 0; q < o.n; ++q)
+    hipLaunchKernelGGL(k_adj_dft_scatter<R>, dim3(nblocks(npts)), dim3(BLOCK), 0, s, bar, idx, G, npts, o.off[q], o.coef);
 }
 template <class R> void launch_record(R *hist, const R *D, const Grid &g, const int *lo, const int *hi, hipStream_t s) {
   const int n0 = hi[0] - lo[0] + 1, n1 = hi[1] - lo[1] + 1, n2 = hi[2] - lo[2] + 1;
@@ -244,14 +269,13 @@ template <class R> void launch_record(R *hist, const R *D, const Grid &g, const 
 }
 
 #define INSTANTIATE_ADJ(R)                                                                                                 \
-  template void launch_adj_upd<R>(const StepArgs<R> &, const AdjSlots<R> &, const AdjDesign<R> &, hipStream_t);           \
-  template void launch_adj_curl<R>(const StepArgs<R> &, const AdjSlots<R> &, hipStream_t);                                \
-  template void launch_adj_gather<R>(const Grid &, const AdjGather<R> &, hipStream_t);                                    \
+  template void launch_adj_phase<R>(const StepArgs<R> &, const AdjSlots<R> &, const AdjDesign<R> &, const AdjSlots<R> &,    \
+                                    hipStream_t);                                                                          \
+  template void launch_adj_gather<R>(const Grid &, const AdjGathers<R> &, hipStream_t);                                    \
   template void launch_adj_halo<R>(const int *, const uint32_t *, const uint32_t *, const int8_t *, const uint16_t *, int, \
                                    R *const *, hipStream_t);                                                               \
-  template void launch_adj_dft<R>(const int64_t *, const double *, const double2 *, const double *, int, int, double, double, \
-                                  double, double *, hipStream_t);                                                          \
-  template void launch_adj_dft_scatter<R>(R *, const int64_t *, const double *, int, int64_t, double, hipStream_t);       \
+  template void launch_adj_dft<R>(R *, const int64_t *, const double *, const double2 *, const double *, int, int, double,  \
+                                  double, double, const AdjOffsets &, double *, hipStream_t);                              \
   template void launch_record<R>(R *, const R *, const Grid &, const int *, const int *, hipStream_t);
 // The build compiles this file once per field precision (MX_REAL), in parallel.
 #ifdef MX_REAL

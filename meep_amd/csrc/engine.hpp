@@ -413,22 +413,31 @@ template <class R> struct AdjGather {
   int step[4]; // +1 or -1: coordinate step of s along ax
   int plus[4]; // 1: g1 (the i + s1 partner), 0: g2
 };
+template <class R> struct AdjGathers {
+  int n; // partners of a half-step
+  AdjGather<R> ga[3];
+};
+struct AdjOffsets { // the points a DFT value averages, relative to its index, and their weight
+  int n;
+  int64_t off[4];
+  double coef;
+};
 
 // launchers (adjoint.hip)
-template <class R> void launch_adj_upd(const StepArgs<R> &a, const AdjSlots<R> &b, const AdjDesign<R> &dz, hipStream_t s);
-template <class R> void launch_adj_curl(const StepArgs<R> &a, const AdjSlots<R> &b, hipStream_t s);
-template <class R> void launch_adj_gather(const Grid &g, const AdjGather<R> &ga, hipStream_t s);
+// update transpose (slots u, design dz), then curl transpose (slots c), of a half-step
+template <class R>
+void launch_adj_phase(const StepArgs<R> &a, const AdjSlots<R> &u, const AdjDesign<R> &dz, const AdjSlots<R> &c, hipStream_t s);
+template <class R> void launch_adj_gather(const Grid &g, const AdjGathers<R> &gs, hipStream_t s);
 // halo transpose: for each owned source point src[q], its halo images dst[first[q] .. first[q+1])
 // with signs sgn: bar[src] += sgn * bar[dst]; bar[dst] = 0 (slot pointers in bars)
 template <class R>
 void launch_adj_halo(const int *first, const uint32_t *src, const uint32_t *dst, const int8_t *sgn, const uint16_t *slot, int nsrc,
                      R *const *bars, hipStream_t s);
 // DFT objective J = sum |a|^2: G[k] = w_k * sum_f 2 Re(conj(a_f(k)) ph_f) with ph_f =
-// exp(i omega_f t) * scale, then bar[idx_k + off] += coef * G[k]
+// exp(i omega_f t) * scale, then bar[idx_k + off] += coef * G[k] for each offset in turn (G: scratch)
 template <class R>
-void launch_adj_dft(const int64_t *idx, const double *w, const double2 *acc, const double *omega, int npts, int nfreq, double time,
-                    double scale_re, double scale_im, double *G, hipStream_t s);
-template <class R> void launch_adj_dft_scatter(R *bar, const int64_t *idx, const double *G, int npts, int64_t off, double coef, hipStream_t s);
+void launch_adj_dft(R *bar, const int64_t *idx, const double *w, const double2 *acc, const double *omega, int npts, int nfreq, double time,
+                    double scale_re, double scale_im, const AdjOffsets &o, double *G, hipStream_t s);
 // copy D at the design box points (loop-axis box, device layout) into hist (box-local)
 template <class R> void launch_record(R *hist, const R *D, const Grid &g, const int *lo, const int *hi, hipStream_t s);
 

@@ -3110,7 +3110,17 @@ template <class R> struct Fields : FieldsBase {
       }
       return out;
     };
-    const std::vector<AdjGather<R>> gD = gathers(AD), gB = gathers(AB);
+    auto together = [](const std::vector<AdjGather<R>> &v) {
+      AdjGathers<R> gs;
+      memset(&gs, 0, sizeof gs);
+      if (v.size() > 3) fail("internal: too many gather partners");
+      for (const AdjGather<R> &ga : v) gs.ga[gs.n++] = ga;
+      return gs;
+    };
+    const AdjGathers<R> gD = together(gathers(AD)), gB = together(gathers(AB));
+    AdjDesign<R> none;
+    memset(&none, 0, sizeof none);
+    none.slot = -1;
     // halo transposes (every halo point, folded planes included), by field-type group
     AdjHalo hal[2];
     build_adj_halo(hal, bar);
@@ -3146,16 +3156,13 @@ template <class R> struct Fields : FieldsBase {
         DftChunk<R> &ch = *o->ch;
         if (tafter % ch.decimation) continue;
         const double time = (is_magnetic(ch.c) || is_B(ch.c)) ? tafter * dt - 0.5 * dt : tafter * dt;
-        launch_adj_dft<R>(static_cast<const int64_t *>(ch.idx.p), static_cast<const double *>(ch.w.p),
+        AdjOffsets of;
+        of.n = ch.avg2 ? 4 : ch.avg1 ? 2 : 1;
+        of.coef = of.n == 4 ? 0.25 : of.n == 2 ? 0.5 : 1.0;
+        of.off[0] = 0, of.off[1] = ch.avg1, of.off[2] = ch.avg2, of.off[3] = ch.avg1 + ch.avg2;
+        launch_adj_dft<R>(B(f[ch.c][0]), static_cast<const int64_t *>(ch.idx.p), static_cast<const double *>(ch.w.p),
                           static_cast<const double2 *>(o->acc.p), static_cast<const double *>(ch.omega.p), ch.npts, ch.nfreq, time,
-                          ch.scale.real(), ch.scale.imag(), static_cast<double *>(o->G.p), stream);
-        R *eb = B(f[ch.c][0]);
-        const int64_t offs[4] = {0, ch.avg1, ch.avg2, ch.avg1 + ch.avg2};
-        const int nof = ch.avg2 ? 4 : ch.avg1 ? 2 : 1;
-        const double coef = nof == 4 ? 0.25 : nof == 2 ? 0.5 : 1.0;
-        for (int q = 0; q < nof; ++q)
-          launch_adj_dft_scatter<R>(eb, static_cast<const int64_t *>(ch.idx.p), static_cast<const double *>(o->G.p), ch.npts, offs[q],
-                                    coef, stream);
+                          ch.scale.real(), ch.scale.imag(), of, static_cast<double *>(o->G.p), stream);
       }
       run_adj_halo(hal[1]);
       AdjDesign<R> dz;
@@ -3164,20 +3171,11 @@ template <class R> struct Fields : FieldsBase {
       for (int k = 0; k < 3; ++k) dz.lo[k] = A.lo[k], dz.hi[k] = A.hi[k];
       dz.hist = hist;
       dz.grad = static_cast<double *>(grad.p);
-      launch_adj_upd<R>(AD, uE, dz, stream);
-      launch_adj_curl<R>(AD, cD, stream);
-      for (const AdjGather<R> &ga : gD) launch_adj_gather<R>(gfull, ga, stream);
+      launch_adj_phase<R>(AD, uE, dz, cD, stream);
+      launch_adj_gather<R>(gfull, gD, stream);
       run_adj_halo(hal[0]);
-      bool any_h = false;
-      for (int q = 0; q < 3; ++q) any_h = any_h || AB.uc[q].f;
-      if (any_h) {
-        AdjDesign<R> none;
-        memset(&none, 0, sizeof none);
-        none.slot = -1;
-        launch_adj_upd<R>(AB, uH, none, stream);
-      }
-      launch_adj_curl<R>(AB, cB, stream);
-      for (const AdjGather<R> &ga : gB) launch_adj_gather<R>(gfull, ga, stream);
+      launch_adj_phase<R>(AB, uH, none, cB, stream);
+      launch_adj_gather<R>(gfull, gB, stream);
     };
     if (A.interval <= 0) {
       for (long n = N - 1; n >= 0; --n)
