@@ -1278,15 +1278,17 @@ static bool r3_launch(const StepArgs<R> &a, bool curl, bool upd, hipStream_t s) 
 template <class R> bool launch_row3(const StepArgs<R> &a, bool curl, bool upd, hipStream_t s) {
   static const bool off = getenv("MEEP_AMD_NO_ROW3") != nullptr;
   if (off) return false;
-  constexpr int V = 16 / sizeof(R), VP = V > 2 ? 2 : V; // the pole-carrying updates take 8-byte groups in FP32
+  // 16-byte groups with poles too: half the address and uPML work of 8-byte ones (384x384x192, two
+  // poles, FP32: the D interior 800 -> 768 us), which these kernels are bound by
+  constexpr int V = 16 / sizeof(R);
   const int PH = a.sgn < 0 ? 1 : 0;
   const bool u = upd;
   if (PH == 0) return u ? r3_launch<R, V, 0, true, 0>(a, curl, upd, s) : r3_launch<R, V, 0, false, 0>(a, curl, upd, s);
   if (!u) return r3_launch<R, V, 1, false, 0>(a, curl, upd, s);
   switch (a.npole) {
     case 0: return r3_launch<R, V, 1, true, 0>(a, curl, upd, s);
-    case 1: return r3_launch<R, VP, 1, true, 1>(a, curl, upd, s);
-    case 2: return r3_launch<R, VP, 1, true, 2>(a, curl, upd, s);
+    case 1: return r3_launch<R, V, 1, true, 1>(a, curl, upd, s);
+    case 2: return r3_launch<R, V, 1, true, 2>(a, curl, upd, s);
     default: return false;
   }
 }
