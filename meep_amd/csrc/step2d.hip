@@ -15,12 +15,13 @@
 // forms, currents, walls, E = chi1inv (D - P - dipoles) or H = B with the f_w branch, and the
 // poles; the uPML branches run only in tiles that meet a profile (uniform per block).
 //
-// Measured, 8 steps a launch: 320 x 160 FP64 (88 tiles) 27 us, of which the load is 4 us and a
-// tile's steps 5.4 us without uPML and 18-19 us in the uPML corners (instruction issue there);
-// per step 47 us -> 4.7 us with the monitors.  401 x 263 FP32 TE with a Drude pole and a field
-// map over the cell: 61 us -> 6.9 us a step.  Rows x columns 32 x 64 with 8 waves: 4 rows a
-// thread keep the state of a tile in registers (up to 256) with every neighbour but one in the
-// same wave.
+// What bounds it: instruction issue in the tiles that meet a uPML corner (about three times a
+// plain tile's time), then the load of a tile before its first step (4 us).  Per step with its
+// monitors, one-step kernels -> here: 320 x 160 FP64 (88 tiles) 47 us -> 5.2 us; 401 x 263 FP32
+// TE with a Drude pole and a field map over the cell 61 us -> 14.7 us; 64 squares of 128 to
+// 512 cells together 181 us -> 76 us.  Rows x columns 32 x 64 with 16 waves of 2 rows each: 4 rows a
+// thread and 8 waves have more neighbours in the same wave but half the waves to issue from
+// (32 us against 19 for up to 8 steps of a 400 x 300 FP32 cell).
 #include "engine.hpp"
 #include "stencil.hpp"
 
@@ -439,13 +440,13 @@ template <class R, bool TM, int NP, int NW, int K> struct Tile2d {
   template <bool FULL> __device__ __forceinline__ void steps(const Mons &mons) {
     constexpr int EC = TM ? 2 : 1, HC = TM ? 1 : 2; // the partners whose row neighbour crosses waves
     for (int s = 0; s < l.nsteps; ++s) {
-      if (TM)
+      if constexpr (TM)
         pair_phase<true, FULL>(s);
       else
         single_phase<true, FULL>(s);
       bH[(wave + 1) * S2_COLS + lane] = e[HC][K - 1];
       __syncthreads();
-      if (TM)
+      if constexpr (TM)
         single_phase<false, FULL>(s);
       else
         pair_phase<false, FULL>(s);
