@@ -308,8 +308,14 @@ struct DevBuf {
     alloc_allowed("a state, plan or staging buffer");
     if (p) (void)hipFree(p);
     p = nullptr;
+    bytes = 0; // the size of what is held: a failed allocation leaves an empty buffer
+    if (!n) return;
+    void *q = nullptr;
+    const hipError_t e = hipMalloc(&q, n);
+    if (e != hipSuccess) (void)hipGetLastError(); // reported here, not by a later launch's check
+    HIPCHECK(e);
+    p = q;
     bytes = n;
-    if (n) HIPCHECK(hipMalloc(&p, n));
   }
 };
 

@@ -16,6 +16,11 @@ OUT = os.path.join(HERE, "_build")
 LIB = os.path.join(OUT, "libmeep_host.so")
 
 
+# stubs that check the buffers a launch would write
+CHECKED = {"launch_farfield": ' if (!out || (a.segs > 1 && !partial) || (!a.px && a.npts > 1))'
+                              ' throw std::runtime_error("far-field launch without its buffers"); '}
+
+
 def launcher_stubs():
     """C++ source defining every `void|bool launch_*(...)` declared in engine.hpp with an empty
     body (a bool launcher reports that it launched nothing, so the host takes its general
@@ -24,7 +29,7 @@ def launcher_stubs():
     decls = re.findall(r"template <class R>\s*(void|bool) (launch_\w+)\(([^;]*?)\);", src, re.S)
     if not decls:
         raise RuntimeError("no launcher declarations found in engine.hpp")
-    out = ['#include "engine.hpp"', "namespace mx {"]
+    out = ['#include <stdexcept>', '#include "engine.hpp"', "namespace mx {"]
     out += [f"template <class R> {ret} {name}({args}) {{{' return false;' if ret == 'bool' else ''}}}"
             for ret, name, args in decls]
     for ret, name, args in decls:
@@ -35,8 +40,12 @@ def launcher_stubs():
     templated = {name for _, name, _ in decls}
     for ret, name, args in re.findall(r"^(void|bool) (launch_\w+)\(([^;]*?)\);", src, re.M | re.S):
         if name not in templated:
-            out.append(f"{ret} {name}({args}) {{{' return false;' if ret == 'bool' else ''}}}")
+            body = CHECKED.get(name, " return false;" if ret == "bool" else "")
+            out.append(f"{ret} {name}({args}) {{{body}}}")
     out.append("}")
+    # the allocation that fails next, and the count of allocations (tests of failure handling)
+    out.append('extern "C" void mock_fail_malloc(long after) { mock_mallocs_left = after; }')
+    out.append('extern "C" long mock_malloc_count() { return mock_mallocs; }')
     return "\n".join(out) + "\n"
 
 

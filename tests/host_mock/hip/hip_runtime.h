@@ -10,7 +10,7 @@
 #include <cstddef>
 #include <cstdint>
 typedef int hipError_t;
-enum { hipSuccess = 0, hipErrorNotReady = 600 };
+enum { hipSuccess = 0, hipErrorOutOfMemory = 2, hipErrorNotReady = 600 };
 typedef void *hipStream_t;
 typedef void *hipEvent_t;
 typedef void *hipGraph_t;
@@ -23,7 +23,18 @@ struct float2 { float x, y; };
 struct int2 { int x, y; };
 inline double2 make_double2(double a, double b) { return {a, b}; }
 inline float2 make_float2(float a, float b) { return {a, b}; }
-inline hipError_t hipMalloc(void **p, size_t n) { *p = calloc(1, n ? n : 1); return hipSuccess; }
+// allocations that succeed before the next one fails (-1: none fails), and the calls made so far
+inline long mock_mallocs_left = -1, mock_mallocs = 0;
+inline hipError_t hipMalloc(void **p, size_t n) {
+  ++mock_mallocs;
+  if (mock_mallocs_left == 0) {
+    mock_mallocs_left = -1;
+    return hipErrorOutOfMemory;
+  }
+  if (mock_mallocs_left > 0) --mock_mallocs_left;
+  *p = calloc(1, n ? n : 1);
+  return hipSuccess;
+}
 template <class T> inline hipError_t hipMalloc(T **p, size_t n) { return hipMalloc((void **)p, n); }
 inline hipError_t hipFree(void *p) { free(p); return hipSuccess; }
 inline hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind) { if (n) memmove(d, s, n); return hipSuccess; }
