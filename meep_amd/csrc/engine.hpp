@@ -496,18 +496,24 @@ struct FarArgs {
   double eps, mu;
   int dim, segs;
   int uniform; // freq[i] = freq[0] + i (freq[1] - freq[0]) to rounding
+  int group;   // frequencies a block takes (farfield_group)
 };
-// Frequencies a block takes together in 3D, sharing a current's geometry and its two phase
-// evaluations.  Full groups of 3 and of 5 cost the same per frequency (1218 us for 3, 2033 us for 5
-// on a plane of 1600 points and 41 k currents, against 1080 us for 2 and 866 us for 1; 4 runs out of
-// registers: 1690 us), so it is 3 unless only 5 leaves no remainder.
-inline int farfield_group(int dim, int nfreq) {
-  if (dim != 3 || nfreq < 1) return 1;
-  return nfreq % 5 == 0 && nfreq % 3 ? 5 : nfreq < 3 ? nfreq : 3;
+constexpr long FARFIELD_BLOCKS = 4096; // blocks that fill the chip many times over
+// Frequencies a block takes together in 3D, sharing a current's geometry and, where they are
+// uniformly spaced, its two phase evaluations.  Measured with 400 points and 10 k currents, us for
+// groups of 2 / 3 / 5: 5 uniform frequencies 394 / 381 / 517, 25 of them 1610 / 1460 / 1710, 4 of
+// them 314 / 353 / 562; 5 uneven ones 337 / 343 / 562, 4 of them 267 / 321 / 501.  So 2 for uneven
+// frequencies (a phase each: a larger group only costs registers) and where 3 leaves a
+// remainder of one of four; 3 for uniform ones.  5 where that leaves no remainder, 3 does, and
+// there are blocks to fill the chip without splitting the currents (its wave per SIMD needs long
+// loops): 4096 points, 41 k currents, 10 frequencies 13.7 / 13.8 / 12.4 ms (with the call's copies).
+inline int farfield_group(int dim, int nfreq, bool uniform, long npts) {
+  if (dim != 3 || nfreq < 2) return 1;
+  if (!uniform || nfreq == 2 || nfreq == 4) return 2;
+  return nfreq % 5 == 0 && nfreq % 3 && npts * (nfreq / 5) >= FARFIELD_BLOCKS ? 5 : 3;
 }
-// partial: npts * nfreq * segs * 12 doubles of scratch; done: a counter per (point, frequency
-// group), zero before and after; out: npts * nfreq * 12 doubles, the (re, im) of Ex Ey Ez Hx Hy Hz
-// per (point, frequency), point-major
-void launch_farfield(const FarArgs &a, double *partial, double *out, unsigned *done, hipStream_t s);
+// partial: npts * nfreq * segs * 12 doubles of scratch (unused by one segment); out: npts * nfreq
+// * 12 doubles, the (re, im) of Ex Ey Ez Hx Hy Hz per (point, frequency), point-major
+void launch_farfield(const FarArgs &a, double *partial, double *out, hipStream_t s);
 
 } // namespace mx

@@ -480,7 +480,7 @@ template <class R> struct N2F : Flux<R> {
   DevBuf sx, sy, sz, f0, d_freq;
   // scratch of the far-field calls, kept while it is small (three allocations and releases were
   // half of a call for one point)
-  DevBuf points, partial, out, done;
+  DevBuf points, partial, out;
   std::mutex in_use; // one call at a time has them
   void trim() {
     for (DevBuf *b : {&points, &partial, &out})
@@ -4530,10 +4530,6 @@ template <class R> struct Fields : FieldsBase {
     const long batch = std::max(1L, (1L << 20) / Nf);
     const long nb = std::min(np, batch);
     const long pairs_max = nb * Nf;
-    // Segments of the current list: enough blocks to fill the chip, down to one current a thread
-    // where a call has few points (a point of 1296 currents: 6 segments)
-    const long fb = farfield_group(gv.dim, Nf), bps = nb * ((Nf + fb - 1) / fb);
-    const int segs = int(std::max(1L, std::min<long>((n.nsrc + 255) / 256, (4096 + bps - 1) / bps)));
     // uniformly spaced frequencies (to a few ulps, as linspace makes them) let the kernel step
     // e^{ikr} from one frequency to the next
     bool uniform = Nf > 1;
@@ -4541,6 +4537,12 @@ template <class R> struct Fields : FieldsBase {
       const double want = n.freq[0] + i * (n.freq[1] - n.freq[0]);
       uniform = std::fabs(n.freq[i] - want) <= 8 * DBL_EPSILON * std::max(std::fabs(n.freq[i]), std::fabs(n.freq[0]));
     }
+    // Segments of the current list: enough blocks to fill the chip, of two currents a thread at
+    // least (one a thread: a point of 10 k currents at 10 frequencies 66 us against 50, the wider
+    // sum over segments)
+    const int fb = farfield_group(gv.dim, Nf, uniform, nb);
+    const long bps = nb * ((Nf + fb - 1) / fb);
+    const int segs = int(std::max(1L, std::min<long>((n.nsrc + 511) / 512, (FARFIELD_BLOCKS + bps - 1) / bps)));
     std::lock_guard<std::mutex> hold(n.in_use);
     auto room = [](DevBuf &b, size_t bytes) {
       if (b.bytes < bytes) b.alloc(bytes);
@@ -4548,10 +4550,6 @@ template <class R> struct Fields : FieldsBase {
     if (nb > 1) room(n.points, 8 * 3 * size_t(nb));
     room(n.partial, 8 * 12 * size_t(pairs_max) * size_t(segs > 1 ? segs : 0));
     room(n.out, 8 * 12 * size_t(pairs_max));
-    if (n.done.bytes < sizeof(unsigned) * size_t(bps)) {
-      n.done.alloc(sizeof(unsigned) * size_t(bps));
-      HIPCHECK(hipMemsetAsync(n.done.p, 0, n.done.bytes, stream));
-    }
     std::vector<double> soa(3 * size_t(nb));
     for (long b0 = 0; b0 < np; b0 += nb) {
       const long m = std::min(nb, np - b0);
@@ -4575,8 +4573,9 @@ template <class R> struct Fields : FieldsBase {
       a.dim = gv.dim;
       a.segs = segs;
       a.uniform = uniform ? 1 : 0;
+      a.group = fb;
       kbegin(7);
-      launch_farfield(a, static_cast<double *>(n.partial.p), static_cast<double *>(n.out.p), static_cast<unsigned *>(n.done.p), stream);
+      launch_farfield(a, static_cast<double *>(n.partial.p), static_cast<double *>(n.out.p), stream);
       HIPCHECK(hipGetLastError());
       kend();
       HIPCHECK(hipMemcpyAsync(out + size_t(b0) * Nf * 12, n.out.p, 8 * 12 * size_t(m) * Nf, hipMemcpyDeviceToHost, stream));
@@ -5946,8 +5945,8 @@ int mp_near2far_green(int dim, const double *x, double freq, double eps, double 
     a.sx = d + 2, a.sy = d + 3, a.sz = d + 4, a.px = d + 5, a.py = d + 6, a.pz = d + 7, a.freq = d + 8;
     const int cls = c0 < 5 ? (c0 == 4 ? 2 : c0) : (c0 == 9 ? 5 : c0 - 2);
     for (int c = 0; c <= 6; ++c) a.cls_lo[c] = c > cls ? 1 : 0;
-    a.nsrc = 1, a.npts = 1, a.nfreq = 1, a.eps = eps, a.mu = mu, a.dim = dim, a.segs = 1, a.uniform = 0;
-    launch_farfield(a, static_cast<double *>(part.p), static_cast<double *>(outb.p), nullptr, nullptr); // one segment: no counter
+    a.nsrc = 1, a.npts = 1, a.nfreq = 1, a.eps = eps, a.mu = mu, a.dim = dim, a.segs = 1, a.uniform = 0, a.group = 1;
+    launch_farfield(a, static_cast<double *>(part.p), static_cast<double *>(outb.p), nullptr); // one segment: no partials
     HIPCHECK(hipGetLastError());
     HIPCHECK(hipMemcpy(EH, outb.p, 12 * 8, hipMemcpyDeviceToHost));
   });

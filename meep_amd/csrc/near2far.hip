@@ -9,8 +9,8 @@
 // consecutive frequencies and one segment of the current list; its 256 threads stride over the
 // segment, compute each current's geometry once for the group, keep the six complex fields of
 // each frequency in registers, and reduce them through the wave and LDS into one partial per
-// frequency.  A second pass adds the partials of each (point, frequency) in segment order, so
-// the result does not depend on timing.
+// frequency.  Where the list is split, a second launch adds the partials of each (point,
+// frequency) in segment order, so the result does not depend on timing.
 //
 // The currents come as SoA lists prepared on the host, sorted by class (Ex Ey Ez Hx Hy Hz):
 // position x, y, z and one amplitude per frequency (frequency-major, so a block's reads of one
@@ -19,6 +19,8 @@
 #include "engine.hpp"
 
 #include <hip/hip_runtime.h>
+
+#include <stdexcept>
 
 namespace mx {
 
@@ -228,10 +230,12 @@ __device__ __forceinline__ void far_classes(Cx (&acc)[FB][6], const FarArgs &a, 
 // (distance, direction, 1/r) is computed once for the group.  In 3D, when the frequencies are
 // uniformly spaced (a.uniform), e^{ikr} of the group's later frequencies follows from the
 // first by repeated multiplication with e^{i dk r}, two phase evaluations per current and
-// group.  The
-// currents come sorted by class (Ex Ey Ez Hx Hy Hz, a.cls_lo), so each class runs a loop of
-// its own with its direction and kind known at compile time.
-template <int DIM, int FB> __global__ __launch_bounds__(FF_BLOCK) void k_farfield(FarArgs a, double *partial, double *out, unsigned *done) {
+// group.  The currents come sorted by class (Ex Ey Ez Hx Hy Hz, a.cls_lo), so each class runs a
+// loop of its own with its direction and kind known at compile time.  The segments' partials are
+// added by a second launch: when each point's last block added them, the fence it takes for that
+// in every block (the XCDs' L2s are written back) made a plane of 400 points slower, 128 -> 552 us
+// at one frequency.
+template <int DIM, int FB> __global__ __launch_bounds__(FF_BLOCK) void k_farfield(FarArgs a, double *partial, double *out) {
   const int b = blockIdx.x;
   const int ngroup = (a.nfreq + FB - 1) / FB;
   const int pair = b / a.segs, seg = b - pair * a.segs;
@@ -266,7 +270,6 @@ template <int DIM, int FB> __global__ __launch_bounds__(FF_BLOCK) void k_farfiel
   const int nq = g.nq;
   // wave reduction, then across the block's waves through LDS; one partial per frequency
   __shared__ double red[FF_BLOCK / 64][12];
-  __shared__ bool last;
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
 #pragma unroll
   for (int q = 0; q < FB; ++q) {
@@ -292,42 +295,36 @@ template <int DIM, int FB> __global__ __launch_bounds__(FF_BLOCK) void k_farfiel
     }
     __syncthreads();
   }
-  if (a.segs == 1) return;
-  // The pair's last block to finish adds the segments' partials, in segment order whichever block
-  // it is (a second launch took 3.2 us of a 40 us call).  Each block publishes its partials
-  // before it counts itself, and the count is left at zero for the next launch.
-  __threadfence();
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    last = __hip_atomic_fetch_add(done + pair, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == unsigned(a.segs) - 1;
-    if (last) __hip_atomic_store(done + pair, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  }
-  __syncthreads();
-  if (!last) return;
-  __threadfence();
-  for (int t = int(threadIdx.x); t < nq * 12; t += FF_BLOCK) {
-    const int q = t / 12, c = t - q * 12;
-    double sum = 0;
-    for (int z = 0; z < a.segs; ++z)
-      sum += __hip_atomic_load(partial + ((size_t(p) * a.nfreq + f_first + q) * a.segs + z) * 12 + c, __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_AGENT);
-    out[(size_t(p) * a.nfreq + f_first + q) * 12 + c] = sum;
-  }
 }
 
-void launch_farfield(const FarArgs &a, double *partial, double *out, unsigned *done, hipStream_t s) {
-  const int fb = farfield_group(a.dim, a.nfreq);
+// out[pair * 12 + q] = the sum over the pair's segments, in segment order
+__global__ void k_farfield_sum(const double *partial, int npair, int segs, double *out) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= npair * 12) return;
+  const int pair = t / 12, q = t - pair * 12;
+  double s = 0;
+  for (int g = 0; g < segs; ++g) s += partial[(size_t(pair) * segs + g) * 12 + q];
+  out[t] = s;
+}
+
+void launch_farfield(const FarArgs &a, double *partial, double *out, hipStream_t s) {
+  const int fb = a.dim == 3 ? a.group : 1;
   const size_t nblk = size_t(a.npts) * ((a.nfreq + fb - 1) / fb) * a.segs;
   const dim3 grid{unsigned(nblk)}, block(FF_BLOCK);
   if (a.dim != 3)
-    hipLaunchKernelGGL((k_farfield<2, 1>), grid, block, 0, s, a, partial, out, done);
+    hipLaunchKernelGGL((k_farfield<2, 1>), grid, block, 0, s, a, partial, out);
   else
     switch (fb) {
-      case 1: hipLaunchKernelGGL((k_farfield<3, 1>), grid, block, 0, s, a, partial, out, done); break;
-      case 2: hipLaunchKernelGGL((k_farfield<3, 2>), grid, block, 0, s, a, partial, out, done); break;
-      case 3: hipLaunchKernelGGL((k_farfield<3, 3>), grid, block, 0, s, a, partial, out, done); break;
-      default: hipLaunchKernelGGL((k_farfield<3, 5>), grid, block, 0, s, a, partial, out, done); break;
+      case 1: hipLaunchKernelGGL((k_farfield<3, 1>), grid, block, 0, s, a, partial, out); break;
+      case 2: hipLaunchKernelGGL((k_farfield<3, 2>), grid, block, 0, s, a, partial, out); break;
+      case 3: hipLaunchKernelGGL((k_farfield<3, 3>), grid, block, 0, s, a, partial, out); break;
+      case 5: hipLaunchKernelGGL((k_farfield<3, 5>), grid, block, 0, s, a, partial, out); break;
+      default: throw std::runtime_error("meep: internal: bad far-field group");
     }
+  if (a.segs > 1) {
+    const int npair = a.npts * a.nfreq;
+    hipLaunchKernelGGL(k_farfield_sum, dim3((npair * 12 + 255) / 256), dim3(256), 0, s, partial, npair, a.segs, out);
+  }
 }
 
 } // namespace mx
