@@ -295,6 +295,10 @@ static void alloc_allowed(const char *what) {
          "with mp_fields_step_n first",
          what);
 }
+struct OutOfMemory : mx_error {
+  explicit OutOfMemory(size_t n)
+      : mx_error("meep: HIP error " + std::string(hipGetErrorString(hipErrorOutOfMemory)) + ": " + std::to_string(n) + " bytes") {}
+};
 struct DevBuf {
   void *p = nullptr;
   size_t bytes = 0;
@@ -313,6 +317,7 @@ struct DevBuf {
     void *q = nullptr;
     const hipError_t e = hipMalloc(&q, n);
     if (e != hipSuccess) (void)hipGetLastError(); // reported here, not by a later launch's check
+    if (e == hipErrorOutOfMemory) throw OutOfMemory(n);
     HIPCHECK(e);
     p = q;
     bytes = n;
@@ -2227,44 +2232,28 @@ template <class R> struct Fields : FieldsBase {
   struct S2Plan {
     long plan_v = -1, dft_v = -1, src_v = -1, ptr_v = -1, builds = 0;
     int margin = 0; // steps a tile has room for
-    bool ok = false;
+    bool shape = false, ok = false;
     std::vector<std::unique_ptr<S2Set>> sets;
   } s2;
-  std::map<const void *, std::unique_ptr<DevBuf>> s2_alt; // each state array's second buffer
+  // each state array's second buffer, in one allocation
+  DevBuf s2_pool;
+  std::map<const void *, char *> s2_alt;
   bool s2_off = getenv("MEEP_AMD_NO_TILE2D") != nullptr;
-  bool s2_nomem = false;
-  // the second buffer of a state array, made as a copy of it; null when memory is short
-  template <class T> T *s2_second(const T *p) {
-    std::unique_ptr<DevBuf> &b = s2_alt[p];
-    if (!b) {
-      std::unique_ptr<DevBuf> n(new DevBuf);
-      if (hipMalloc(&n->p, sizeof(T) * gv.ntot) != hipSuccess) {
-        (void)hipGetLastError();
-        n->p = nullptr;
-        s2_nomem = true;
-        return nullptr;
-      }
-      n->bytes = sizeof(T) * gv.ntot;
-      HIPCHECK(hipMemcpyAsync(n->p, p, sizeof(T) * gv.ntot, hipMemcpyDeviceToDevice, stream));
-      b = std::move(n);
-    }
-    return static_cast<T *>(b->p);
-  }
-  // Whether the tile kernel takes this chunk's next steps: 2D, no periodic halos, no
-  // conductivity, no magnetic poles and at most S2_POLES electric ones, every source in a table
-  // or box, every DFT chunk in the deferred group, and nothing left to allocate.
-  bool s2_ready(int margin) {
+  // Whether the tile kernel can take this chunk's next steps, memory apart: 2D, no periodic
+  // halos, no conductivity, no magnetic poles and at most S2_POLES electric ones, every source in
+  // a table or box, every DFT chunk of the deferred form, and no state array left to allocate.
+  bool s2_shape(int margin) {
     if (s2_off || gv.dim != 2 || !use_fast || whole_rows_env >= 0) return false;
     if (!plan_valid || srcplan_stale() || t > INT32_MAX / 2) return false;
     if (s2.plan_v == plan_version && s2.dft_v == dft_version && s2.src_v == src_version && s2.ptr_v == ptr_version && s2.margin == margin)
-      return s2.ok;
+      return s2.shape;
     s2.margin = margin;
     ++s2.builds;
     s2.plan_v = plan_version;
     s2.dft_v = dft_version;
     s2.src_v = src_version;
     s2.ptr_v = ptr_version;
-    s2.ok = false;
+    s2.shape = s2.ok = false;
     s2.sets.clear();
     if (any_cond || n_conn[0] || n_conn[1] || wrap_dir[0] || wrap_dir[1] || have_fmp_H() || int(pols.size()) > S2_POLES) return false;
     for (auto &p : pols)
@@ -2284,7 +2273,7 @@ template <class R> struct Fields : FieldsBase {
         if (upd_pending(cmp, which, 3, ph && fmp)) return false;
       }
     if (splan.rec.size() > S2_VALS || dft_chunks.size() > S2_MONS) return false;
-    if (!dft_chunks.empty() && !dft_group()) return false;
+    if (!dft_chunks.empty() && !dft_groupable()) return false;
     for (auto &cp : dft_chunks)
       if (!f[cp->c][0]) return false;
     if (!boxes_valid) compute_boxes();
@@ -2295,16 +2284,83 @@ template <class R> struct Fields : FieldsBase {
       if (!have) continue;
       if (have != 3 || !s2_set(tm, fmp)) return false;
     }
-    if (s2_nomem) { // no room for the second buffers: one step per launch
-      HIPCHECK(hipStreamSynchronize(stream));
-      s2.sets.clear();
-      s2_alt.clear();
-      s2_off = true;
-      return false;
-    }
-    return s2.ok = !s2.sets.empty();
+    return s2.shape = !s2.sets.empty();
   }
-  // the launch arguments and monitor tables of one polarisation; false when its plan has
+  // ... and its second buffers and tables are in place.  Where memory for them is short the chunk
+  // keeps stepping one by one.
+  bool s2_ready(int margin) {
+    if (!s2_shape(margin)) return false;
+    if (s2.ok) return true;
+    try {
+      s2.ok = s2_second() && (dft_chunks.empty() || dft_group());
+      for (auto &S : s2.sets)
+        if (s2.ok) s2_finish(*S);
+    } catch (const OutOfMemory &) {
+      s2.ok = false;
+    }
+    if (!s2.ok) {
+      s2_drop();
+      s2_off = true;
+    }
+    return s2.ok;
+  }
+  // the second buffers and the plan given back
+  void s2_drop() {
+    HIPCHECK(hipStreamSynchronize(stream));
+    s2.plan_v = -1;
+    s2.shape = s2.ok = false;
+    s2.sets.clear();
+    s2_alt.clear();
+    s2_pool.alloc(0);
+  }
+  // The arrays of a set's arguments and the second pointers beside them, as (array, second
+  // pointer, bytes of an element).
+  template <class F> static void s2_pairs(Step2dArgs<R> &a, F &&fn) {
+    for (S2Comp<R> &c : a.c) {
+      fn(c.f, c.fo);
+      fn(c.e, c.eo);
+      fn(c.fu, c.fuo);
+      fn(c.fw, c.fwo);
+      for (int p = 0; p < S2_POLES; ++p) fn(c.P[p], c.Po[p]), fn(c.Pp[p], c.Ppo[p]);
+    }
+  }
+  // Second buffers of every array of the plan, copies of the arrays; false where they would not
+  // fit, or would leave less than half of the device's memory free: a chunk so large is no
+  // longer bound by launches, and what its owner allocates later has to fit as it did without them.
+  bool s2_second() {
+    std::vector<std::pair<const void *, size_t>> need;
+    bool have = true;
+    for (auto &S : s2.sets)
+      for (int cmp = 0; cmp < ncmp(); ++cmp)
+        s2_pairs(S->a[cmp][0], [&](auto *in, auto *) {
+          if (!in) return;
+          need.push_back({in, sizeof(*in) * gv.ntot});
+          have = have && s2_alt.count(in);
+        });
+    if (!have) {
+      size_t total = 0, free = 0, all = 0;
+      for (auto &q : need) total += (q.second + 255) / 256 * 256;
+      HIPCHECK(hipStreamSynchronize(stream));
+      s2_alt.clear();
+      s2_pool.alloc(0);
+      HIPCHECK(hipMemGetInfo(&free, &all));
+      if (free < total || free - total < all / 2) return false;
+      s2_pool.alloc(total);
+      char *at = static_cast<char *>(s2_pool.p);
+      for (auto &q : need) {
+        s2_alt[q.first] = at;
+        HIPCHECK(hipMemcpyAsync(at, q.first, q.second, hipMemcpyDeviceToDevice, stream));
+        at += (q.second + 255) / 256 * 256;
+      }
+    }
+    for (auto &S : s2.sets)
+      for (int cmp = 0; cmp < ncmp(); ++cmp)
+        s2_pairs(S->a[cmp][0], [&](auto *in, auto *&out) {
+          if (in) out = reinterpret_cast<std::remove_reference_t<decltype(out)>>(s2_alt.at(in));
+        });
+    return true;
+  }
+  // the launch arguments of one polarisation, second pointers apart; false when its plan has
   // another shape than the kernel's
   bool s2_set(bool tm, bool fmp) {
     std::unique_ptr<S2Set> S(new S2Set);
@@ -2374,21 +2430,17 @@ template <class R> struct Fields : FieldsBase {
         if (!u.f && d < 2 && pml_in(d)) return false;
         if ((k.dsigu >= 0 && !k.fu) || (u.f && u.dsigw >= 0 && !u.fw)) return false;
         c.f = k.f;
-        c.fo = s2_second(k.f);
         if (u.f) {
           c.e = u.f;
-          c.eo = s2_second(static_cast<const R *>(u.f));
           c.chi = u.u;
         }
-        if (k.dsigu >= 0) c.fu = k.fu, c.fuo = s2_second(static_cast<const double *>(k.fu));
-        if (u.f && u.dsigw >= 0) c.fw = u.fw, c.fwo = s2_second(static_cast<const double *>(u.fw));
+        if (k.dsigu >= 0) c.fu = k.fu;
+        if (u.f && u.dsigw >= 0) c.fw = u.fw;
         if (!mag && u.f)
           for (int p = 0; p < a.npole; ++p) {
             if (!u.P[p]) continue;
             c.P[p] = u.P[p];
             c.Pp[p] = u.Pp[p];
-            c.Po[p] = s2_second(static_cast<const R *>(u.P[p]));
-            c.Ppo[p] = s2_second(static_cast<const R *>(u.Pp[p]));
             c.sigma[p] = u.sigma[p];
             c.sigval[p] = u.sigval[p];
             if ((u.sigone >> p) & 1) c.sigone |= 1 << p;
@@ -2397,29 +2449,26 @@ template <class R> struct Fields : FieldsBase {
         for (int q = 0; q < 2; ++q) c.lo[q] = ax.lo[1 + q], c.hi[q] = ax.hi[1 + q], c.mhi[q] = ax.mhi[1 + q], c.mlo[q] = ax.mlo[1 + q];
       }
     }
-    s2_monitors(*S);
-    for (int cmp = 0; cmp < ncmp(); ++cmp) { // the other parity: every pair exchanged
-      s2_check(S->a[cmp][0]);
-      S->a[cmp][1] = S->a[cmp][0];
-      for (S2Comp<R> &c : S->a[cmp][1].c) {
-        auto swap = [](auto *&in, auto *&out) {
+    s2.sets.push_back(std::move(S));
+    return true;
+  }
+  // a set's monitor tables, its arguments for the other parity (every pair exchanged), and the upload
+  void s2_finish(S2Set &S) {
+    s2_monitors(S);
+    std::vector<Step2dArgs<R>> all;
+    for (int cmp = 0; cmp < 2; ++cmp) {
+      if (cmp < ncmp()) {
+        s2_check(S.a[cmp][0]);
+        S.a[cmp][1] = S.a[cmp][0];
+        s2_pairs(S.a[cmp][1], [](auto *&in, auto *&out) {
           auto *o = out;
           out = const_cast<std::remove_const_t<std::remove_pointer_t<std::remove_reference_t<decltype(in)>>> *>(in);
           in = o;
-        };
-        swap(c.f, c.fo);
-        swap(c.e, c.eo);
-        swap(c.fu, c.fuo);
-        swap(c.fw, c.fwo);
-        for (int p = 0; p < S2_POLES; ++p) swap(c.P[p], c.Po[p]), swap(c.Pp[p], c.Ppo[p]);
+        });
       }
+      for (int par = 0; par < 2; ++par) all.push_back(S.a[cmp][par]);
     }
-    std::vector<Step2dArgs<R>> all;
-    for (int cmp = 0; cmp < 2; ++cmp)
-      for (int par = 0; par < 2; ++par) all.push_back(S->a[cmp][par]);
-    upload_vec(S->args, all);
-    s2.sets.push_back(std::move(S));
-    return true;
+    upload_vec(S.args, all);
   }
   // every pointer the tile kernel can dereference, and the tiles against its registers and lanes
   static void s2_check(const Step2dArgs<R> &a) {
@@ -2965,7 +3014,7 @@ template <class R> struct Fields : FieldsBase {
       const void *from = a.p;
       if (second) {
         auto it = s2_alt.find(a.p);
-        if (it != s2_alt.end()) from = it->second->p;
+        if (it != s2_alt.end()) from = it->second;
       }
       HIPCHECK(hipMemcpyAsync(cp.data.back()->p, from, a.esz * gv.ntot, hipMemcpyDeviceToDevice, stream));
     }
@@ -3454,7 +3503,7 @@ template <class R> struct Fields : FieldsBase {
   // every chunk's phases fit the flush kernel's table.
   struct DftGroup {
     long dft_v = -1, plan_v = -1;
-    bool ok = false;
+    bool fits = false, built = false, ok = false;
     DevBuf items, snap_item, snap_first, flush_item, flush_first;
     unsigned snap_nblk = 0, flush_nblk = 0;
     std::vector<int> decs; // the chunks' distinct decimations
@@ -3466,37 +3515,51 @@ template <class R> struct Fields : FieldsBase {
     }
     bool hits(long t0, long t1) const { return most_hits(t0, t1) > 0; }
   } dgroup;
-  bool dft_group() {
-    if (dgroup.dft_v == dft_version && dgroup.plan_v == plan_version) return dgroup.ok;
+  // whether every chunk's phases fit the flush kernel's table (no device memory needed)
+  bool dft_groupable() {
+    if (dgroup.dft_v == dft_version && dgroup.plan_v == plan_version) return dgroup.fits;
     flush_dft_group(); // steps deferred under the old tables
     dgroup.dft_v = dft_version;
     dgroup.plan_v = plan_version;
-    dgroup.ok = false;
+    dgroup.fits = dgroup.built = dgroup.ok = false;
     dgroup.decs.clear();
-    std::vector<BatchDft<R>> items;
-    std::vector<uint32_t> pts, quads, item, first;
     for (auto &cp : dft_chunks) {
       DftChunk<R> &ch = *cp;
       if (!f[ch.c][0]) continue;
       if (std::find(dgroup.decs.begin(), dgroup.decs.end(), ch.decimation) == dgroup.decs.end()) dgroup.decs.push_back(ch.decimation);
       if (ch.defer < DFT_DEFER || ch.npts < 1) return false;
-      if (ch.nsnap) fail("internal: deferred DFT steps pending");
-      items.push_back(batch_dft(ch));
-      pts.push_back(uint32_t(ch.npts));
-      const size_t q = size_t(ch.npts) * size_t((ch.nfreq + 3) / 4);
-      if (q >= (size_t(1) << 31)) return false;
-      quads.push_back(uint32_t(q));
+      if (size_t(ch.npts) * size_t((ch.nfreq + 3) / 4) >= (size_t(1) << 31)) return false;
     }
-    if (items.empty()) return false;
-    upload_vec(dgroup.items, items);
-    block_tables(pts, 256, item, first);
-    upload_vec(dgroup.snap_item, item);
-    upload_vec(dgroup.snap_first, first);
-    dgroup.snap_nblk = unsigned(item.size());
-    block_tables(quads, 256, item, first);
-    upload_vec(dgroup.flush_item, item);
-    upload_vec(dgroup.flush_first, first);
-    dgroup.flush_nblk = unsigned(item.size());
+    return dgroup.fits = !dgroup.decs.empty();
+  }
+  // the tables; false where memory for them is short (each chunk then accumulates by itself)
+  bool dft_group() {
+    if (!dft_groupable()) return false;
+    if (dgroup.built) return dgroup.ok;
+    dgroup.built = true;
+    try {
+      std::vector<BatchDft<R>> items;
+      std::vector<uint32_t> pts, quads, item, first;
+      for (auto &cp : dft_chunks) {
+        DftChunk<R> &ch = *cp;
+        if (!f[ch.c][0]) continue;
+        if (ch.nsnap) fail("internal: deferred DFT steps pending");
+        items.push_back(batch_dft(ch));
+        pts.push_back(uint32_t(ch.npts));
+        quads.push_back(uint32_t(size_t(ch.npts) * size_t((ch.nfreq + 3) / 4)));
+      }
+      upload_vec(dgroup.items, items);
+      block_tables(pts, 256, item, first);
+      upload_vec(dgroup.snap_item, item);
+      upload_vec(dgroup.snap_first, first);
+      dgroup.snap_nblk = unsigned(item.size());
+      block_tables(quads, 256, item, first);
+      upload_vec(dgroup.flush_item, item);
+      upload_vec(dgroup.flush_first, first);
+      dgroup.flush_nblk = unsigned(item.size());
+    } catch (const OutOfMemory &) {
+      return false;
+    }
     return dgroup.ok = true;
   }
   // the open window of deferred steps: window_t + 1 .. window_end
@@ -4916,11 +4979,20 @@ template <class R> struct Batch : BatchBase {
   std::vector<int> tile_decs;
   bool tiles_ready() {
     bool fresh = tile_builds.size() == sims.size();
-    for (Fields<R> *F : sims)
-      if (!F->s2_ready(S2_BATCH)) {
-        tile_builds.clear();
-        return false;
-      }
+    // every member's shape before any member allocates: second buffers are of no use to a batch
+    // that the kernel does not take whole
+    bool ready = true;
+    for (Fields<R> *F : sims) ready = ready && F->s2_shape(S2_BATCH);
+    if (ready) {
+      for (Fields<R> *F : sims) ready = ready && F->s2_ready(S2_BATCH);
+      if (!ready) // memory is short
+        for (Fields<R> *F : sims) F->s2_drop();
+    }
+    if (!ready) {
+      tile_builds.clear();
+      tgroups.clear();
+      return false;
+    }
     for (size_t q = 0; q < sims.size() && fresh; ++q) fresh = tile_builds[q] == sims[q]->s2.builds;
     if (fresh) return true;
     tgroups.clear();

@@ -45,6 +45,7 @@ def launcher_stubs():
     out.append("}")
     # the allocation that fails next, and the count of allocations (tests of failure handling)
     out.append('extern "C" void mock_fail_malloc(long after) { mock_mallocs_left = after; }')
+    out.append('extern "C" void mock_set_free(size_t n) { mock_free = n; }')
     out.append('extern "C" long mock_malloc_count() { return mock_mallocs; }')
     return "\n".join(out) + "\n"
 

@@ -35,6 +35,9 @@ inline hipError_t hipMalloc(void **p, size_t n) {
   *p = calloc(1, n ? n : 1);
   return hipSuccess;
 }
+// free and total device memory as hipMemGetInfo gives them
+inline size_t mock_free = size_t(256) << 30, mock_total = size_t(288) << 30;
+inline hipError_t hipMemGetInfo(size_t *f, size_t *t) { *f = mock_free, *t = mock_total; return hipSuccess; }
 template <class T> inline hipError_t hipMalloc(T **p, size_t n) { return hipMalloc((void **)p, n); }
 inline hipError_t hipFree(void *p) { free(p); return hipSuccess; }
 inline hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind) { if (n) memmove(d, s, n); return hipSuccess; }

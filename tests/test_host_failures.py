@@ -13,14 +13,17 @@ from meep_amd.capi import Ez, MeepError, fields, gaussian_src_time, structure
 @pytest.fixture(scope="module")
 def host_lib():
     from host_mock import build
-    return capi.bind(ctypes.CDLL(build.build()))
+    lib = capi.bind(ctypes.CDLL(build.build()))
+    lib.mock_fail_malloc.argtypes = [ctypes.c_long]
+    lib.mock_set_free.argtypes = [ctypes.c_size_t]
+    lib.mock_malloc_count.restype = ctypes.c_long
+    return lib
 
 
 def test_far_fields_after_a_failed_allocation(host_lib):
     """A far-field call whose scratch cannot be allocated raises; the next one allocates it (the
     scratch outlives a call, and a launch with a buffer that was never allocated would write
     through a null pointer)."""
-    host_lib.mock_fail_malloc.argtypes = [ctypes.c_long]
     for after in range(20):
         s = structure(host_lib, dim=2, size=(3.0, 2.5), a=10, pml=[(d, side, 0.5) for d in (0, 1) for side in (0, 1)])
         f = fields(s)
@@ -41,3 +44,97 @@ def test_far_fields_after_a_failed_allocation(host_lib):
         if not failed:
             break
     assert after >= 2 and not failed  # some allocation was made to fail, and the last round reached none
+
+
+def plain_2d(lib, nx=40, ny=60):
+    s = structure(lib, dim=2, size=(nx / 10, ny / 10), a=10, pml=capi.pml(0.3)[:4])
+    s.set_chi1inv(Ez, np.full(s.shape, 0.5))
+    s.add_susceptibility(lambda x, y, z: 1.0 if x < 2.0 else 0.0, 1.0, 0.1)
+    f = fields(s)
+    f.use_real_fields()
+    f.add_volume_source(Ez, gaussian_src_time(0.6, 0.6), (1.5, 2.0, 0), (1.5, 2.0, 0))
+    f.add_dft_flux(0, (2.5, 1.0, 0), (2.5, 5.0, 0), np.linspace(0.4, 0.8, 3), decimation_factor=1)
+    f.step()
+    return s, f
+
+
+def _raised(lib):
+    """How many of the allocations of a step_n call raise when they fail; the call after one that
+    raised, and the steps after one that did not, always go on."""
+    n = 0
+    for after in range(60):
+        s, f = plain_2d(lib)
+        lib.mock_fail_malloc(after)
+        before = lib.mock_malloc_count()
+        try:
+            f.step_n(16)
+            assert f.t == 17
+        except MeepError as e:
+            assert "internal" not in str(e)
+            n += 1
+        made = lib.mock_malloc_count() - before
+        lib.mock_fail_malloc(-1)
+        t = f.t
+        f.step_n(16)
+        f.step()
+        assert f.t == t + 17
+        if made <= after:
+            return n
+    raise AssertionError("every round ran out of memory")
+
+
+def test_second_buffers_that_do_not_fit(host_lib, monkeypatch):
+    """A 2D chunk whose second buffers or tile tables cannot be allocated steps one by one: no
+    allocation raises that does not raise without the tile kernel."""
+    monkeypatch.setenv("MEEP_AMD_NO_TILE2D", "1")
+    plain = _raised(host_lib)
+    monkeypatch.delenv("MEEP_AMD_NO_TILE2D")
+    assert _raised(host_lib) <= plain
+
+
+def _allocations(lib, call):
+    before = lib.mock_malloc_count()
+    call()
+    return lib.mock_malloc_count() - before
+
+
+def test_second_buffers_leave_half_of_the_memory(host_lib, monkeypatch):
+    """With less than half of the device's memory left the chunk takes no second buffers."""
+    host_lib.mock_set_free(144 << 30)
+    try:
+        s, f = plain_2d(host_lib)
+        short = _allocations(host_lib, lambda: f.step_n(16))
+    finally:
+        host_lib.mock_set_free(256 << 30)
+    s, f = plain_2d(host_lib)
+    ample = _allocations(host_lib, lambda: f.step_n(16))
+    monkeypatch.setenv("MEEP_AMD_NO_TILE2D", "1")
+    s, f = plain_2d(host_lib)
+    assert short == _allocations(host_lib, lambda: f.step_n(16)) < ample
+
+
+@pytest.mark.parametrize("short", [False, True], ids=["3d_member", "memory"])
+def test_batch_that_the_tile_kernel_does_not_take(host_lib, monkeypatch, short):
+    """A batch with a member that the tile kernel does not take, or without the memory for its
+    second buffers, steps all of its members one by one; no member allocates second buffers
+    that the batch then does not use."""
+    def run():
+        sims = [plain_2d(host_lib, 40 + 7 * q, 50) for q in range(3)]
+        if not short:
+            s = structure(host_lib, dim=3, size=(1.2, 1.0, 1.0), a=10)
+            f = fields(s)
+            f.add_volume_source(Ez, gaussian_src_time(0.6, 0.6), (0.5, 0.5, 0.5), (0.5, 0.5, 0.5))
+            f.step()
+            sims.append((s, f))
+        b = capi.batch([f for _, f in sims], use_graph=False, autotune=False)
+        n = _allocations(host_lib, lambda: b.step_n(12))
+        assert all(f.t == 13 for _, f in sims)
+        return n
+    if short:
+        host_lib.mock_set_free(144 << 30)
+    try:
+        got = run()
+    finally:
+        host_lib.mock_set_free(256 << 30)
+    monkeypatch.setenv("MEEP_AMD_NO_TILE2D", "1")
+    assert got == run()
