@@ -2210,6 +2210,7 @@ template <class R> struct Fields : FieldsBase {
   void advance(long n, bool probe) {
     for (long q = 0; q < n;) {
       const long tail = probe && !flux_vols.empty() ? 1 : 0;
+      rows_hint = n - q;
       if (n - q - tail >= 2 && (dft_defer_steps || dft_off) && s2_ready(S2_STEPS)) {
         const long did = s2_run(n - q - tail);
         q += did;
@@ -2218,7 +2219,6 @@ template <class R> struct Fields : FieldsBase {
           continue;
         }
       }
-      rows_hint = n - q;
       one_step(probe && q == n - 1);
       ++q;
     }
@@ -2550,6 +2550,24 @@ template <class R> struct Fields : FieldsBase {
       b.nmon = int(mons[cmp].size());
     }
   }
+  // Everything that the next m steps allocate, before the first of them: an allocation that failed
+  // between two launches would leave the state in the second buffers, where no reader looks.
+  void s2_reserve(long m) {
+    if (src_row(t) && rows_t0 + rows_n < t + m) { // rows of an earlier call that end too soon
+      rows_n = 0;
+      src_row(t);
+    }
+    if (!adj || !adj->recording) return;
+    Adj &A = *adj;
+    if (A.interval > 0) {
+      if (seg_active) return;
+      const long first = t - A.t0;
+      for (long q = first / A.interval + 1; q * A.interval <= first + m; ++q)
+        if (A.spare.size() < size_t(q - first / A.interval)) A.spare.push_back(state_copies());
+    }
+    else
+      while (long(A.hist.size()) * HBLK < A.nrec + m) add_history_block();
+  }
   // Up to m steps by the tile kernel; returns the steps taken.  The launches of a call come in
   // an even number, so that the state ends where every other reader has it: a last launch that
   // would leave it in the second buffers is split in two, and a single step is left to the
@@ -2558,6 +2576,7 @@ template <class R> struct Fields : FieldsBase {
   long s2_run(long m) {
     const long m0 = m;
     int parity = 0;
+    s2_reserve(m);
     while (m > 0) {
       // 8 steps a launch against 3, 4 and 6: 1.97 / 3.7, 3.0, 2.9 ms for 400 steps of a 320 x 160
       // FP64 cell (the launch and the tile load cost as much as four steps)
@@ -2579,9 +2598,7 @@ template <class R> struct Fields : FieldsBase {
         if (m == 1) break;
         T = (m + 1) / 2;
       }
-      rows_hint = m;
       const double *row = src_row(t);
-      if (row && t + T > rows_t0 + rows_n) fail("internal: source rows shorter than the tile kernel's steps");
       const bool hits = dft && dgroup.hits(t, t + T);
       if (hits && !window_open) window_open = true, window_t = t;
       kbegin(MP_K_STEP_DE);
@@ -2630,10 +2647,6 @@ template <class R> struct Fields : FieldsBase {
       a.rec = static_cast<R *>(A.seg.p) + size_t(A.nrec - seg_first) * A.npts;
     }
     else {
-      if (size_t(A.nrec / HBLK) >= A.hist.size()) {
-        A.hist.emplace_back(new DevBuf);
-        A.hist.back()->alloc(sizeof(R) * A.npts * HBLK);
-      }
       if (A.nrec % HBLK + T > HBLK) fail("internal: recorded steps cross a history block");
       a.rec = static_cast<R *>(A.hist[size_t(A.nrec / HBLK)]->p) + size_t(A.nrec % HBLK) * A.npts;
     }
@@ -2930,6 +2943,7 @@ template <class R> struct Fields : FieldsBase {
       std::vector<std::unique_ptr<DevBuf>> data; // one per state array, in state_arrays() order
     };
     std::vector<Checkpoint> cps;
+    std::vector<std::vector<std::unique_ptr<DevBuf>>> spare; // memory of checkpoints still to be taken
     DevBuf seg; // checkpoint mode: one segment of history
   };
   static constexpr long HBLK = 256;
@@ -3008,17 +3022,39 @@ template <class R> struct Fields : FieldsBase {
     HIPCHECK(hipStreamSynchronize(stream));
     typename Adj::Checkpoint cp;
     cp.t = t;
-    for (const StateArr &a : state_arrays()) {
-      cp.data.emplace_back(new DevBuf);
-      cp.data.back()->alloc(a.esz * gv.ntot);
+    const std::vector<StateArr> arrays = state_arrays();
+    if (!adj->spare.empty() && adj->spare.back().size() == arrays.size()) {
+      cp.data = std::move(adj->spare.back());
+      adj->spare.pop_back();
+    }
+    else {
+      adj->spare.clear(); // reserved before arrays came
+      cp.data = state_copies();
+    }
+    for (size_t q = 0; q < arrays.size(); ++q) {
+      const StateArr &a = arrays[q];
       const void *from = a.p;
       if (second) {
         auto it = s2_alt.find(a.p);
         if (it != s2_alt.end()) from = it->second;
       }
-      HIPCHECK(hipMemcpyAsync(cp.data.back()->p, from, a.esz * gv.ntot, hipMemcpyDeviceToDevice, stream));
+      HIPCHECK(hipMemcpyAsync(cp.data[q]->p, from, a.esz * gv.ntot, hipMemcpyDeviceToDevice, stream));
     }
     adj->cps.push_back(std::move(cp));
+  }
+  // memory for one checkpoint
+  std::vector<std::unique_ptr<DevBuf>> state_copies() const {
+    std::vector<std::unique_ptr<DevBuf>> v;
+    for (const StateArr &a : state_arrays()) {
+      v.emplace_back(new DevBuf);
+      v.back()->alloc(a.esz * gv.ntot);
+    }
+    return v;
+  }
+  void add_history_block() {
+    std::unique_ptr<DevBuf> b(new DevBuf);
+    b->alloc(sizeof(R) * adj->npts * HBLK);
+    adj->hist.push_back(std::move(b));
   }
   // the D at the design points after step (t - t0 - 1) -> history
   void record_design() {
@@ -3034,10 +3070,7 @@ template <class R> struct Fields : FieldsBase {
       dst = static_cast<R *>(A.seg.p) + size_t(n - seg_first) * A.npts;
     }
     else {
-      if (size_t(n / HBLK) >= A.hist.size()) {
-        A.hist.emplace_back(new DevBuf);
-        A.hist.back()->alloc(sizeof(R) * A.npts * HBLK);
-      }
+      if (size_t(n / HBLK) >= A.hist.size()) add_history_block();
       dst = static_cast<R *>(A.hist[n / HBLK]->p) + size_t(n % HBLK) * A.npts;
     }
     const int dc = A.c + 10;

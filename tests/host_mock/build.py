@@ -16,8 +16,9 @@ OUT = os.path.join(HERE, "_build")
 LIB = os.path.join(OUT, "libmeep_host.so")
 
 
-# stubs that check the buffers a launch would write
-CHECKED = {"launch_farfield": ' if (!out || (a.segs > 1 && !partial) || (!a.px && a.npts > 1))'
+# stubs that check the buffers a launch would write, or count launches
+CHECKED = {"launch_step2d": " ++mock_step2d; ",
+           "launch_farfield": ' if (!out || (a.segs > 1 && !partial) || (!a.px && a.npts > 1))'
                               ' throw std::runtime_error("far-field launch without its buffers"); '}
 
 
@@ -29,8 +30,8 @@ def launcher_stubs():
     decls = re.findall(r"template <class R>\s*(void|bool) (launch_\w+)\(([^;]*?)\);", src, re.S)
     if not decls:
         raise RuntimeError("no launcher declarations found in engine.hpp")
-    out = ['#include <stdexcept>', '#include "engine.hpp"', "namespace mx {"]
-    out += [f"template <class R> {ret} {name}({args}) {{{' return false;' if ret == 'bool' else ''}}}"
+    out = ['#include <stdexcept>', '#include "engine.hpp"', "static long mock_step2d = 0;", "namespace mx {"]
+    out += [f"template <class R> {ret} {name}({args}) {{{CHECKED.get(name, ' return false;' if ret == 'bool' else '')}}}"
             for ret, name, args in decls]
     for ret, name, args in decls:
         for real in ("float", "double"):
@@ -45,6 +46,7 @@ def launcher_stubs():
     out.append("}")
     # the allocation that fails next, and the count of allocations (tests of failure handling)
     out.append('extern "C" void mock_fail_malloc(long after) { mock_mallocs_left = after; }')
+    out.append('extern "C" long mock_step2d_launches() { return mock_step2d; }')
     out.append('extern "C" void mock_set_free(size_t n) { mock_free = n; }')
     out.append('extern "C" long mock_malloc_count() { return mock_mallocs; }')
     return "\n".join(out) + "\n"

@@ -16,7 +16,7 @@ def host_lib():
     lib = capi.bind(ctypes.CDLL(build.build()))
     lib.mock_fail_malloc.argtypes = [ctypes.c_long]
     lib.mock_set_free.argtypes = [ctypes.c_size_t]
-    lib.mock_malloc_count.restype = ctypes.c_long
+    lib.mock_malloc_count.restype = lib.mock_step2d_launches.restype = ctypes.c_long
     return lib
 
 
@@ -138,3 +138,30 @@ def test_batch_that_the_tile_kernel_does_not_take(host_lib, monkeypatch, short):
         host_lib.mock_set_free(256 << 30)
     monkeypatch.setenv("MEEP_AMD_NO_TILE2D", "1")
     assert got == run()
+
+
+@pytest.mark.parametrize("interval", [0, 20], ids=["history", "checkpoints"])
+def test_recording_that_runs_out_of_memory(host_lib, interval):
+    """The tile kernel's state is where every reader looks after an even number of launches: an
+    allocation of the reverse mode's recording that fails leaves it there, and the fields go on."""
+    import adjoint_cases as AC
+    for after in range(400):
+        s, f, mon = AC.build(host_lib, AC.rho_grid())
+        adj = capi.adjoint(f, mon, Ez, AC.DESIGN[0], AC.DESIGN[1], checkpoint_interval=interval)
+        f.step_n(9)
+        host_lib.mock_fail_malloc(after)
+        before, launches = host_lib.mock_malloc_count(), host_lib.mock_step2d_launches()
+        failed = False
+        try:
+            f.step_n(700 if interval == 0 else 60)
+        except MeepError as e:
+            assert "internal" not in str(e)
+            failed = True
+        made = host_lib.mock_malloc_count() - before
+        host_lib.mock_fail_malloc(-1)
+        assert (host_lib.mock_step2d_launches() - launches) % 2 == 0, after
+        f.step_n(30)
+        adj.gradient()
+        if made <= after:
+            break
+    assert not failed and after >= 2
