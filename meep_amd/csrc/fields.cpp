@@ -454,6 +454,9 @@ template <class R> struct DftChunk {
   cdouble stored_weight = 1.0;
   bool empty[3] = {};
   int vc = -1; // near2far: the equivalent current's component
+  // 2D: the host's idx and w, from which the tile kernel's monitor tables are made
+  std::vector<uint32_t> h_idx;
+  std::vector<double> h_w;
   cdouble extra_weight = 1.0; // dft_force: the readout's factor (src/dft.cpp:97,224)
   bool sqrt_w = false;        // accumulated with the square root of the integration weight
 };
@@ -2056,6 +2059,7 @@ template <class R> struct Fields : FieldsBase {
   // bumped when a step swaps the P / P_prev pointers (pswap) and when a DFT monitor is added
   // or removed: a batch plan records device pointers and DFT chunk lists, so either makes it stale
   long ptr_version = 0, dft_version = 0;
+  int p_order = 0; // changes with each swap
   void prepare_images(SrcVol &sv) {
     if (sv.img_version == plan_version) return;
     std::vector<int> ks;
@@ -2188,6 +2192,7 @@ template <class R> struct Fields : FieldsBase {
         for (int c = 0; c < 5; ++c)
           for (int cmp = 0; cmp < 2; ++cmp) std::swap(p.P[c][cmp], p.Pp[c][cmp]);
       ++ptr_version;
+      p_order ^= 1;
     }
     if (!plan_valid) rebuild_plan();
     boundaries(1); // D, P_E, E (step_boundaries D_stuff .. E_stuff)
@@ -2211,7 +2216,8 @@ template <class R> struct Fields : FieldsBase {
     for (long q = 0; q < n;) {
       const long tail = probe && !flux_vols.empty() ? 1 : 0;
       rows_hint = n - q;
-      if (n - q - tail >= 2 && (dft_defer_steps || dft_off) && s2_ready(S2_STEPS)) {
+      const bool several = dft_defer_steps || dft_off;
+      if (several && n - q - tail >= 2 && s2_ready(S2_STEPS, n - q - tail) && (dft_off || dft_chunks.empty() || dft_group())) {
         const long did = s2_run(n - q - tail);
         q += did;
         if (did) {
@@ -2220,21 +2226,42 @@ template <class R> struct Fields : FieldsBase {
         }
       }
       one_step(probe && q == n - 1);
+      if (several) ++s2_plan(S2_STEPS).waited;
       ++q;
     }
   }
-  struct S2Set { // one polarisation: its launch arguments by part (real, imaginary) and parity
+  // One polarisation: its launch arguments by part (real, imaginary), order of P and P_prev (as
+  // p_order) and parity.  A step taken alone swaps P and P_prev, so both orders are kept.
+  struct S2Set {
     bool tm;
-    Step2dArgs<R> a[2][2];
-    DevBuf args, mon_first, mon, mons[2]; // args: a, row by row
-    const Step2dArgs<R> *dev(int cmp, int parity) const { return static_cast<const Step2dArgs<R> *>(args.p) + 2 * cmp + parity; }
+    Step2dArgs<R> a[2][2][2];
+    DevBuf args; // a, row by row
+    const Step2dArgs<R> *dev(int cmp, int order, int parity) const {
+      return static_cast<const Step2dArgs<R> *>(args.p) + (2 * cmp + order) * 2 + parity;
+    }
+  };
+  // the monitor tables of one polarisation: tiles' first entries, entries, chunks by part
+  struct S2Monitors {
+    long plan_v = -1, dft_v = -1;
+    int n = 0, mask = 0;
+    size_t entry_at = 0, mons_at[2] = {0, 0};
+    DevBuf buf;
   };
   struct S2Plan {
-    long plan_v = -1, dft_v = -1, src_v = -1, ptr_v = -1, builds = 0;
+    long plan_v = -1, dft_v = -1, src_v = -1, pool_v = -1, builds = 0;
     int margin = 0; // steps a tile has room for
+    // steps taken one by one, in calls of several, while the plan was not built
+    long waited = 0;
     bool shape = false, ok = false;
     std::vector<std::unique_ptr<S2Set>> sets;
-  } s2;
+    S2Monitors mons[2];
+  } s2[2]; // for a chunk stepped alone and in a batch
+  S2Plan &s2_plan(int margin) {
+    S2Plan &p = s2[margin == S2_STEPS ? 0 : 1];
+    p.margin = margin;
+    return p;
+  }
+  long pool_version = 0; // changes with the second buffers
   // each state array's second buffer, in one allocation
   DevBuf s2_pool;
   std::map<const void *, char *> s2_alt;
@@ -2243,16 +2270,15 @@ template <class R> struct Fields : FieldsBase {
   // halos, no conductivity, no magnetic poles and at most S2_POLES electric ones, every source in
   // a table or box, every DFT chunk of the deferred form, and no state array left to allocate.
   bool s2_shape(int margin) {
+    S2Plan &s2 = s2_plan(margin);
     if (s2_off || gv.dim != 2 || !use_fast || whole_rows_env >= 0) return false;
     if (!plan_valid || srcplan_stale() || t > INT32_MAX / 2) return false;
-    if (s2.plan_v == plan_version && s2.dft_v == dft_version && s2.src_v == src_version && s2.ptr_v == ptr_version && s2.margin == margin)
-      return s2.shape;
-    s2.margin = margin;
+    if (s2.plan_v == plan_version && s2.dft_v == dft_version && s2.src_v == src_version) return s2.shape;
     ++s2.builds;
+    if (s2.plan_v != plan_version || s2.dft_v != dft_version) s2.waited = 0;
     s2.plan_v = plan_version;
     s2.dft_v = dft_version;
     s2.src_v = src_version;
-    s2.ptr_v = ptr_version;
     s2.shape = s2.ok = false;
     s2.sets.clear();
     if (any_cond || n_conn[0] || n_conn[1] || wrap_dir[0] || wrap_dir[1] || have_fmp_H() || int(pols.size()) > S2_POLES) return false;
@@ -2282,36 +2308,65 @@ template <class R> struct Fields : FieldsBase {
       int have = 0;
       for (int d = 0; d < 3; ++d) have += f[dir_comp(tm == (d == 2) ? 10 : 15, d)][0] != nullptr;
       if (!have) continue;
-      if (have != 3 || !s2_set(tm, fmp)) return false;
+      if (have != 3 || !s2_set(s2, tm, fmp)) return false;
     }
     return s2.shape = !s2.sets.empty();
   }
-  // ... and its second buffers and tables are in place.  Where memory for them is short the chunk
-  // keeps stepping one by one.
-  bool s2_ready(int margin) {
+  // Steps that a chunk takes one by one, in calls of several, before the second buffers and monitor
+  // tables of its plan are made: about their cost, in steps that the tile kernel then saves.  A
+  // first call of 9 steps of a 320 x 160 FP64 cell with a flux line takes 0.85 ms either way; with
+  // 105 k monitor points (401 x 263 FP32) a first call of 40 steps 1.7 ms with tiles, 2.5 ms
+  // without, of 9 steps 1.5 to 2.2 and 0.9 ms.  Sources may change without this: their plan is
+  // arguments alone.
+  long s2_worth() const {
+    size_t pts = 0;
+    for (auto &cp : dft_chunks) pts += size_t(cp->npts);
+    return S2_WORTH + long(pts / S2_WORTH_POINTS);
+  }
+  static constexpr long S2_WORTH = 8, S2_WORTH_POINTS = 4096;
+  // whether the buffers and monitor tables of the plan are still to be made
+  bool s2_unbuilt(int margin) {
+    const S2Plan &s2 = s2_plan(margin);
+    for (const S2Monitors &m : s2.mons)
+      if (m.plan_v == plan_version && m.dft_v == dft_version) return false;
+    return true;
+  }
+  // ... and, for a call of n steps, its second buffers and tables are in place.  Where memory for
+  // them is short the chunk keeps stepping one by one.
+  bool s2_ready(int margin, long n) {
     if (!s2_shape(margin)) return false;
-    if (s2.ok) return true;
+    S2Plan &s2 = s2_plan(margin);
+    if (s2.ok && s2.pool_v == pool_version) return true;
+    if (s2_unbuilt(margin) && s2.waited + n < s2_worth()) return false;
     try {
-      s2.ok = s2_second() && (dft_chunks.empty() || dft_group());
+      s2.ok = s2_second(s2);
+      for (auto &cp : dft_chunks)
+        if (s2.ok) batch_dft(*cp); // the ring of deferred values
       for (auto &S : s2.sets)
-        if (s2.ok) s2_finish(*S);
+        if (s2.ok) s2_finish(s2, *S);
     } catch (const OutOfMemory &) {
       s2.ok = false;
     }
+    ++s2.builds;
+    s2.pool_v = pool_version;
     if (!s2.ok) {
       s2_drop();
       s2_off = true;
     }
     return s2.ok;
   }
-  // the second buffers and the plan given back
+  // the second buffers and the plans given back
   void s2_drop() {
     HIPCHECK(hipStreamSynchronize(stream));
-    s2.plan_v = -1;
-    s2.shape = s2.ok = false;
-    s2.sets.clear();
+    for (S2Plan &p : s2) {
+      p.plan_v = -1;
+      p.shape = p.ok = false;
+      p.sets.clear();
+      for (S2Monitors &m : p.mons) m.plan_v = -1, m.buf.alloc(0);
+    }
     s2_alt.clear();
     s2_pool.alloc(0);
+    ++pool_version;
   }
   // The arrays of a set's arguments and the second pointers beside them, as (array, second
   // pointer, bytes of an element).
@@ -2327,12 +2382,12 @@ template <class R> struct Fields : FieldsBase {
   // Second buffers of every array of the plan, copies of the arrays; false where they would not
   // fit, or would leave less than half of the device's memory free: a chunk so large is no
   // longer bound by launches, and what its owner allocates later has to fit as it did without them.
-  bool s2_second() {
+  bool s2_second(S2Plan &s2) {
     std::vector<std::pair<const void *, size_t>> need;
     bool have = true;
     for (auto &S : s2.sets)
       for (int cmp = 0; cmp < ncmp(); ++cmp)
-        s2_pairs(S->a[cmp][0], [&](auto *in, auto *) {
+        s2_pairs(S->a[cmp][0][0], [&](auto *in, auto *) {
           if (!in) return;
           need.push_back({in, sizeof(*in) * gv.ntot});
           have = have && s2_alt.count(in);
@@ -2343,6 +2398,7 @@ template <class R> struct Fields : FieldsBase {
       HIPCHECK(hipStreamSynchronize(stream));
       s2_alt.clear();
       s2_pool.alloc(0);
+      ++pool_version;
       HIPCHECK(hipMemGetInfo(&free, &all));
       if (free < total || free - total < all / 2) return false;
       s2_pool.alloc(total);
@@ -2355,14 +2411,14 @@ template <class R> struct Fields : FieldsBase {
     }
     for (auto &S : s2.sets)
       for (int cmp = 0; cmp < ncmp(); ++cmp)
-        s2_pairs(S->a[cmp][0], [&](auto *in, auto *&out) {
+        s2_pairs(S->a[cmp][0][0], [&](auto *in, auto *&out) {
           if (in) out = reinterpret_cast<std::remove_reference_t<decltype(out)>>(s2_alt.at(in));
         });
     return true;
   }
   // the launch arguments of one polarisation, second pointers apart; false when its plan has
   // another shape than the kernel's
-  bool s2_set(bool tm, bool fmp) {
+  bool s2_set(S2Plan &s2, bool tm, bool fmp) {
     std::unique_ptr<S2Set> S(new S2Set);
     S->tm = tm;
     const int margin = s2.margin;
@@ -2382,7 +2438,7 @@ template <class R> struct Fields : FieldsBase {
       AB.src = AD.src = nullptr;
       check_args(AB, true, true, true);
       check_args(AD, true, true, true);
-      Step2dArgs<R> &a = S->a[cmp][0];
+      Step2dArgs<R> &a = S->a[cmp][0][0];
       memset(&a, 0, sizeof a);
       const Grid &g = AD.g;
       a.nx = gv.num[0];
@@ -2439,8 +2495,8 @@ template <class R> struct Fields : FieldsBase {
         if (!mag && u.f)
           for (int p = 0; p < a.npole; ++p) {
             if (!u.P[p]) continue;
-            c.P[p] = u.P[p];
-            c.Pp[p] = u.Pp[p];
+            c.P[p] = p_order ? u.Pp[p] : u.P[p]; // of order 0
+            c.Pp[p] = p_order ? u.P[p] : u.Pp[p];
             c.sigma[p] = u.sigma[p];
             c.sigval[p] = u.sigval[p];
             if ((u.sigone >> p) & 1) c.sigone |= 1 << p;
@@ -2452,21 +2508,29 @@ template <class R> struct Fields : FieldsBase {
     s2.sets.push_back(std::move(S));
     return true;
   }
-  // a set's monitor tables, its arguments for the other parity (every pair exchanged), and the upload
-  void s2_finish(S2Set &S) {
-    s2_monitors(S);
+  // a set's monitor tables, its arguments for the other order of P and P_prev and for the other
+  // parity (every pair of buffers exchanged), and the upload
+  void s2_finish(S2Plan &s2, S2Set &S) {
+    s2_monitors(s2.mons[S.tm ? 1 : 0], S);
     std::vector<Step2dArgs<R>> all;
     for (int cmp = 0; cmp < 2; ++cmp) {
       if (cmp < ncmp()) {
-        s2_check(S.a[cmp][0]);
-        S.a[cmp][1] = S.a[cmp][0];
-        s2_pairs(S.a[cmp][1], [](auto *&in, auto *&out) {
-          auto *o = out;
-          out = const_cast<std::remove_const_t<std::remove_pointer_t<std::remove_reference_t<decltype(in)>>> *>(in);
-          in = o;
-        });
+        s2_check(S.a[cmp][0][0]);
+        S.a[cmp][1][0] = S.a[cmp][0][0];
+        for (S2Comp<R> &c : S.a[cmp][1][0].c)
+          for (int p = 0; p < S2_POLES; ++p) std::swap(c.P[p], c.Pp[p]), std::swap(c.Po[p], c.Ppo[p]);
       }
-      for (int par = 0; par < 2; ++par) all.push_back(S.a[cmp][par]);
+      for (int order = 0; order < 2; ++order) {
+        if (cmp < ncmp()) {
+          S.a[cmp][order][1] = S.a[cmp][order][0];
+          s2_pairs(S.a[cmp][order][1], [](auto *&in, auto *&out) {
+            auto *o = out;
+            out = const_cast<std::remove_const_t<std::remove_pointer_t<std::remove_reference_t<decltype(in)>>> *>(in);
+            in = o;
+          });
+        }
+        for (int par = 0; par < 2; ++par) all.push_back(S.a[cmp][order][par]);
+      }
     }
     upload_vec(S.args, all);
   }
@@ -2483,71 +2547,97 @@ template <class R> struct Fields : FieldsBase {
     if (a.sig[1]) ok = ok && a.c[2].fu && a.c[2].fuo && a.c[1].fw && a.c[1].fwo && a.c[1].e;
     if (!ok) fail("internal: bad 2D tile plan");
   }
-  // the monitor points of each tile
-  void s2_monitors(S2Set &S) {
-    Step2dArgs<R> &a = S.a[0][0];
-    const size_t nt = size_t(a.ntx) * size_t(a.nty);
-    std::vector<std::vector<S2Entry>> lists(nt);
-    std::vector<S2Mon<R>> mons[2];
-    int mask = 0;
-    for (auto &cp : dft_chunks) {
-      DftChunk<R> &ch = *cp;
-      const int d = comp_dir(ch.c);
-      const bool mag = is_magnetic(ch.c) || is_B(ch.c);
-      if ((S.tm != (d == 2)) != mag) continue; // of the other polarisation
-      S2Mon<R> m;
-      memset(&m, 0, sizeof m);
-      m.npts = uint32_t(ch.npts);
-      m.fld = d + (is_D(ch.c) || is_B(ch.c) ? 3 : 0);
-      m.dec = ch.decimation;
-      auto off = [&](int64_t o) {
-        if (o != 0 && o != 1 && o != gv.st[0]) fail("internal: DFT centring offset");
-        return o == 0 ? 0 : o == 1 ? 1 : S2_COLS;
-      };
-      m.o1 = off(ch.avg1);
-      m.o2 = off(ch.avg2);
-      mask |= 1 << m.fld;
-      const size_t ci = mons[0].size();
-      m.snap = static_cast<R *>(ch.snap.p);
-      mons[0].push_back(m);
-      m.snap += size_t(DFT_DEFER) * size_t(ch.npts);
-      mons[1].push_back(m);
-      std::vector<int64_t> idx(size_t(ch.npts));
-      std::vector<double> w(size_t(ch.npts));
-      HIPCHECK(hipMemcpy(idx.data(), ch.idx.p, sizeof(int64_t) * idx.size(), hipMemcpyDeviceToHost));
-      HIPCHECK(hipMemcpy(w.data(), ch.w.p, sizeof(double) * w.size(), hipMemcpyDeviceToHost));
-      for (size_t k = 0; k < idx.size(); ++k) {
-        const int x = int(idx[k] / gv.st[0]), y = int(idx[k] % gv.st[0]);
-        if (x < 0 || x > a.nx || y < 0 || y > a.ny) fail("internal: DFT point outside the grid");
-        const int tx = x / a.cx, ty = y / a.cy;
-        const int lx = x - tx * a.cx + a.margin, ly = y - ty * a.cy + a.margin;
-        if (tx >= a.ntx || ty >= a.nty || lx + 1 >= S2_ROWS || ly + 1 >= S2_COLS) fail("internal: DFT point outside its tile");
-        S2Entry e;
-        memset(&e, 0, sizeof e);
-        e.w = w[k];
-        e.k = uint32_t(k);
-        e.pos = uint16_t(lx * S2_COLS + ly);
-        e.chunk = uint16_t(ci);
-        lists[size_t(tx) * size_t(a.nty) + size_t(ty)].push_back(e);
+  // the monitor points of each tile, made anew where monitors or arrays have changed
+  void s2_monitors(S2Monitors &M, S2Set &S) {
+    if (M.plan_v != plan_version || M.dft_v != dft_version) {
+      M.dft_v = -1;
+      const Step2dArgs<R> &a = S.a[0][0][0];
+      const size_t nt = size_t(a.ntx) * size_t(a.nty);
+      std::vector<S2Mon<R>> mons[2];
+      std::vector<const DftChunk<R> *> chunks;
+      M.mask = 0;
+      size_t total = 0;
+      for (auto &cp : dft_chunks) {
+        DftChunk<R> &ch = *cp;
+        const int d = comp_dir(ch.c);
+        const bool mag = is_magnetic(ch.c) || is_B(ch.c);
+        if ((S.tm != (d == 2)) != mag) continue; // of the other polarisation
+        S2Mon<R> m;
+        memset(&m, 0, sizeof m);
+        m.npts = uint32_t(ch.npts);
+        m.fld = d + (is_D(ch.c) || is_B(ch.c) ? 3 : 0);
+        m.dec = ch.decimation;
+        auto off = [&](int64_t o) {
+          if (o != 0 && o != 1 && o != gv.st[0]) fail("internal: DFT centring offset");
+          return o == 0 ? 0 : o == 1 ? 1 : S2_COLS;
+        };
+        m.o1 = off(ch.avg1);
+        m.o2 = off(ch.avg2);
+        M.mask |= 1 << m.fld;
+        m.snap = static_cast<R *>(ch.snap.p);
+        mons[0].push_back(m);
+        m.snap += size_t(DFT_DEFER) * size_t(ch.npts);
+        mons[1].push_back(m);
+        chunks.push_back(&ch);
+        total += ch.h_idx.size();
+        if (ch.h_idx.size() != size_t(ch.npts) || ch.h_w.size() != size_t(ch.npts)) fail("internal: DFT points not kept");
       }
+      M.n = int(chunks.size());
+      if (total >= (size_t(1) << 32)) fail("internal: too many DFT points for the tile kernel");
+      // entries by tile, in chunk and point order: the tiles' counts, their first entries, the entries
+      std::vector<uint32_t> tile(total), first(nt + 1, 0);
+      std::vector<uint16_t> pos(total);
+      size_t q = 0;
+      for (const DftChunk<R> *ch : chunks) {
+        const uint32_t st = uint32_t(gv.st[0]);
+        uint32_t x = 0, y = 0, last = UINT32_MAX - 1;
+        for (uint32_t i : ch->h_idx) {
+          if (i == last + 1 && y + 1 < st)
+            ++y;
+          else
+            x = i / st, y = i - x * st;
+          last = i;
+          if (int(x) > a.nx || int(y) > a.ny) fail("internal: DFT point outside the grid");
+          const int tx = int(x) / a.cx, ty = int(y) / a.cy;
+          const int lx = int(x) - tx * a.cx + a.margin, ly = int(y) - ty * a.cy + a.margin;
+          if (tx >= a.ntx || ty >= a.nty || lx + 1 >= S2_ROWS || ly + 1 >= S2_COLS) fail("internal: DFT point outside its tile");
+          tile[q] = uint32_t(tx * a.nty + ty);
+          pos[q] = uint16_t(lx * S2_COLS + ly);
+          ++first[tile[q] + 1];
+          ++q;
+        }
+      }
+      for (size_t k = 0; k < nt; ++k) first[k + 1] += first[k];
+      auto up = [](size_t n) { return (n + 255) / 256 * 256; };
+      M.entry_at = up(sizeof(uint32_t) * first.size());
+      M.mons_at[0] = M.entry_at + up(sizeof(S2Entry) * total);
+      M.mons_at[1] = M.mons_at[0] + up(sizeof(S2Mon<R>) * chunks.size());
+      std::vector<char> host(M.mons_at[1] + up(sizeof(S2Mon<R>) * chunks.size()));
+      memcpy(host.data(), first.data(), sizeof(uint32_t) * first.size());
+      S2Entry *entry = reinterpret_cast<S2Entry *>(host.data() + M.entry_at);
+      q = 0;
+      for (size_t ci = 0; ci < chunks.size(); ++ci)
+        for (size_t k = 0; k < chunks[ci]->h_idx.size(); ++k, ++q) {
+          S2Entry &e = entry[first[tile[q]]++];
+          e.w = chunks[ci]->h_w[k];
+          e.k = uint32_t(k);
+          e.pos = pos[q];
+          e.chunk = uint16_t(ci);
+        }
+      for (int cmp = 0; cmp < 2; ++cmp)
+        if (M.n) memcpy(host.data() + M.mons_at[cmp], mons[cmp].data(), sizeof(S2Mon<R>) * chunks.size());
+      if (M.n) upload_vec(M.buf, host);
+      M.plan_v = plan_version;
+      M.dft_v = dft_version;
     }
-    if (mons[0].empty()) return;
-    std::vector<uint32_t> first(1, 0);
-    std::vector<S2Entry> all;
-    for (auto &l : lists) {
-      all.insert(all.end(), l.begin(), l.end());
-      first.push_back(uint32_t(all.size()));
-    }
-    upload_vec(S.mon_first, first);
-    upload_vec(S.mon, all);
-    for (int cmp = 0; cmp < ncmp(); ++cmp) {
-      upload_vec(S.mons[cmp], mons[cmp]);
-      Step2dArgs<R> &b = S.a[cmp][0];
-      b.mon_first = static_cast<const uint32_t *>(S.mon_first.p);
-      b.mon = static_cast<const S2Entry *>(S.mon.p);
-      b.mons = static_cast<const S2Mon<R> *>(S.mons[cmp].p);
-      b.monmask = mask;
-      b.nmon = int(mons[cmp].size());
+    for (int cmp = 0; cmp < ncmp() && M.n; ++cmp) {
+      Step2dArgs<R> &b = S.a[cmp][0][0];
+      const char *base = static_cast<const char *>(M.buf.p);
+      b.mon_first = reinterpret_cast<const uint32_t *>(base);
+      b.mon = reinterpret_cast<const S2Entry *>(base + M.entry_at);
+      b.mons = reinterpret_cast<const S2Mon<R> *>(base + M.mons_at[cmp]);
+      b.monmask = M.mask;
+      b.nmon = M.n;
     }
   }
   // Everything that the next m steps allocate, before the first of them: an allocation that failed
@@ -2576,11 +2666,12 @@ template <class R> struct Fields : FieldsBase {
   long s2_run(long m) {
     const long m0 = m;
     int parity = 0;
+    const S2Plan &plan = s2_plan(S2_STEPS);
     s2_reserve(m);
     while (m > 0) {
       // 8 steps a launch against 3, 4 and 6: 1.97 / 3.7, 3.0, 2.9 ms for 400 steps of a 320 x 160
       // FP64 cell (the launch and the tile load cost as much as four steps)
-      long T = std::min<long>(m, s2.margin);
+      long T = std::min<long>(m, plan.margin);
       const bool rec = adj && adj->recording;
       if (rec) {
         Adj &A = *adj;
@@ -2602,12 +2693,12 @@ template <class R> struct Fields : FieldsBase {
       const bool hits = dft && dgroup.hits(t, t + T);
       if (hits && !window_open) window_open = true, window_t = t;
       kbegin(MP_K_STEP_DE);
-      for (auto &S : s2.sets)
+      for (auto &S : plan.sets)
         for (int cmp = 0; cmp < ncmp(); ++cmp) {
-          const Step2dArgs<R> &a = S->a[cmp][parity];
+          const Step2dArgs<R> &a = S->a[cmp][p_order][parity];
           Step2dLaunch<R> l;
           memset(&l, 0, sizeof l);
-          l.items = S->dev(cmp, parity);
+          l.items = S->dev(cmp, p_order, parity);
           l.ntile = uint32_t(a.ntx) * uint32_t(a.nty);
           l.nsteps = int(T);
           l.vrow = row;
@@ -4064,6 +4155,10 @@ template <class R> struct Fields : FieldsBase {
       HIPCHECK(hipMemcpy(ch->idx.p, idx.data(), sizeof(int64_t) * idx.size(), hipMemcpyHostToDevice));
       HIPCHECK(hipMemcpy(ch->w.p, w.data(), sizeof(double) * w.size(), hipMemcpyHostToDevice));
       HIPCHECK(hipMemcpy(ch->omega.p, om.data(), sizeof(double) * om.size(), hipMemcpyHostToDevice));
+      if (gv.dim == 2) {
+        ch->h_idx.assign(idx.begin(), idx.end());
+        ch->h_w = std::move(w);
+      }
       ch->acc_kind = dft_acc;
       ch->defer = ch->nfreq * DFT_DEFER <= DFT_FLUSH_TAB ? DFT_DEFER : 1;
       const size_t nacc = size_t(ch->npts) * ch->nfreq;
@@ -5002,22 +5097,38 @@ template <class R> struct Batch : BatchBase {
   struct TileGroup {
     bool tm;
     int npole, monmask = 0;
-    std::vector<Step2dArgs<R>> host[2]; // by parity
-    std::vector<size_t> sim;
-    DevBuf items[2], blk_item, blk_tile;
+    struct Item { // one part of one polarisation of member sim
+      const typename Fields<R>::S2Set *set;
+      int cmp;
+      size_t sim;
+    };
+    std::vector<Item> items;
+    size_t at[2]; // first row of the items in tile_args, by parity
+    DevBuf blk_item, blk_tile;
     uint32_t ntile = 0;
   };
   std::vector<std::unique_ptr<TileGroup>> tgroups;
+  std::vector<Step2dArgs<R>> tile_host;
+  DevBuf tile_args;
   std::vector<long> tile_builds;
   std::vector<int> tile_decs;
-  bool tiles_ready() {
-    bool fresh = tile_builds.size() == sims.size();
+  // Steps that a batch takes one by one, over its calls, before it makes the members' second
+  // buffers and tables: 10 ms for 64 members of 128 to 512 cells, 0.12 ms saved a step; 0.6 ms for 8
+  // members of 60 to 160 cells, 0.05 ms saved a step
+  static constexpr long S2_BATCH_WORTH = 64;
+  long tile_waited = 0;
+  bool tiles_ready(long m) {
     // every member's shape before any member allocates: second buffers are of no use to a batch
     // that the kernel does not take whole
-    bool ready = true;
+    bool ready = true, wait = false;
     for (Fields<R> *F : sims) ready = ready && F->s2_shape(S2_BATCH);
+    for (Fields<R> *F : sims) wait = wait || (ready && F->s2_unbuilt(S2_BATCH));
+    if (wait && tile_waited + m < S2_BATCH_WORTH) {
+      tile_waited += m;
+      return false;
+    }
     if (ready) {
-      for (Fields<R> *F : sims) ready = ready && F->s2_ready(S2_BATCH);
+      for (Fields<R> *F : sims) ready = ready && F->s2_ready(S2_BATCH, S2_BATCH_WORTH + F->s2_worth());
       if (!ready) // memory is short
         for (Fields<R> *F : sims) F->s2_drop();
     }
@@ -5026,7 +5137,9 @@ template <class R> struct Batch : BatchBase {
       tgroups.clear();
       return false;
     }
-    for (size_t q = 0; q < sims.size() && fresh; ++q) fresh = tile_builds[q] == sims[q]->s2.builds;
+    tile_waited = 0;
+    bool fresh = tile_builds.size() == sims.size();
+    for (size_t q = 0; q < sims.size() && fresh; ++q) fresh = tile_builds[q] == sims[q]->s2_plan(S2_BATCH).builds;
     if (fresh) return true;
     tgroups.clear();
     tile_builds.clear();
@@ -5034,34 +5147,33 @@ template <class R> struct Batch : BatchBase {
     std::map<int, TileGroup *> by;
     for (size_t q = 0; q < sims.size(); ++q) {
       Fields<R> *F = sims[q];
-      tile_builds.push_back(F->s2.builds);
+      tile_builds.push_back(F->s2_plan(S2_BATCH).builds);
       for (int d : F->dft_chunks.empty() ? std::vector<int>() : F->dgroup.decs)
         if (std::find(tile_decs.begin(), tile_decs.end(), d) == tile_decs.end()) tile_decs.push_back(d);
-      for (auto &S : F->s2.sets)
+      for (auto &S : F->s2_plan(S2_BATCH).sets)
         for (int cmp = 0; cmp < F->ncmp(); ++cmp) {
-          const int key = 2 * S->a[cmp][0].npole + (S->tm ? 1 : 0);
+          const Step2dArgs<R> &a = S->a[cmp][0][0];
+          const int key = 2 * a.npole + (S->tm ? 1 : 0);
           TileGroup *&g = by[key];
           if (!g) {
             tgroups.emplace_back(g = new TileGroup);
             g->tm = S->tm;
-            g->npole = S->a[cmp][0].npole;
+            g->npole = a.npole;
           }
-          for (int par = 0; par < 2; ++par) {
-            g->host[par].push_back(S->a[cmp][par]);
-            g->host[par].back().vofs = int64_t(row_off[q]);
-          }
-          g->sim.push_back(q);
-          g->monmask |= S->a[cmp][0].monmask;
+          g->items.push_back({S.get(), cmp, q});
+          g->monmask |= a.monmask;
         }
       HIPCHECK(hipStreamSynchronize(F->stream)); // the second buffers are copies made there
     }
     for (auto &g : tgroups) {
       std::vector<uint32_t> item, tile;
-      for (size_t k = 0; k < g->host[0].size(); ++k)
-        for (uint32_t b = 0; b < uint32_t(g->host[0][k].ntx) * uint32_t(g->host[0][k].nty); ++b) {
+      for (size_t k = 0; k < g->items.size(); ++k) {
+        const Step2dArgs<R> &a = g->items[k].set->a[g->items[k].cmp][0][0];
+        for (uint32_t b = 0; b < uint32_t(a.ntx) * uint32_t(a.nty); ++b) {
           item.push_back(uint32_t(k));
           tile.push_back(b);
         }
+      }
       g->ntile = uint32_t(item.size());
       upload_vec(g->blk_item, item);
       upload_vec(g->blk_tile, tile);
@@ -5076,11 +5188,20 @@ template <class R> struct Batch : BatchBase {
   }
   // the m >= 2 steps of a call, an even number of launches (the state ends in its own buffers)
   void run_tiles(long m, const double *vrow, int64_t stride) {
+    tile_host.clear();
     for (auto &g : tgroups)
       for (int par = 0; par < 2; ++par) {
-        for (size_t k = 0; k < g->sim.size(); ++k) g->host[par][k].t0 = sims[g->sim[k]]->t;
-        upload_vec(g->items[par], g->host[par]);
+        g->at[par] = tile_host.size();
+        for (const auto &it : g->items) {
+          const Fields<R> *F = sims[it.sim];
+          tile_host.push_back(it.set->a[it.cmp][F->p_order][par]);
+          tile_host.back().vofs = int64_t(row_off[it.sim]);
+          tile_host.back().t0 = F->t;
+        }
       }
+    const size_t bytes = sizeof(Step2dArgs<R>) * tile_host.size();
+    if (tile_args.bytes != bytes) tile_args.alloc(bytes);
+    HIPCHECK(hipMemcpy(tile_args.p, tile_host.data(), bytes, hipMemcpyHostToDevice));
     long nl = (m + S2_BATCH - 1) / S2_BATCH;
     nl += nl & 1;
     long s = 0, w = 0;
@@ -5099,7 +5220,7 @@ template <class R> struct Batch : BatchBase {
       for (auto &g : tgroups) {
         Step2dLaunch<R> l;
         memset(&l, 0, sizeof l);
-        l.items = static_cast<const Step2dArgs<R> *>(g->items[q & 1].p);
+        l.items = static_cast<const Step2dArgs<R> *>(tile_args.p) + g->at[q & 1];
         l.blk_item = static_cast<const uint32_t *>(g->blk_item.p);
         l.blk_tile = static_cast<const uint32_t *>(g->blk_tile.p);
         l.ntile = g->ntile;
@@ -5168,7 +5289,7 @@ template <class R> struct Batch : BatchBase {
     }
     const double *drows = static_cast<const double *>(rows.p);
     call_steps = m;
-    if (m >= 2 && (dft_host.empty() || dft_defer) && tiles_ready()) {
+    if (m >= 2 && (dft_host.empty() || dft_defer) && tiles_ready(m)) {
       auto t0 = std::chrono::steady_clock::now();
       run_tiles(m, drows, int64_t(rl));
       finish(m, t0);
