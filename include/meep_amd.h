@@ -242,11 +242,13 @@ int mp_fields_get_times(mp_fields *f, double *times7);
    counterpart in the reference; feeds the time sinks above and bench.py's roofline).
    which: MP_K_STEP_BH (curl B + H update: every launch of the phase), MP_K_STEP_DE (curl D +
    E/P update: every launch of the phase), MP_K_HALO, MP_K_DFT, MP_K_SRC, and the interior-box
-   launch alone of each phase, MP_K_BH_INTERIOR and MP_K_DE_INTERIOR, and the near-to-far field
-   sums, MP_K_FARFIELD.  Times accumulate in
+   launch alone of each phase, MP_K_BH_INTERIOR and MP_K_DE_INTERIOR (while timing is on it is
+   always a launch of its own), the near-to-far field sums, MP_K_FARFIELD, and the launches that
+   take several whole steps of a 2D chunk, MP_K_TILE2D (both phases: in none of the classes above,
+   and half in each of the sinks 0 and 2).  Times accumulate in
    milliseconds until mp_fields_reset_kernel_timing. */
 enum { MP_K_STEP_BH = 0, MP_K_STEP_DE = 1, MP_K_HALO = 2, MP_K_DFT = 3, MP_K_SRC = 4, MP_K_BH_INTERIOR = 5,
-       MP_K_DE_INTERIOR = 6, MP_K_FARFIELD = 7 };
+       MP_K_DE_INTERIOR = 6, MP_K_FARFIELD = 7, MP_K_TILE2D = 8 };
 int mp_fields_set_kernel_timing(mp_fields *f, int on);
 int mp_fields_get_kernel_timing(mp_fields *f, int which, double *total_ms, long *launches);
 int mp_fields_reset_kernel_timing(mp_fields *f);

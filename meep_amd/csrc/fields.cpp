@@ -576,9 +576,9 @@ template <class R> struct Fields : FieldsBase {
     hipEvent_t a, b;
   };
   std::vector<Pending> pending;
-  static constexpr int NKIND = 8; // the MP_K_* classes
-  double k_ms[NKIND] = {0, 0, 0, 0, 0, 0, 0, 0};
-  long k_n[NKIND] = {0, 0, 0, 0, 0, 0, 0, 0};
+  static constexpr int NKIND = 9; // the MP_K_* classes
+  double k_ms[NKIND] = {};
+  long k_n[NKIND] = {};
   int open_kind = -1;
   hipEvent_t open_ev = nullptr;
   hipEvent_t get_event() {
@@ -1385,21 +1385,20 @@ template <class R> struct Fields : FieldsBase {
       // fetched just before (forward differences prefetch their neighbour naturally)
       b.rev = fast && kind == MP_K_STEP_DE ? 1 : 0;
       set_box(b, interior.lo, interior.hi, curl, upd, fast);
-      // the interior launch alone is timed too (the class of the phase's largest kernel)
+      // the interior launch alone is timed too (the class of the phase's largest kernel): while
+      // timing is on it does not join the slabs' launch
       hipEvent_t e0 = nullptr;
       if (ktiming) {
         e0 = get_event();
         HIPCHECK(hipEventRecord(e0, stream));
       }
-      bool done = fast && launch_row3<R>(b, curl, upd, stream);
-      if (!done && !slabs.empty() && (!fast || rows_pml))
-        rest.insert(rest.begin(), interior);
-      else if (!done) {
-        launch_box(b, interior.lo, interior.hi, curl, upd, fast, rows_pml);
-        done = true;
+      if (!(fast && launch_row3<R>(b, curl, upd, stream))) {
+        if (!ktiming && !slabs.empty() && (!fast || rows_pml))
+          rest.insert(rest.begin(), interior);
+        else
+          launch_box(b, interior.lo, interior.hi, curl, upd, fast, rows_pml);
       }
       if (ktiming) {
-        if (!done) launch_box_list(b, rest, curl, upd, fast, true), rest.clear();
         hipEvent_t e1 = get_event();
         HIPCHECK(hipEventRecord(e1, stream));
         pending.push_back({kind == MP_K_STEP_BH ? MP_K_BH_INTERIOR : MP_K_DE_INTERIOR, e0, e1});
@@ -2692,7 +2691,7 @@ template <class R> struct Fields : FieldsBase {
       const double *row = src_row(t);
       const bool hits = dft && dgroup.hits(t, t + T);
       if (hits && !window_open) window_open = true, window_t = t;
-      kbegin(MP_K_STEP_DE);
+      kbegin(MP_K_TILE2D);
       for (auto &S : plan.sets)
         for (int cmp = 0; cmp < ncmp(); ++cmp) {
           const Step2dArgs<R> &a = S->a[cmp][p_order][parity];
@@ -3521,8 +3520,8 @@ template <class R> struct Fields : FieldsBase {
     timers[6] += std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
     if (ktiming) {
       resolve_events();
-      timers[0] = k_ms[MP_K_STEP_BH] * 1e-3;
-      timers[2] = k_ms[MP_K_STEP_DE] * 1e-3;
+      timers[0] = (k_ms[MP_K_STEP_BH] + 0.5 * k_ms[MP_K_TILE2D]) * 1e-3;
+      timers[2] = (k_ms[MP_K_STEP_DE] + 0.5 * k_ms[MP_K_TILE2D]) * 1e-3;
       timers[4] = k_ms[MP_K_HALO] * 1e-3;
       timers[5] = k_ms[MP_K_DFT] * 1e-3;
     }

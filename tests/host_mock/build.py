@@ -17,7 +17,7 @@ LIB = os.path.join(OUT, "libmeep_host.so")
 
 
 # stubs that check the buffers a launch would write, or count launches
-CHECKED = {"launch_step2d": " ++mock_step2d; ",
+CHECKED = {"launch_step2d": " ++mock_step2d; ", "launch_fast": " ++mock_fast; ",
            "launch_farfield": ' if (!out || (a.segs > 1 && !partial) || (!a.px && a.npts > 1))'
                               ' throw std::runtime_error("far-field launch without its buffers"); '}
 
@@ -30,7 +30,7 @@ def launcher_stubs():
     decls = re.findall(r"template <class R>\s*(void|bool) (launch_\w+)\(([^;]*?)\);", src, re.S)
     if not decls:
         raise RuntimeError("no launcher declarations found in engine.hpp")
-    out = ['#include <stdexcept>', '#include "engine.hpp"', "static long mock_step2d = 0;", "namespace mx {"]
+    out = ['#include <stdexcept>', '#include "engine.hpp"', "static long mock_step2d = 0, mock_fast = 0;", "namespace mx {"]
     out += [f"template <class R> {ret} {name}({args}) {{{CHECKED.get(name, ' return false;' if ret == 'bool' else '')}}}"
             for ret, name, args in decls]
     for ret, name, args in decls:
@@ -47,6 +47,7 @@ def launcher_stubs():
     # the allocation that fails next, and the count of allocations (tests of failure handling)
     out.append('extern "C" void mock_fail_malloc(long after) { mock_mallocs_left = after; }')
     out.append('extern "C" long mock_step2d_launches() { return mock_step2d; }')
+    out.append('extern "C" long mock_fast_launches() { return mock_fast; }')
     out.append('extern "C" void mock_set_free(size_t n) { mock_free = n; }')
     out.append('extern "C" long mock_malloc_count() { return mock_mallocs; }')
     return "\n".join(out) + "\n"
