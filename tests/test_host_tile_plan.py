@@ -85,3 +85,25 @@ def test_a_batch_and_a_member_alone_keep_both_plans(host_lib):
         made, launches = counted(host_lib, lambda: f.step_n(4))
         assert made <= 2 and launches > 0
         assert counted(host_lib, lambda: b.step_n(4))[1] > 0
+
+
+def test_scenarios_plan_with_no_kernel_forced(host_lib):
+    """Every scenario's default plan validates, the tile kernel's where it takes the cell."""
+    from scenarios import SCENARIOS
+    from test_gpu_tile_calls import PLAIN_2D
+    for name in sorted(SCENARIOS):
+        for single in (False, True):
+            s, f, _ = SCENARIOS[name][0](host_lib, single=single)
+            launches = counted(host_lib, lambda: f.step_n(30))[1]
+            f.step()
+            assert f.t == 31 and (launches > 0) == PLAIN_2D.get(name, False), name
+
+
+def test_batches_of_2d_members_take_the_tile_kernel(host_lib):
+    import test_gpu_tile_calls as TC
+    sims = TC.members(host_lib, False)
+    b = capi.batch([f for _, f, _ in sims], use_graph=False, autotune=False)
+    seen = []
+    TC.drive(sims, lambda n: seen.append((n, counted(host_lib, lambda: b.step_n(n))[1])))
+    took = {n: t for n, t in seen}
+    assert all(took[n] > 0 for n in (80, 3, 7, 70, 40)), seen
