@@ -23,6 +23,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include <algorithm>
 #include <cstdlib>
 #include <cstring>
@@ -214,7 +216,11 @@ __device__ __forceinline__ void step_slot(const StepArgs<R> &a, uint32_t i, int 
 // A launch's boxes are one launch because each is small beside the chip: the four x and y uPML
 // slabs of a 131 x 118 x 125 cell took 4 x 10.2 us as launches of their own and fill a
 // fraction of the 256 CUs each.  The block finds its box by its index (uniform selects over
-// constant offsets); a box's geometry travels in scalar registers.
+// constant offsets); a box's geometry travels in scalar registers.  A launch of one box takes that
+// box alone: the set's further 350 bytes of arguments, read before a block's first load, cost a
+// cell that is all latency 2.5 us a launch (1D, one pole, FP64: 21 us a step, 26.5 with the set;
+// 2D TE with uPML along Y, FP64: 28, 33).  Behind a branch on the count they cost launches of
+// several boxes as much (2D, conductivity, FP64: 21 us a step, 32 with the branch).
 __device__ __forceinline__ LaunchBox pick_box(const BoxSet &bs, uint32_t lb) {
   LaunchBox x = bs.b[0];
 #pragma unroll
@@ -222,6 +228,7 @@ __device__ __forceinline__ LaunchBox pick_box(const BoxSet &bs, uint32_t lb) {
     if (k < bs.n && lb >= bs.b[k].first) x = bs.b[k];
   return x;
 }
+__device__ __forceinline__ LaunchBox pick_box(const LaunchBox &x, uint32_t) { return x; }
 // the launch box in a batch item's own grid
 __device__ __forceinline__ LaunchBox item_box(const Grid &g, int g0, int ngroups) {
   LaunchBox x;
@@ -247,8 +254,8 @@ __device__ __forceinline__ void step_body(const StepArgs<R> &a, const LaunchBox 
   step_slot<R, CURL, UPD, 2>(a, i, j0, j1, j2, vrow);
 }
 
-template <class R, bool CURL, bool UPD>
-__global__ __launch_bounds__(BLOCK) void k_step(const StepArgs<R> a, const BoxSet bs) {
+template <class R, bool CURL, bool UPD, class Boxes>
+__global__ __launch_bounds__(BLOCK) void k_step(const StepArgs<R> a, const Boxes bs) {
   const uint32_t lb = xcd_block();
   const LaunchBox x = pick_box(bs, lb);
   const uint32_t t = (lb - x.first) * uint32_t(BLOCK) + threadIdx.x;
@@ -731,8 +738,8 @@ __device__ __forceinline__ void fast_body_slot(const StepArgs<R> &a, const Launc
 // slot's registers, and the three blocks of a tile, dealt to the same XCD, share the partner
 // rows in its L2.  A curl alone keeps the three slots in one thread (measured faster there:
 // its threads are light, and the shared centre rows are loaded once).
-template <class R, int V, bool CURL, bool UPD, bool PML, int NP>
-__global__ __launch_bounds__(BLOCK) void k_fast(const StepArgs<R> a, const BoxSet bs) {
+template <class R, int V, bool CURL, bool UPD, bool PML, int NP, class Boxes>
+__global__ __launch_bounds__(BLOCK) void k_fast(const StepArgs<R> a, const Boxes bs) {
   const uint32_t lb = xcd_block(a.rev);
   const uint32_t q = UPD ? lb / 3u : lb;
   const LaunchBox x = pick_box(bs, q);
@@ -1568,12 +1575,19 @@ template <class R> void launch_step(const StepArgs<R> &a, const BoxSet &boxes, b
     bs.b[k].count = box_count("meep: launch box too large for one launch",
                               size_t(bs.b[k].an[0]) * size_t(bs.b[k].an[1]) * size_t(bs.b[k].an[2]));
   const unsigned nb = (box_blocks(bs) + 7u) / 8u * 8u;
-  if (curl && upd)
-    hipLaunchKernelGGL((k_step<R, true, true>), dim3(nb), dim3(BLOCK), 0, s, a, bs);
-  else if (curl)
-    hipLaunchKernelGGL((k_step<R, true, false>), dim3(nb), dim3(BLOCK), 0, s, a, bs);
-  else if (upd)
-    hipLaunchKernelGGL((k_step<R, false, true>), dim3(nb), dim3(BLOCK), 0, s, a, bs);
+  auto launch = [&](const auto &boxes) {
+    using Boxes = std::decay_t<decltype(boxes)>;
+    if (curl && upd)
+      hipLaunchKernelGGL((k_step<R, true, true, Boxes>), dim3(nb), dim3(BLOCK), 0, s, a, boxes);
+    else if (curl)
+      hipLaunchKernelGGL((k_step<R, true, false, Boxes>), dim3(nb), dim3(BLOCK), 0, s, a, boxes);
+    else if (upd)
+      hipLaunchKernelGGL((k_step<R, false, true, Boxes>), dim3(nb), dim3(BLOCK), 0, s, a, boxes);
+  };
+  if (bs.n == 1)
+    launch(bs.b[0]);
+  else
+    launch(bs);
 }
 
 template <class R, int V, bool PML, int NP>
@@ -1587,12 +1601,31 @@ void launch_fast_np(const StepArgs<R> &a, const BoxSet &boxes, bool curl, bool u
   }
   const unsigned n = box_blocks(bs);
   const unsigned nb = ((upd ? 3u * n : n) + 7u) / 8u * 8u; // with an update, one slot per block
-  if (curl && upd)
-    hipLaunchKernelGGL((k_fast<R, V, true, true, PML, NP>), dim3(nb), dim3(BLOCK), 0, s, a, bs);
-  else if (curl)
-    hipLaunchKernelGGL((k_fast<R, V, true, false, PML, NP>), dim3(nb), dim3(BLOCK), 0, s, a, bs);
-  else if (upd)
-    hipLaunchKernelGGL((k_fast<R, V, false, true, PML, NP>), dim3(nb), dim3(BLOCK), 0, s, a, bs);
+  // a curl alone knows no poles, and an update alone with uPML always takes the set: kernels that
+  // no launch reaches would only lengthen the load of the library's code
+  auto launch = [&](const auto &boxes) {
+    using Boxes = std::decay_t<decltype(boxes)>;
+    constexpr bool one = std::is_same_v<Boxes, LaunchBox>;
+    if (curl && upd)
+      hipLaunchKernelGGL((k_fast<R, V, true, true, PML, NP, Boxes>), dim3(nb), dim3(BLOCK), 0, s, a, boxes);
+    else if (curl) {
+      if constexpr (NP == 0) hipLaunchKernelGGL((k_fast<R, V, true, false, PML, NP, Boxes>), dim3(nb), dim3(BLOCK), 0, s, a, boxes);
+    }
+    else if (upd) {
+      if constexpr (PML && one)
+        hipLaunchKernelGGL((k_fast<R, V, false, true, PML, NP, BoxSet>), dim3(nb), dim3(BLOCK), 0, s, a, bs);
+      else
+        hipLaunchKernelGGL((k_fast<R, V, false, true, PML, NP, Boxes>), dim3(nb), dim3(BLOCK), 0, s, a, boxes);
+    }
+  };
+  if (bs.n == 1) {
+    launch(bs.b[0]);
+    return;
+  }
+  if constexpr (PML) // without uPML there is an interior alone
+    launch(bs);
+  else
+    throw std::runtime_error("meep: internal: several boxes without uPML");
 }
 // The pole-carrying updates hold P, P_prev and sigma of every pole in registers: in FP32 they
 // take 8-byte groups (V = 2) to keep the occupancy of the 16-byte form's plain kernels.
