@@ -1285,17 +1285,20 @@ static bool r3_launch(const StepArgs<R> &a, bool curl, bool upd, hipStream_t s) 
 template <class R> bool launch_row3(const StepArgs<R> &a, bool curl, bool upd, hipStream_t s) {
   static const bool off = getenv("MEEP_AMD_NO_ROW3") != nullptr;
   if (off) return false;
-  // 16-byte groups with poles too: half the address and uPML work of 8-byte ones (384x384x192, two
-  // poles, FP32: the D interior 800 -> 768 us), which these kernels are bound by
-  constexpr int V = 16 / sizeof(R);
+  constexpr int V = 16 / sizeof(R), VP = V > 2 ? 2 : V;
+  // With poles in FP32, 16-byte groups halve the address and uPML work that these kernels are bound
+  // by, and the waves in flight: us of the D interior for 8- / 16-byte groups with two poles, 56x60x64
+  // 14.8 / 18.6, 128x128x128 47.5 / 48.2, 160x150x170 98.6 / 94.4, 384x384x192 800 / 768; with one
+  // 13.1 / 17.2, 37.9 / 38.3, 85.0 / 79.8.  The line is between the second and the third.
+  const bool wide = size_t(a.g.an[0]) * size_t(a.g.an[1]) * size_t(a.g.an[2]) >= (size_t(5) << 19);
   const int PH = a.sgn < 0 ? 1 : 0;
   const bool u = upd;
   if (PH == 0) return u ? r3_launch<R, V, 0, true, 0>(a, curl, upd, s) : r3_launch<R, V, 0, false, 0>(a, curl, upd, s);
   if (!u) return r3_launch<R, V, 1, false, 0>(a, curl, upd, s);
   switch (a.npole) {
     case 0: return r3_launch<R, V, 1, true, 0>(a, curl, upd, s);
-    case 1: return r3_launch<R, V, 1, true, 1>(a, curl, upd, s);
-    case 2: return r3_launch<R, V, 1, true, 2>(a, curl, upd, s);
+    case 1: return wide ? r3_launch<R, V, 1, true, 1>(a, curl, upd, s) : r3_launch<R, VP, 1, true, 1>(a, curl, upd, s);
+    case 2: return wide ? r3_launch<R, V, 1, true, 2>(a, curl, upd, s) : r3_launch<R, VP, 1, true, 2>(a, curl, upd, s);
     default: return false;
   }
 }
