@@ -3627,7 +3627,13 @@ template <class R> struct Fields : FieldsBase {
   struct DftGroup {
     long dft_v = -1, plan_v = -1;
     bool fits = false, built = false, ok = false;
-    DevBuf items, snap_item, snap_first, flush_item, flush_first;
+    long waited = 0; // steps accumulated chunk by chunk before the tables were built
+    DevBuf tab; // the items, then the two launches' block tables
+    size_t snap_at = 0, flush_at = 0;
+    const BatchDft<R> *items() const { return static_cast<const BatchDft<R> *>(tab.p); }
+    const uint32_t *table(size_t at, unsigned skip) const {
+      return reinterpret_cast<const uint32_t *>(static_cast<const char *>(tab.p) + at) + skip;
+    }
     unsigned snap_nblk = 0, flush_nblk = 0;
     std::vector<int> decs; // the chunks' distinct decimations
     // whether a chunk accumulates, and the most times one does, in the steps t0 + 1 .. t1
@@ -3645,6 +3651,7 @@ template <class R> struct Fields : FieldsBase {
     dgroup.dft_v = dft_version;
     dgroup.plan_v = plan_version;
     dgroup.fits = dgroup.built = dgroup.ok = false;
+    dgroup.waited = 0;
     dgroup.decs.clear();
     for (auto &cp : dft_chunks) {
       DftChunk<R> &ch = *cp;
@@ -3655,10 +3662,14 @@ template <class R> struct Fields : FieldsBase {
     }
     return dgroup.fits = !dgroup.decs.empty();
   }
-  // the tables; false where memory for them is short (each chunk then accumulates by itself)
-  bool dft_group() {
+  // The tables; false where memory for them is short (each chunk then accumulates by itself).
+  // `now` false: built once there are chunks and steps enough (the tables take 0.1 ms, a chunk's own
+  // launches 3 us a step).
+  static constexpr long DFT_GROUP_WORTH = 32;
+  bool dft_group(bool now = true) {
     if (!dft_groupable()) return false;
     if (dgroup.built) return dgroup.ok;
+    if (!now && (dgroup.waited++ + rows_hint) * long(dft_chunks.size()) < DFT_GROUP_WORTH) return false;
     dgroup.built = true;
     try {
       std::vector<BatchDft<R>> items;
@@ -3666,20 +3677,26 @@ template <class R> struct Fields : FieldsBase {
       for (auto &cp : dft_chunks) {
         DftChunk<R> &ch = *cp;
         if (!f[ch.c][0]) continue;
-        if (ch.nsnap) fail("internal: deferred DFT steps pending");
+        flush_dft(ch); // steps deferred by itself
         items.push_back(batch_dft(ch));
         pts.push_back(uint32_t(ch.npts));
         quads.push_back(uint32_t(size_t(ch.npts) * size_t((ch.nfreq + 3) / 4)));
       }
-      upload_vec(dgroup.items, items);
-      block_tables(pts, 256, item, first);
-      upload_vec(dgroup.snap_item, item);
-      upload_vec(dgroup.snap_first, first);
-      dgroup.snap_nblk = unsigned(item.size());
-      block_tables(quads, 256, item, first);
-      upload_vec(dgroup.flush_item, item);
-      upload_vec(dgroup.flush_first, first);
-      dgroup.flush_nblk = unsigned(item.size());
+      // one allocation and one copy: a first short call of a simulation should not pay for ten
+      std::vector<char> host(sizeof(BatchDft<R>) * items.size());
+      memcpy(host.data(), items.data(), host.size());
+      auto append = [&](const std::vector<uint32_t> &counts, size_t &at, unsigned &nblk) {
+        block_tables(counts, 256, item, first);
+        at = host.size();
+        nblk = unsigned(item.size());
+        const char *a = reinterpret_cast<const char *>(item.data()), *b = reinterpret_cast<const char *>(first.data());
+        host.insert(host.end(), a, a + sizeof(uint32_t) * item.size());
+        host.insert(host.end(), b, b + sizeof(uint32_t) * first.size());
+      };
+      static_assert(sizeof(BatchDft<R>) % sizeof(uint32_t) == 0, "aligned tables");
+      append(pts, dgroup.snap_at, dgroup.snap_nblk);
+      append(quads, dgroup.flush_at, dgroup.flush_nblk);
+      upload_vec(dgroup.tab, host);
     } catch (const OutOfMemory &) {
       return false;
     }
@@ -3690,9 +3707,8 @@ template <class R> struct Fields : FieldsBase {
   long window_t = 0, window_end = 0;
   void flush_dft_group() {
     if (!window_open) return;
-    launch_dft_flush_batch<R>(static_cast<const BatchDft<R> *>(dgroup.items.p), static_cast<const uint32_t *>(dgroup.flush_item.p),
-                              static_cast<const uint32_t *>(dgroup.flush_first.p), dgroup.flush_nblk, window_t,
-                              window_end - window_t, stream);
+    launch_dft_flush_batch<R>(dgroup.items(), dgroup.table(dgroup.flush_at, 0), dgroup.table(dgroup.flush_at, dgroup.flush_nblk),
+                              dgroup.flush_nblk, window_t, window_end - window_t, stream);
     window_open = false;
   }
   // chunk ch as a batch item, its ring of deferred values allocated
@@ -3714,13 +3730,13 @@ template <class R> struct Fields : FieldsBase {
   // chunks whose phases for DFT_DEFER steps fit the flush kernel's table keep this step's
   // point values and accumulate every DFT_DEFER steps (and at the end of every step_n call)
   void update_dfts() {
-    if (dft_defer_steps && !dft_chunks.empty() && dft_group()) {
+    if (dft_defer_steps && !dft_chunks.empty() && dft_group(false)) {
       if (!dgroup.hits(t - 1, t)) return;
       kbegin(MP_K_DFT);
       if (!window_open) window_open = true, window_t = t - 1;
       window_end = t;
-      launch_dft_snap_batch<R>(static_cast<const BatchDft<R> *>(dgroup.items.p), static_cast<const uint32_t *>(dgroup.snap_item.p),
-                               static_cast<const uint32_t *>(dgroup.snap_first.p), dgroup.snap_nblk, window_t, t - window_t, stream);
+      launch_dft_snap_batch<R>(dgroup.items(), dgroup.table(dgroup.snap_at, 0), dgroup.table(dgroup.snap_at, dgroup.snap_nblk),
+                               dgroup.snap_nblk, window_t, t - window_t, stream);
       if (dgroup.most_hits(window_t, t) == DFT_DEFER) flush_dft_group();
       kend();
       return;

@@ -1930,8 +1930,6 @@ void launch_conn_batch(const BatchConn *items, const uint32_t *blk_item, const u
   template void launch_step_batch<R>(const BatchItem<R> *, const uint32_t *, const uint32_t *, unsigned, int, bool, bool, int, \
                                      const double *, hipStream_t);                                 \
   template void launch_dft_batch<R>(const BatchDft<R> *, const uint32_t *, const uint32_t *, unsigned, long, hipStream_t); \
-  template void launch_dft_snap_batch<R>(const BatchDft<R> *, const uint32_t *, const uint32_t *, unsigned, long, long, hipStream_t); \
-  template void launch_dft_flush_batch<R>(const BatchDft<R> *, const uint32_t *, const uint32_t *, unsigned, long, long, hipStream_t); \
   template void launch_conn_batch<R>(const BatchConn *, const uint32_t *, const uint32_t *, unsigned, hipStream_t);
 #define INSTANTIATE(R)                                                                             \
   template void launch_step<R>(const StepArgs<R> &, const BoxSet &, bool, bool, hipStream_t);                      \
@@ -1949,11 +1947,14 @@ void launch_conn_batch(const BatchConn *items, const uint32_t *blk_item, const u
   template void launch_dft<R>(const DftArgs<R> &, hipStream_t);                                    \
   template void launch_dft_snap<R>(const DftArgs<R> &, R *, R *, hipStream_t);                     \
   template void launch_dft_flush<R>(const DftArgs<R> &, const DftDefer<R> &, hipStream_t);         \
+  template void launch_dft_snap_batch<R>(const BatchDft<R> *, const uint32_t *, const uint32_t *, unsigned, long, long, hipStream_t); \
+  template void launch_dft_flush_batch<R>(const BatchDft<R> *, const uint32_t *, const uint32_t *, unsigned, long, long, hipStream_t); \
   template void launch_check<R>(const R *const *, const int64_t *, const double *, int, int *,     \
                                 hipStream_t);                                                      \
   template void launch_flux_plane<R>(const FluxPlaneArgs<R> &, double *, hipStream_t);
 // The build compiles this file once per field precision (MX_REAL) and part (MX_PART 1: the
-// single-chunk launchers, 2: the batched ones), in parallel.
+// single-chunk launchers and those of grouped DFT chunks, 2: the batched ones, whose code a program
+// without batches never loads), in parallel.
 #ifdef MX_REAL
 #if MX_PART != 2
 INSTANTIATE(MX_REAL)

@@ -107,3 +107,18 @@ def test_batches_of_2d_members_take_the_tile_kernel(host_lib):
     TC.drive(sims, lambda n: seen.append((n, counted(host_lib, lambda: b.step_n(n))[1])))
     took = {n: t for n, t in seen}
     assert all(took[n] > 0 for n in (80, 3, 7, 70, 40)), seen
+
+
+def test_a_first_short_call_makes_few_allocations(host_lib):
+    """Beside the chunks' rings of deferred values and the source rows: nothing while the steps and
+    chunks are few, one allocation for the grouped launches' tables after that."""
+    s = structure(host_lib, dim=3, size=(2.0, 1.8, 1.6), a=8)
+    f = fields(s)
+    f.use_real_fields()
+    f.add_volume_source(Ez, gaussian_src_time(0.6, 0.6), (1.0, 0.9, 0.8), (1.0, 0.9, 0.8))
+    fl = [f.add_dft_flux(d, (0.4, 0.4, 0.4), hi, [0.5, 0.6], decimation_factor=1)
+          for d, hi in ((0, (0.4, 1.4, 1.2)), (1, (1.6, 0.4, 1.2)), (2, (1.6, 1.4, 0.4)))]
+    f.step()
+    chunks = sum(m.num_chunks(w) for m in fl for w in (0, 1))
+    assert counted(host_lib, lambda: f.step_n(2))[0] <= chunks + 1
+    assert counted(host_lib, lambda: f.step_n(40))[0] <= 2
