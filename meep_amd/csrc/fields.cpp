@@ -2261,9 +2261,11 @@ template <class R> struct Fields : FieldsBase {
     return p;
   }
   long pool_version = 0; // changes with the second buffers
-  // each state array's second buffer, in one allocation
-  DevBuf s2_pool;
-  std::map<const void *, char *> s2_alt;
+  // Each state array's second buffer, an allocation of the array's own size: the runtime reuses
+  // released ones of the sizes that programs build and drop simulations with, and maps a block of
+  // some MB anew each time (a gradient that builds its simulation each pass: 47 ms, 62 ms with
+  // the second buffers in one block).
+  std::map<const void *, std::unique_ptr<DevBuf>> s2_alt;
   bool s2_off = getenv("MEEP_AMD_NO_TILE2D") != nullptr;
   // Whether the tile kernel can take this chunk's next steps, memory apart: 2D, no periodic
   // halos, no conductivity, no magnetic poles and at most S2_POLES electric ones, every source in
@@ -2364,7 +2366,6 @@ template <class R> struct Fields : FieldsBase {
       for (S2Monitors &m : p.mons) m.plan_v = -1, m.buf.alloc(0);
     }
     s2_alt.clear();
-    s2_pool.alloc(0);
     ++pool_version;
   }
   // The arrays of a set's arguments and the second pointers beside them, as (array, second
@@ -2393,25 +2394,23 @@ template <class R> struct Fields : FieldsBase {
         });
     if (!have) {
       size_t total = 0, free = 0, all = 0;
-      for (auto &q : need) total += (q.second + 255) / 256 * 256;
+      for (auto &q : need) total += q.second;
       HIPCHECK(hipStreamSynchronize(stream));
       s2_alt.clear();
-      s2_pool.alloc(0);
       ++pool_version;
       HIPCHECK(hipMemGetInfo(&free, &all));
       if (free < total || free - total < all / 2) return false;
-      s2_pool.alloc(total);
-      char *at = static_cast<char *>(s2_pool.p);
       for (auto &q : need) {
-        s2_alt[q.first] = at;
-        HIPCHECK(hipMemcpyAsync(at, q.first, q.second, hipMemcpyDeviceToDevice, stream));
-        at += (q.second + 255) / 256 * 256;
+        std::unique_ptr<DevBuf> b(new DevBuf);
+        b->alloc(q.second);
+        HIPCHECK(hipMemcpyAsync(b->p, q.first, q.second, hipMemcpyDeviceToDevice, stream));
+        s2_alt[q.first] = std::move(b);
       }
     }
     for (auto &S : s2.sets)
       for (int cmp = 0; cmp < ncmp(); ++cmp)
         s2_pairs(S->a[cmp][0][0], [&](auto *in, auto *&out) {
-          if (in) out = reinterpret_cast<std::remove_reference_t<decltype(out)>>(s2_alt.at(in));
+          if (in) out = static_cast<std::remove_reference_t<decltype(out)>>(s2_alt.at(in)->p);
         });
     return true;
   }
@@ -3126,7 +3125,7 @@ template <class R> struct Fields : FieldsBase {
       const void *from = a.p;
       if (second) {
         auto it = s2_alt.find(a.p);
-        if (it != s2_alt.end()) from = it->second;
+        if (it != s2_alt.end()) from = it->second->p;
       }
       HIPCHECK(hipMemcpyAsync(cp.data[q]->p, from, a.esz * gv.ntot, hipMemcpyDeviceToDevice, stream));
     }
