@@ -2244,7 +2244,8 @@ template <class R> struct Fields : FieldsBase {
     long plan_v = -1, dft_v = -1;
     int n = 0, mask = 0;
     size_t entry_at = 0, mons_at[2] = {0, 0};
-    DevBuf buf;
+    std::shared_ptr<DevBuf> buf; // the tables, from byte `at` of a buffer that a batch's members share
+    size_t at = 0;
   };
   struct S2Plan {
     long plan_v = -1, dft_v = -1, src_v = -1, pool_v = -1, builds = 0;
@@ -2265,7 +2266,12 @@ template <class R> struct Fields : FieldsBase {
   // released ones of the sizes that programs build and drop simulations with, and maps a block of
   // some MB anew each time (a gradient that builds its simulation each pass: 47 ms, 62 ms with
   // the second buffers in one block).
-  std::map<const void *, std::unique_ptr<DevBuf>> s2_alt;
+  // A batch allocates those of all its members at once.
+  struct S2Second {
+    char *p;
+    std::shared_ptr<DevBuf> of;
+  };
+  std::map<const void *, S2Second> s2_alt;
   bool s2_off = getenv("MEEP_AMD_NO_TILE2D") != nullptr;
   // Whether the tile kernel can take this chunk's next steps, memory apart: 2D, no periodic
   // halos, no conductivity, no magnetic poles and at most S2_POLES electric ones, every source in
@@ -2332,29 +2338,46 @@ template <class R> struct Fields : FieldsBase {
       if (m.plan_v == plan_version && m.dft_v == dft_version) return false;
     return true;
   }
+  bool s2_built(int margin) {
+    const S2Plan &s2 = s2_plan(margin);
+    return s2.ok && s2.pool_v == pool_version;
+  }
   // ... and, for a call of n steps, its second buffers and tables are in place.  Where memory for
   // them is short the chunk keeps stepping one by one.
   bool s2_ready(int margin, long n) {
     if (!s2_shape(margin)) return false;
+    if (s2_built(margin)) return true;
+    if (s2_unbuilt(margin) && s2_plan(margin).waited + n < s2_worth()) return false;
     S2Plan &s2 = s2_plan(margin);
-    if (s2.ok && s2.pool_v == pool_version) return true;
-    if (s2_unbuilt(margin) && s2.waited + n < s2_worth()) return false;
+    bool ok = false;
     try {
-      s2.ok = s2_second(s2);
-      for (auto &cp : dft_chunks)
-        if (s2.ok) batch_dft(*cp); // the ring of deferred values
+      ok = s2_second(s2);
       for (auto &S : s2.sets)
-        if (s2.ok) s2_finish(s2, *S);
+        if (ok) {
+          S2Monitors &M = s2.mons[S->tm ? 1 : 0];
+          std::vector<char> host;
+          if (s2_tables(M, *S, host)) {
+            M.buf.reset(new DevBuf);
+            M.at = 0;
+            upload_vec(*M.buf, host);
+            s2_tables_done(M);
+          }
+          upload_vec(S->args, s2_finish(s2, *S));
+        }
     } catch (const OutOfMemory &) {
-      s2.ok = false;
+      ok = false;
     }
-    ++s2.builds;
-    s2.pool_v = pool_version;
-    if (!s2.ok) {
+    s2_done(s2, ok);
+    if (!ok) {
       s2_drop();
       s2_off = true;
     }
-    return s2.ok;
+    return ok;
+  }
+  void s2_done(S2Plan &s2, bool ok) {
+    ++s2.builds;
+    s2.pool_v = pool_version;
+    s2.ok = ok;
   }
   // the second buffers and the plans given back
   void s2_drop() {
@@ -2363,7 +2386,7 @@ template <class R> struct Fields : FieldsBase {
       p.plan_v = -1;
       p.shape = p.ok = false;
       p.sets.clear();
-      for (S2Monitors &m : p.mons) m.plan_v = -1, m.buf.alloc(0);
+      for (S2Monitors &m : p.mons) m.plan_v = -1, m.buf.reset();
     }
     s2_alt.clear();
     ++pool_version;
@@ -2379,41 +2402,71 @@ template <class R> struct Fields : FieldsBase {
       for (int p = 0; p < S2_POLES; ++p) fn(c.P[p], c.Po[p]), fn(c.Pp[p], c.Ppo[p]);
     }
   }
-  // Second buffers of every array of the plan, copies of the arrays; false where they would not
-  // fit, or would leave less than half of the device's memory free: a chunk so large is no
-  // longer bound by launches, and what its owner allocates later has to fit as it did without them.
-  bool s2_second(S2Plan &s2) {
-    std::vector<std::pair<const void *, size_t>> need;
+  // The plan's arrays, where some of them lack their second buffer: bytes, and whether the kernel
+  // writes every point of the grid (D, B, E and H; the others in parts of it).
+  struct S2Need {
+    const void *p;
+    size_t bytes;
+    bool whole;
+  };
+  std::vector<S2Need> s2_need(S2Plan &s2) {
+    std::vector<S2Need> need;
     bool have = true;
     for (auto &S : s2.sets)
-      for (int cmp = 0; cmp < ncmp(); ++cmp)
-        s2_pairs(S->a[cmp][0][0], [&](auto *in, auto *) {
+      for (int cmp = 0; cmp < ncmp(); ++cmp) {
+        Step2dArgs<R> &a = S->a[cmp][0][0];
+        s2_pairs(a, [&](auto *in, auto *) {
           if (!in) return;
-          need.push_back({in, sizeof(*in) * gv.ntot});
+          bool whole = false;
+          for (const S2Comp<R> &c : a.c) whole = whole || in == static_cast<const void *>(c.f) || in == static_cast<const void *>(c.e);
+          need.push_back({in, sizeof(*in) * gv.ntot, whole});
           have = have && s2_alt.count(in);
         });
-    if (!have) {
-      size_t total = 0, free = 0, all = 0;
-      for (auto &q : need) total += q.second;
+      }
+    if (have) need.clear();
+    return need;
+  }
+  // Whether second buffers of `total` bytes fit and leave at least half of the device's memory free:
+  // a chunk so large is no longer bound by launches, and what its owner allocates later has to
+  // fit as it did without them.
+  static bool s2_room(size_t total) {
+    size_t free = 0, all = 0;
+    HIPCHECK(hipMemGetInfo(&free, &all));
+    return free >= total && free - total >= all / 2;
+  }
+  // the second buffers, copies of the arrays; false where there is no room
+  bool s2_second(S2Plan &s2) {
+    const std::vector<S2Need> need = s2_need(s2);
+    if (!need.empty()) {
+      size_t total = 0;
+      for (const S2Need &q : need) total += q.bytes;
       HIPCHECK(hipStreamSynchronize(stream));
       s2_alt.clear();
       ++pool_version;
-      HIPCHECK(hipMemGetInfo(&free, &all));
-      if (free < total || free - total < all / 2) return false;
-      for (auto &q : need) {
-        std::unique_ptr<DevBuf> b(new DevBuf);
-        b->alloc(q.second);
-        HIPCHECK(hipMemcpyAsync(b->p, q.first, q.second, hipMemcpyDeviceToDevice, stream));
-        s2_alt[q.first] = std::move(b);
+      if (!s2_room(total)) return false;
+      for (const S2Need &q : need) {
+        std::shared_ptr<DevBuf> b(new DevBuf);
+        b->alloc(q.bytes);
+        HIPCHECK(hipMemcpyAsync(b->p, q.p, q.bytes, hipMemcpyDeviceToDevice, stream));
+        s2_alt[q.p] = {static_cast<char *>(b->p), b};
       }
     }
-    for (auto &S : s2.sets)
-      for (int cmp = 0; cmp < ncmp(); ++cmp)
-        s2_pairs(S->a[cmp][0][0], [&](auto *in, auto *&out) {
-          if (in) out = static_cast<std::remove_reference_t<decltype(out)>>(s2_alt.at(in)->p);
-        });
     return true;
   }
+  // the same from byte `at` of a zeroed buffer, on stream s; returns the byte after them
+  size_t s2_second_in(const std::vector<S2Need> &need, const std::shared_ptr<DevBuf> &buf, size_t at, hipStream_t s) {
+    s2_alt.clear();
+    ++pool_version;
+    for (const S2Need &q : need) {
+      if (at + q.bytes > buf->bytes) fail("internal: second buffers outside their allocation");
+      char *to = static_cast<char *>(buf->p) + at;
+      if (!q.whole) HIPCHECK(hipMemcpyAsync(to, q.p, q.bytes, hipMemcpyDeviceToDevice, s));
+      s2_alt[q.p] = {to, buf};
+      at += s2_aligned(q.bytes);
+    }
+    return at;
+  }
+  static size_t s2_aligned(size_t n) { return (n + 255) / 256 * 256; }
   // the launch arguments of one polarisation, second pointers apart; false when its plan has
   // another shape than the kernel's
   bool s2_set(S2Plan &s2, bool tm, bool fmp) {
@@ -2506,10 +2559,23 @@ template <class R> struct Fields : FieldsBase {
     s2.sets.push_back(std::move(S));
     return true;
   }
-  // a set's monitor tables, its arguments for the other order of P and P_prev and for the other
-  // parity (every pair of buffers exchanged), and the upload
-  void s2_finish(S2Plan &s2, S2Set &S) {
-    s2_monitors(s2.mons[S.tm ? 1 : 0], S);
+  // A set's second pointers, its monitor tables' addresses, its arguments for the other order of P
+  // and P_prev and for the other parity (every pair of buffers exchanged); returns them row by row.
+  std::vector<Step2dArgs<R>> s2_finish(S2Plan &s2, S2Set &S) {
+    const S2Monitors &M = s2.mons[S.tm ? 1 : 0];
+    for (int cmp = 0; cmp < ncmp(); ++cmp) {
+      Step2dArgs<R> &b = S.a[cmp][0][0];
+      s2_pairs(b, [&](auto *in, auto *&out) {
+        if (in) out = reinterpret_cast<std::remove_reference_t<decltype(out)>>(s2_alt.at(in).p);
+      });
+      if (!M.n) continue;
+      const char *base = static_cast<const char *>(M.buf->p) + M.at;
+      b.mon_first = reinterpret_cast<const uint32_t *>(base);
+      b.mon = reinterpret_cast<const S2Entry *>(base + M.entry_at);
+      b.mons = reinterpret_cast<const S2Mon<R> *>(base + M.mons_at[cmp]);
+      b.monmask = M.mask;
+      b.nmon = M.n;
+    }
     std::vector<Step2dArgs<R>> all;
     for (int cmp = 0; cmp < 2; ++cmp) {
       if (cmp < ncmp()) {
@@ -2530,7 +2596,7 @@ template <class R> struct Fields : FieldsBase {
         for (int par = 0; par < 2; ++par) all.push_back(S.a[cmp][order][par]);
       }
     }
-    upload_vec(S.args, all);
+    return all;
   }
   // every pointer the tile kernel can dereference, and the tiles against its registers and lanes
   static void s2_check(const Step2dArgs<R> &a) {
@@ -2545,98 +2611,92 @@ template <class R> struct Fields : FieldsBase {
     if (a.sig[1]) ok = ok && a.c[2].fu && a.c[2].fuo && a.c[1].fw && a.c[1].fwo && a.c[1].e;
     if (!ok) fail("internal: bad 2D tile plan");
   }
-  // the monitor points of each tile, made anew where monitors or arrays have changed
-  void s2_monitors(S2Monitors &M, S2Set &S) {
-    if (M.plan_v != plan_version || M.dft_v != dft_version) {
-      M.dft_v = -1;
-      const Step2dArgs<R> &a = S.a[0][0][0];
-      const size_t nt = size_t(a.ntx) * size_t(a.nty);
-      std::vector<S2Mon<R>> mons[2];
-      std::vector<const DftChunk<R> *> chunks;
-      M.mask = 0;
-      size_t total = 0;
-      for (auto &cp : dft_chunks) {
-        DftChunk<R> &ch = *cp;
-        const int d = comp_dir(ch.c);
-        const bool mag = is_magnetic(ch.c) || is_B(ch.c);
-        if ((S.tm != (d == 2)) != mag) continue; // of the other polarisation
-        S2Mon<R> m;
-        memset(&m, 0, sizeof m);
-        m.npts = uint32_t(ch.npts);
-        m.fld = d + (is_D(ch.c) || is_B(ch.c) ? 3 : 0);
-        m.dec = ch.decimation;
-        auto off = [&](int64_t o) {
-          if (o != 0 && o != 1 && o != gv.st[0]) fail("internal: DFT centring offset");
-          return o == 0 ? 0 : o == 1 ? 1 : S2_COLS;
-        };
-        m.o1 = off(ch.avg1);
-        m.o2 = off(ch.avg2);
-        M.mask |= 1 << m.fld;
-        m.snap = static_cast<R *>(ch.snap.p);
-        mons[0].push_back(m);
-        m.snap += size_t(DFT_DEFER) * size_t(ch.npts);
-        mons[1].push_back(m);
-        chunks.push_back(&ch);
-        total += ch.h_idx.size();
-        if (ch.h_idx.size() != size_t(ch.npts) || ch.h_w.size() != size_t(ch.npts)) fail("internal: DFT points not kept");
-      }
-      M.n = int(chunks.size());
-      if (total >= (size_t(1) << 32)) fail("internal: too many DFT points for the tile kernel");
-      // entries by tile, in chunk and point order: the tiles' counts, their first entries, the entries
-      std::vector<uint32_t> tile(total), first(nt + 1, 0);
-      std::vector<uint16_t> pos(total);
-      size_t q = 0;
-      for (const DftChunk<R> *ch : chunks) {
-        const uint32_t st = uint32_t(gv.st[0]);
-        uint32_t x = 0, y = 0, last = UINT32_MAX - 1;
-        for (uint32_t i : ch->h_idx) {
-          if (i == last + 1 && y + 1 < st)
-            ++y;
-          else
-            x = i / st, y = i - x * st;
-          last = i;
-          if (int(x) > a.nx || int(y) > a.ny) fail("internal: DFT point outside the grid");
-          const int tx = int(x) / a.cx, ty = int(y) / a.cy;
-          const int lx = int(x) - tx * a.cx + a.margin, ly = int(y) - ty * a.cy + a.margin;
-          if (tx >= a.ntx || ty >= a.nty || lx + 1 >= S2_ROWS || ly + 1 >= S2_COLS) fail("internal: DFT point outside its tile");
-          tile[q] = uint32_t(tx * a.nty + ty);
-          pos[q] = uint16_t(lx * S2_COLS + ly);
-          ++first[tile[q] + 1];
-          ++q;
-        }
-      }
-      for (size_t k = 0; k < nt; ++k) first[k + 1] += first[k];
-      auto up = [](size_t n) { return (n + 255) / 256 * 256; };
-      M.entry_at = up(sizeof(uint32_t) * first.size());
-      M.mons_at[0] = M.entry_at + up(sizeof(S2Entry) * total);
-      M.mons_at[1] = M.mons_at[0] + up(sizeof(S2Mon<R>) * chunks.size());
-      std::vector<char> host(M.mons_at[1] + up(sizeof(S2Mon<R>) * chunks.size()));
-      memcpy(host.data(), first.data(), sizeof(uint32_t) * first.size());
-      S2Entry *entry = reinterpret_cast<S2Entry *>(host.data() + M.entry_at);
-      q = 0;
-      for (size_t ci = 0; ci < chunks.size(); ++ci)
-        for (size_t k = 0; k < chunks[ci]->h_idx.size(); ++k, ++q) {
-          S2Entry &e = entry[first[tile[q]]++];
-          e.w = chunks[ci]->h_w[k];
-          e.k = uint32_t(k);
-          e.pos = pos[q];
-          e.chunk = uint16_t(ci);
-        }
-      for (int cmp = 0; cmp < 2; ++cmp)
-        if (M.n) memcpy(host.data() + M.mons_at[cmp], mons[cmp].data(), sizeof(S2Mon<R>) * chunks.size());
-      if (M.n) upload_vec(M.buf, host);
-      M.plan_v = plan_version;
-      M.dft_v = dft_version;
+  // the monitor points of each tile, where monitors or arrays have changed since they were made: the
+  // tables to go into M.buf, from M.at (false: nothing to do)
+  bool s2_tables(S2Monitors &M, S2Set &S, std::vector<char> &host) {
+    if (M.plan_v == plan_version && M.dft_v == dft_version) return false;
+    M.dft_v = -1;
+    const Step2dArgs<R> &a = S.a[0][0][0];
+    const size_t nt = size_t(a.ntx) * size_t(a.nty);
+    std::vector<S2Mon<R>> mons[2];
+    std::vector<const DftChunk<R> *> chunks;
+    M.mask = 0;
+    size_t total = 0;
+    for (auto &cp : dft_chunks) {
+      DftChunk<R> &ch = *cp;
+      const int d = comp_dir(ch.c);
+      const bool mag = is_magnetic(ch.c) || is_B(ch.c);
+      if ((S.tm != (d == 2)) != mag) continue; // of the other polarisation
+      S2Mon<R> m;
+      memset(&m, 0, sizeof m);
+      m.npts = uint32_t(ch.npts);
+      m.fld = d + (is_D(ch.c) || is_B(ch.c) ? 3 : 0);
+      m.dec = ch.decimation;
+      auto off = [&](int64_t o) {
+        if (o != 0 && o != 1 && o != gv.st[0]) fail("internal: DFT centring offset");
+        return o == 0 ? 0 : o == 1 ? 1 : S2_COLS;
+      };
+      m.o1 = off(ch.avg1);
+      m.o2 = off(ch.avg2);
+      M.mask |= 1 << m.fld;
+      batch_dft(ch); // its ring of deferred values
+      m.snap = static_cast<R *>(ch.snap.p);
+      mons[0].push_back(m);
+      m.snap += size_t(DFT_DEFER) * size_t(ch.npts);
+      mons[1].push_back(m);
+      chunks.push_back(&ch);
+      total += ch.h_idx.size();
+      if (ch.h_idx.size() != size_t(ch.npts) || ch.h_w.size() != size_t(ch.npts)) fail("internal: DFT points not kept");
     }
-    for (int cmp = 0; cmp < ncmp() && M.n; ++cmp) {
-      Step2dArgs<R> &b = S.a[cmp][0][0];
-      const char *base = static_cast<const char *>(M.buf.p);
-      b.mon_first = reinterpret_cast<const uint32_t *>(base);
-      b.mon = reinterpret_cast<const S2Entry *>(base + M.entry_at);
-      b.mons = reinterpret_cast<const S2Mon<R> *>(base + M.mons_at[cmp]);
-      b.monmask = M.mask;
-      b.nmon = M.n;
+    M.n = int(chunks.size());
+    if (total >= (size_t(1) << 32)) fail("internal: too many DFT points for the tile kernel");
+    // entries by tile, in chunk and point order: the tiles' counts, their first entries, the entries
+    std::vector<uint32_t> tile(total), first(nt + 1, 0);
+    std::vector<uint16_t> pos(total);
+    size_t q = 0;
+    for (const DftChunk<R> *ch : chunks) {
+      const uint32_t st = uint32_t(gv.st[0]);
+      uint32_t x = 0, y = 0, last = UINT32_MAX - 1;
+      for (uint32_t i : ch->h_idx) {
+        if (i == last + 1 && y + 1 < st)
+          ++y;
+        else
+          x = i / st, y = i - x * st;
+        last = i;
+        if (int(x) > a.nx || int(y) > a.ny) fail("internal: DFT point outside the grid");
+        const int tx = int(x) / a.cx, ty = int(y) / a.cy;
+        const int lx = int(x) - tx * a.cx + a.margin, ly = int(y) - ty * a.cy + a.margin;
+        if (tx >= a.ntx || ty >= a.nty || lx + 1 >= S2_ROWS || ly + 1 >= S2_COLS) fail("internal: DFT point outside its tile");
+        tile[q] = uint32_t(tx * a.nty + ty);
+        pos[q] = uint16_t(lx * S2_COLS + ly);
+        ++first[tile[q] + 1];
+        ++q;
+      }
     }
+    for (size_t k = 0; k < nt; ++k) first[k + 1] += first[k];
+    auto up = s2_aligned;
+    M.entry_at = up(sizeof(uint32_t) * first.size());
+    M.mons_at[0] = M.entry_at + up(sizeof(S2Entry) * total);
+    M.mons_at[1] = M.mons_at[0] + up(sizeof(S2Mon<R>) * chunks.size());
+    host.assign(M.mons_at[1] + up(sizeof(S2Mon<R>) * chunks.size()), 0);
+    memcpy(host.data(), first.data(), sizeof(uint32_t) * first.size());
+    S2Entry *entry = reinterpret_cast<S2Entry *>(host.data() + M.entry_at);
+    q = 0;
+    for (size_t ci = 0; ci < chunks.size(); ++ci)
+      for (size_t k = 0; k < chunks[ci]->h_idx.size(); ++k, ++q) {
+        S2Entry &e = entry[first[tile[q]]++];
+        e.w = chunks[ci]->h_w[k];
+        e.k = uint32_t(k);
+        e.pos = pos[q];
+        e.chunk = uint16_t(ci);
+      }
+    for (int cmp = 0; cmp < 2; ++cmp)
+      if (M.n) memcpy(host.data() + M.mons_at[cmp], mons[cmp].data(), sizeof(S2Mon<R>) * chunks.size());
+    return true;
+  }
+  void s2_tables_done(S2Monitors &M) {
+    M.plan_v = plan_version;
+    M.dft_v = dft_version;
   }
   // Everything that the next m steps allocate, before the first of them: an allocation that failed
   // between two launches would leave the state in the second buffers, where no reader looks.
@@ -3125,7 +3185,7 @@ template <class R> struct Fields : FieldsBase {
       const void *from = a.p;
       if (second) {
         auto it = s2_alt.find(a.p);
-        if (it != s2_alt.end()) from = it->second->p;
+        if (it != s2_alt.end()) from = it->second.p;
       }
       HIPCHECK(hipMemcpyAsync(cp.data[q]->p, from, a.esz * gv.ntot, hipMemcpyDeviceToDevice, stream));
     }
@@ -5127,24 +5187,77 @@ template <class R> struct Batch : BatchBase {
   std::vector<long> tile_builds;
   std::vector<int> tile_decs;
   // Steps that a batch takes one by one, over its calls, before it makes the members' second
-  // buffers and tables: 10 ms for 64 members of 128 to 512 cells, 0.12 ms saved a step; 0.6 ms for 8
-  // members of 60 to 160 cells, 0.05 ms saved a step
-  static constexpr long S2_BATCH_WORTH = 64;
+  // buffers and tables: about 2 ms for 64 members of 128 to 512 cells, 0.12 ms saved a step
+  static constexpr long S2_BATCH_WORTH = 16;
   long tile_waited = 0;
+  bool tiles_off = false; // second buffers did not fit
+  // The second buffers and monitor tables of every member that lacks them, one allocation and one
+  // upload for all (a member's own cost 0.17 ms each); false where memory for them is short.
+  bool build_tiles() {
+    std::vector<Fields<R> *> todo;
+    for (Fields<R> *F : sims)
+      if (!F->s2_built(S2_BATCH)) todo.push_back(F);
+    if (todo.empty()) return true;
+    try {
+      std::vector<std::vector<typename Fields<R>::S2Need>> needs;
+      size_t total = 0;
+      for (Fields<R> *F : todo) {
+        needs.push_back(F->s2_need(F->s2_plan(S2_BATCH)));
+        for (const auto &q : needs.back()) total += Fields<R>::s2_aligned(q.bytes);
+      }
+      if (total) {
+        if (!Fields<R>::s2_room(total)) return false;
+        std::shared_ptr<DevBuf> buf(new DevBuf);
+        buf->alloc(total);
+        HIPCHECK(hipMemsetAsync(buf->p, 0, total, stream));
+        size_t at = 0;
+        for (size_t q = 0; q < todo.size(); ++q)
+          if (!needs[q].empty()) {
+            HIPCHECK(hipStreamSynchronize(todo[q]->stream));
+            at = todo[q]->s2_second_in(needs[q], buf, at, stream);
+          }
+      }
+      std::vector<char> host, one;
+      std::shared_ptr<DevBuf> tab(new DevBuf);
+      std::vector<std::pair<Fields<R> *, typename Fields<R>::S2Monitors *>> fresh;
+      for (Fields<R> *F : todo)
+        for (auto &S : F->s2_plan(S2_BATCH).sets) {
+          auto &M = F->s2_plan(S2_BATCH).mons[S->tm ? 1 : 0];
+          if (!F->s2_tables(M, *S, one)) continue;
+          M.at = host.size();
+          host.insert(host.end(), one.begin(), one.end());
+          fresh.push_back({F, &M});
+        }
+      if (!fresh.empty()) upload_vec(*tab, host);
+      for (auto &q : fresh) {
+        q.second->buf = tab;
+        q.first->s2_tables_done(*q.second);
+      }
+      for (Fields<R> *F : todo) {
+        auto &plan = F->s2_plan(S2_BATCH);
+        for (auto &S : plan.sets) F->s2_finish(plan, *S);
+        F->s2_done(plan, true);
+      }
+    } catch (const OutOfMemory &) {
+      return false;
+    }
+    return true;
+  }
   bool tiles_ready(long m) {
     // every member's shape before any member allocates: second buffers are of no use to a batch
     // that the kernel does not take whole
     bool ready = true, wait = false;
     for (Fields<R> *F : sims) ready = ready && F->s2_shape(S2_BATCH);
-    for (Fields<R> *F : sims) wait = wait || (ready && F->s2_unbuilt(S2_BATCH));
+    for (Fields<R> *F : sims) wait = wait || (ready && !tiles_off && F->s2_unbuilt(S2_BATCH));
     if (wait && tile_waited + m < S2_BATCH_WORTH) {
       tile_waited += m;
       return false;
     }
-    if (ready) {
-      for (Fields<R> *F : sims) ready = ready && F->s2_ready(S2_BATCH, S2_BATCH_WORTH + F->s2_worth());
-      if (!ready) // memory is short
-        for (Fields<R> *F : sims) F->s2_drop();
+    ready = ready && !tiles_off;
+    if (ready && !build_tiles()) { // memory is short
+      tiles_off = true;
+      for (Fields<R> *F : sims) F->s2_drop();
+      ready = false;
     }
     if (!ready) {
       tile_builds.clear();
@@ -5177,7 +5290,6 @@ template <class R> struct Batch : BatchBase {
           g->items.push_back({S.get(), cmp, q});
           g->monmask |= a.monmask;
         }
-      HIPCHECK(hipStreamSynchronize(F->stream)); // the second buffers are copies made there
     }
     for (auto &g : tgroups) {
       std::vector<uint32_t> item, tile;

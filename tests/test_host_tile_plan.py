@@ -122,3 +122,17 @@ def test_a_first_short_call_makes_few_allocations(host_lib):
     chunks = sum(m.num_chunks(w) for m in fl for w in (0, 1))
     assert counted(host_lib, lambda: f.step_n(2))[0] <= chunks + 1
     assert counted(host_lib, lambda: f.step_n(40))[0] <= 2
+
+
+def test_a_batch_builds_its_members_plans_together(host_lib):
+    """Second buffers and monitor tables of all members are one allocation each: what building costs
+    does not grow with the members (a member's own rings of deferred values apart)."""
+    made = []
+    for count in (2, 12):
+        sims = [cell(host_lib, npole=q % 2, nx=40 + 3 * q) for q in range(count)]
+        b = capi.batch([f for _, f in sims], use_graph=False, autotune=False)
+        b.step_n(2)  # the first step and the one-step plan
+        n, launches = counted(host_lib, lambda: b.step_n(40))
+        assert launches > 0
+        made.append(n)
+    assert made[0] == made[1], made
