@@ -18,8 +18,11 @@
 // What bounds it: instruction issue in the tiles that meet a uPML corner (about three times a
 // plain tile's time), then the load of a tile before its first step (4 us).  Per step with its
 // monitors, one-step kernels -> here: 320 x 160 FP64 (88 tiles) 47 us -> 5.2 us; 401 x 263 FP32
-// TE with a Drude pole and a field map over the cell 61 us -> 14.7 us; 64 squares of 128 to
-// 512 cells together 181 us -> 76 us.  Rows x columns 32 x 64 with 16 waves of 2 rows each: 4 rows a
+// TE with a Drude pole and a field map over the cell 61 us -> 14.2 us; 64 squares of 128 to
+// 512 cells together 181 us -> 75 us.  A plain tile pays for the registers of a uPML tile: 113 to
+// 128 VGPRs, with spills of 0 to 34 of them in FP32 (20 to 140 bytes of scratch a lane from TM with
+// two poles on) and 16 (TM, no pole) to 153 (TE, two poles; 400 bytes) in FP64, and 83 to 185
+// SGPRs in every form.  Rows x columns 32 x 64 with 16 waves of 2 rows each: 4 rows a
 // thread and 8 waves have more neighbours in the same wave but half the waves to issue from
 // (32 us against 19 for up to 8 steps of a 400 x 300 FP32 cell).
 #include "engine.hpp"

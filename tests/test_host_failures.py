@@ -43,7 +43,7 @@ def test_far_fields_after_a_failed_allocation(host_lib):
         n2f.farfield((1.5, 9.0, 0))
         if not failed:
             break
-    assert after >= 2 and not failed  # some allocation was made to fail, and the last round reached none
+    assert after >= 2 and not failed  # some allocation was made to fail, and the last pass reached none
 
 
 def plain_2d(lib, nx=40, ny=60):
@@ -80,7 +80,7 @@ def _raised(lib):
         assert f.t == t + 17
         if made <= after:
             return n
-    raise AssertionError("every round ran out of memory")
+    raise AssertionError("every pass ran out of memory")
 
 
 def test_second_buffers_that_do_not_fit(host_lib, monkeypatch):
