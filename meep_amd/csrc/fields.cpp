@@ -2426,13 +2426,13 @@ template <class R> struct Fields : FieldsBase {
     if (have) need.clear();
     return need;
   }
-  // Whether second buffers of `total` bytes fit and leave at least half of the device's memory free:
-  // a chunk so large is no longer bound by launches, and what its owner allocates later has to
-  // fit as it did without them.
+  // Whether second buffers of `total` bytes may be taken: an eighth of the free memory at most, and an
+  // eighth of the device's stays free.  A chunk so large is no longer bound by launches, and what
+  // its owner allocates later has to fit as it did without them.
   static bool s2_room(size_t total) {
     size_t free = 0, all = 0;
     HIPCHECK(hipMemGetInfo(&free, &all));
-    return free >= total && free - total >= all / 2;
+    return total <= free / 8 && free - total >= all / 8;
   }
   // the second buffers, copies of the arrays; false where there is no room
   bool s2_second(S2Plan &s2) {

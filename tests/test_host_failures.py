@@ -98,9 +98,9 @@ def _allocations(lib, call):
     return lib.mock_malloc_count() - before
 
 
-def test_second_buffers_leave_half_of_the_memory(host_lib, monkeypatch):
-    """With less than half of the device's memory left the chunk takes no second buffers."""
-    host_lib.mock_set_free(144 << 30)
+def test_second_buffers_leave_memory_free(host_lib, monkeypatch):
+    """With less than an eighth of the device's memory left the chunk takes no second buffers."""
+    host_lib.mock_set_free(36 << 30)
     try:
         s, f = plain_2d(host_lib)
         short = _allocations(host_lib, lambda: f.step_n(16))
@@ -131,7 +131,7 @@ def test_batch_that_the_tile_kernel_does_not_take(host_lib, monkeypatch, short):
         assert all(f.t == 13 for _, f in sims)
         return n
     if short:
-        host_lib.mock_set_free(144 << 30)
+        host_lib.mock_set_free(36 << 30)
     try:
         got = run()
     finally:
