@@ -566,8 +566,8 @@ def run_batch2d(args, lib, steps=None, warmup=None):
         "workload": f"{BATCH_N} independent 2D TM simulations, square sides 128-512 cells (seeded), "
                     "resolution 10, eps 16x16 blocks in [1, 12], 10-cell uPML, Gaussian Ez point "
                     "source fcen in [0.1, 0.3] df = 0.1 fcen, 16-frequency flux line with FP64 "
-                    "accumulators; one launch per launch group for all simulations, "
-                    f"{'eager' if args.batch_eager else 'hipGraph'} step loop, autotuned block size {block}",
+                    "accumulators; all simulations stepped together (several steps a launch; calls too short for "
+                    f"that one by one, {'eager' if args.batch_eager else 'from a hipGraph'}, block size {block})",
         "cells": cells, "simulations": BATCH_N, "resolution": BATCH_A, "courant": 0.5, "parallelism": "none"},
         steps, warmup)
     line["roofline"] = {"bound": "hbm", "kernel": "whole batched step (all launches)",
